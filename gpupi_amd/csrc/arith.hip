@@ -100,8 +100,11 @@ hipError_t length_max(BatchMPContext *ctx, const BatchMPArray &A, bool bits, uin
     return hipSuccess;
 }
 
-// Default schoolbook -> NTT crossover on L_a + L_b (tuned by measurement).
-constexpr int kDefaultNttMinLimbs = 384;
+// Default schoolbook -> NTT crossover on L_a + L_b: the matrix-core products
+// are faster than the one-tile NTT over their whole range (4096 rows of
+// 2000 x 2000 limbs 277 against 300 us, 16384 of 501 x 503 limbs 85 against
+// 269 us, one row of 1203 x 901 limbs 10 against 25 us).
+constexpr int kDefaultNttMinLimbs = (int)gpupi::kMulMfmaMaxTotal + 1;
 
 // Scratch of the allocation-free multiply (batch_mp_mul_noalloc): the NTT's
 // residue planes, spill words and carry flags.  Each device holds its own

@@ -36,12 +36,10 @@ __device__ __forceinline__ uint64_t ballot64(bool p) { return (uint64_t)__ballot
 __device__ __forceinline__ uint64_t resolve_carries(uint64_t G, uint64_t P, uint32_t cin,
                                                     uint32_t *cout) {
     const uint64_t X = G | P;
-    const uint64_t s1 = X + G;
-    const uint32_t c1 = s1 < X;
-    const uint64_t s2 = s1 + (uint64_t)cin;
-    const uint32_t c2 = s2 < s1;
-    *cout = c1 | c2;
-    return s2 ^ X ^ G;
+    uint32_t c;
+    const uint32_t lo = __builtin_addc((uint32_t)X, (uint32_t)G, cin, &c);
+    const uint32_t hi = __builtin_addc((uint32_t)(X >> 32), (uint32_t)(G >> 32), c, cout);
+    return (((uint64_t)hi << 32) | lo) ^ X ^ G;
 }
 
 // Internal stream-aware launchers (defined across the .hip sources).
@@ -85,6 +83,12 @@ hipError_t launch_length_max(const uint32_t *A, uint32_t N, uint32_t L, uint32_t
 hipError_t launch_mul_naive(const uint32_t *A, const uint32_t *B, uint32_t *C, uint32_t N,
                             uint32_t L_a, uint32_t L_b, uint32_t stride_A, uint32_t stride_B,
                             uint32_t stride_C, hipStream_t stream);
+// Products C = A B of N rows on the matrix cores, LA, LB >= 1 and LA + LB at
+// most kMulMfmaMaxTotal (16 tiles of 256 limbs; one limb per tile boundary is
+// left for the recoding's extra digits).
+constexpr uint32_t kMulMfmaMaxTotal = 4088;
+hipError_t launch_mul_mfma(const uint32_t *A, const uint32_t *B, uint32_t *C, uint32_t N, uint32_t LA, uint32_t LB,
+                           uint32_t sA, uint32_t sB, uint32_t sC, hipStream_t stream);
 bool mul_naive_supports(uint32_t L_a, uint32_t L_b);
 
 hipError_t launch_mul_ntt(const uint32_t *A, const uint32_t *B, uint32_t *C, void *workspace,

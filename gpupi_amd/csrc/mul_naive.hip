@@ -56,16 +56,14 @@ __global__ void __launch_bounds__(256) mul_thread_kernel(const uint32_t *A, cons
 constexpr uint32_t kPad = 4;
 
 // Dynamic LDS: a[LA] | 4 zero words | b[LB] | 4 zero words (b indexed -4..LB+3).
-// One wave per product; lane l computes the CPL columns k0 = g0 + CPL l ..
-// (CPL = 2 for products of at most 128 limbs, so that every lane works; 4
-// otherwise), sliding a CPL-wide window of b down the a loop.  Column k =
+// One wave per product; lane l computes the CPL columns k0 = g0 + CPL l ..,
+// sliding a CPL-wide window of b down the a loop.  Column k =
 // x + 2^32 y + 2^64 z becomes limbs as x_k + y_(k-1) + z_(k-2), and the
 // remaining carries go through one ballot resolution per 64 CPL columns.
-template <int CPL>
+constexpr int CPL = 4;
 __global__ void __launch_bounds__(64) mul_wave_kernel(const uint32_t *A, const uint32_t *B, uint32_t *C,
                                                       uint32_t LA, uint32_t LB, uint32_t sA,
                                                       uint32_t sB, uint32_t sC) {
-    static_assert(CPL == 2 || CPL == 4, "two or four columns per lane");
     extern __shared__ uint32_t lds[];
     const uint32_t row = blockIdx.x;
     const uint32_t lane = threadIdx.x;
@@ -206,7 +204,7 @@ const ThreadLauncher kThreadLaunchers[kThreadMaxShort + 1] = {
 }  // namespace
 
 namespace {
-// mul_wave_kernel<4> may take up to 160 KB of dynamic LDS; the attribute is
+// mul_wave_kernel may take up to 160 KB of dynamic LDS; the attribute is
 // a property of the current device, set once per device (serving threads
 // launch concurrently).
 std::mutex g_lds_attr_mu;
@@ -218,7 +216,7 @@ hipError_t allow_large_lds() {
     std::lock_guard<std::mutex> lk(g_lds_attr_mu);
     const uint64_t bit = dev >= 0 && dev < 64 ? 1ull << dev : 0ull;
     if (bit != 0 && (g_lds_attr_done & bit) != 0) return hipSuccess;
-    GPUPI_RETURN_IF(hipFuncSetAttribute((const void *)mul_wave_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    GPUPI_RETURN_IF(hipFuncSetAttribute((const void *)mul_wave_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                         160 * 1024));
     g_lds_attr_done |= bit;
     return hipSuccess;
@@ -257,16 +255,16 @@ hipError_t launch_mul_naive(const uint32_t *A, const uint32_t *B, uint32_t *C, u
         kThreadLaunchers[L_b](A, B, C, N, L_a, stride_A, stride_B, stride_C, stream);
         return hipGetLastError();
     }
+    // on the matrix cores (262144 products of 17 x 17 limbs 96 us against
+    // 122 us with one wave per product here, of 63 x 64 limbs 139 against
+    // 325 us, one of 190 x 190 limbs 5 against 29 us)
+    if (total <= kMulMfmaMaxTotal)
+        return launch_mul_mfma(A, B, C, N, L_a, L_b, stride_A, stride_B, stride_C, stream);
     if (!wave_ok) return hipErrorInvalidValue;
     if (N > 0x7fffffffu) return hipErrorInvalidValue;
     const size_t lds = (size_t)(L_a + kPad + L_b + kPad) * sizeof(uint32_t);
     if (lds > 65536) GPUPI_RETURN_IF(allow_large_lds());
-    if (total <= 2u * kWave) {
-        hipLaunchKernelGGL(mul_wave_kernel<2>, dim3(N), dim3(kWave), lds, stream, A, B, C, L_a, L_b, stride_A,
-                           stride_B, stride_C);
-        return hipGetLastError();
-    }
-    hipLaunchKernelGGL(mul_wave_kernel<4>, dim3(N), dim3(kWave), lds, stream, A, B, C, L_a, L_b, stride_A,
+    hipLaunchKernelGGL(mul_wave_kernel, dim3(N), dim3(kWave), lds, stream, A, B, C, L_a, L_b, stride_A,
                        stride_B, stride_C);
     return hipGetLastError();
 }

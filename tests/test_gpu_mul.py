@@ -608,3 +608,57 @@ def test_tuner_times_every_split_and_restores_the_plan(ctx):
     res = tune.tune_splits(ctx, ops, 16, reps=1, shared=True)
     assert sorted(lv for lv, _ in res) == sorted((m0, 16 - m0) for m0, _ in tune.splits(16))
     assert g.ntt_get_split(16) == before
+
+
+# Lengths around the matrix-core products' edges: a block of 32 digits (8
+# limbs), 32 blocks (256 limbs, a tile and a step of the shorter operand), the
+# one-, two- and four-group shapes, the longest total and one past it.
+MFMA_SHAPES = [(17, 17), (18, 40), (63, 64), (64, 64), (120, 136), (127, 130), (128, 128), (17, 3000), (247, 249),
+               (248, 248), (255, 256), (256, 257), (300, 212), (511, 513), (512, 512), (760, 776), (1016, 1016),
+               (1016, 3072), (1025, 1023), (127, 3961), (1500, 1700), (2040, 2048), (2044, 2044), (2044, 2045)]
+
+
+@pytest.mark.parametrize("la,lb", MFMA_SHAPES)
+@pytest.mark.parametrize("n", [1, 3, 513])
+def test_matrix_core_products(la, lb, n):
+    """Products of 17..4088 limbs against Python integers: random limbs and
+    the words at which the recoding to signed digits and the carries run
+    longest (0x7f7f7f7f passes the recoding's carry on, all ones and powers of
+    two pass the product's), rows apart, a broadcast operand, both operand
+    orders; nothing is written past a row."""
+    rng = np.random.default_rng(la * 5000 + lb + n)
+    words = (0, 0x7F7F7F7F, 0x7F7F7F80, 0x80808080, 0xFFFFFFFF, 1)
+    kinds = len(words) + 2
+
+    def rows(count, length, shift):
+        out = rng.integers(0, 1 << 32, size=(count, length), dtype=np.uint32)
+        for i in range(count):
+            k = (i + shift) % kinds
+            if k < len(words):
+                out[i] = words[k]
+            elif k == len(words):  # long runs of both kinds
+                out[i, : length // 2] = 0x7F7F7F7F
+        return out
+
+    def value(x):
+        return int.from_bytes(np.ascontiguousarray(x).tobytes(), "little")
+
+    with g.Context() as ctx:
+        for shift in range(kinds) if n < kinds else (3,):
+            A, B = rows(n, la, shift), rows(n, lb, 5 * shift + 1)
+            bufa, va = g.upload_rows(A, la + 3, 0xDEADBEEF)
+            bufb, vb = g.upload_rows(B, lb + 1, 0xDEADBEEF)
+            want = [value(a) * value(b) for a, b in zip(A, B)]
+            for x, y in ((va, vb), (vb, va)):
+                bufc, vc = g.upload_rows(np.zeros((n, la + lb), np.uint32), la + lb + 2, 0xABCD1234)
+                g.check(ctx.mul(x, y, vc))
+                g.synchronize()
+                full = bufc.download(np.uint32).reshape(n, la + lb + 2)
+                assert [value(r[: la + lb]) for r in full] == want
+                assert (full[:, la + lb:] == 0xABCD1234).all()
+        # one row of A against every row of B
+        bufc, vc = g.upload_rows(np.zeros((n, la + lb), np.uint32))
+        g.check(ctx.mul(va.view(stride=0), vb, vc))
+        g.synchronize()
+        got = g.download_rows(vc, bufc)
+        assert [value(r) for r in got] == [value(A[0]) * value(b) for b in B]
