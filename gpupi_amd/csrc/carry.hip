@@ -13,6 +13,8 @@
 // tiny kernel: each chunk looks back at its predecessors' (generate,
 // all-propagate) flags and, only if its carry-in is 1, ripples it through
 // its own limbs.  Rows of at most kThreadRowMax limbs use one thread per row.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace gpupi {
@@ -185,12 +187,11 @@ __global__ void __launch_bounds__(256) carry_fixup_kernel(uint32_t *C, uint32_t 
     }
 }
 
-// The spill-add of NTT products with four limbs per lane (16-byte loads and
-// stores): one wave per chunk of 1024 limbs of one row, the same chunk and
-// flag layout as addsub_chunk_kernel<SpillAdd, 16>.  Each lane settles its
-// four limbs for a carry-in of zero, the lanes' (generate, propagate) pairs
-// go through one ballot resolution per 256 limbs, and the lane adds its
-// carry-in.  Every row must start 16-byte aligned.
+// The spill-add of NTT products of more than 512 limbs with four limbs per
+// lane (16-byte loads and stores at any limb): one wave per chunk of 1024
+// limbs of one row.  Each lane settles its four limbs for a carry-in of zero,
+// the lanes' (generate, propagate) pairs go through one ballot resolution per
+// 256 limbs, and the lane adds its carry-in.
 __global__ void __launch_bounds__(256) spill_add_vec_kernel(uint32_t *C, uint32_t stride_C, uint32_t L_c,
                                                             SpillArgs sp, uint32_t chunks_per_row,
                                                             uint64_t total_chunks, uint8_t *flags) {
@@ -208,11 +209,9 @@ __global__ void __launch_bounds__(256) spill_add_vec_kernel(uint32_t *C, uint32_
     for (int s = 0; s < kSeg; ++s) {
         const uint32_t j0 = chunk * (uint32_t)(kSeg * 4 * kWave) + (uint32_t)s * (4 * kWave) + 4 * lane;
         if (j0 + 4 <= L_c) {
-            const uint4 v = *reinterpret_cast<const uint4 *>(out + j0);
-            x[s][0] = v.x;
-            x[s][1] = v.y;
-            x[s][2] = v.z;
-            x[s][3] = v.w;
+            const Quad v = *reinterpret_cast<const Quad *>(out + j0);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) x[s][t] = v.w[t];
         } else {
 #pragma unroll
             for (int t = 0; t < 4; ++t) x[s][t] = j0 + t < L_c ? out[j0 + t] : 0u;
@@ -253,7 +252,7 @@ __global__ void __launch_bounds__(256) spill_add_vec_kernel(uint32_t *C, uint32_
             r[t] = v;
         }
         if (j0 + 4 <= L_c) {
-            *reinterpret_cast<uint4 *>(out + j0) = make_uint4(r[0], r[1], r[2], r[3]);
+            *reinterpret_cast<Quad *>(out + j0) = Quad{{r[0], r[1], r[2], r[3]}};
         } else {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
@@ -372,36 +371,25 @@ __global__ void __launch_bounds__(256) ragged_assembly_fixup_kernel(const Ragged
     }
 }
 
-// Row-aligned 16-byte access: the base is 16-byte aligned and, with more
-// than one row, so is every row.
-bool rows_aligned(const void *p, uint32_t N, uint32_t stride) {
-    return p != nullptr && (((uintptr_t)p) & 15u) == 0 && (N <= 1 || (stride & 3u) == 0);
-}
-
-// Four limbs x[0..4) of row `row` from limb j0 on (zero outside [0, L)).
-__device__ __forceinline__ void load4(const uint32_t *p, uint32_t row, uint32_t stride, int64_t j0, uint32_t L,
-                                      bool vec, uint32_t *x) {
-    const uint32_t *r = p + (size_t)row * stride;
-    if (vec && j0 >= 0 && j0 + 4 <= (int64_t)L) {
-        const uint4 v = *reinterpret_cast<const uint4 *>(r + j0);
-        x[0] = v.x;
-        x[1] = v.y;
-        x[2] = v.z;
-        x[3] = v.w;
+// Four limbs x[0..4) of the row r from limb j0 on (zero outside [0, L)).
+__device__ __forceinline__ void load4(const uint32_t *r, int64_t j0, uint32_t L, uint32_t *x) {
+    if (j0 >= 0 && j0 + 4 <= (int64_t)L) {
+        const Quad v = *reinterpret_cast<const Quad *>(r + j0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) x[t] = v.w[t];
     } else {
 #pragma unroll
         for (int t = 0; t < 4; ++t) x[t] = (j0 + t >= 0 && j0 + t < (int64_t)L) ? r[j0 + t] : 0u;
     }
 }
 
-// Add, Sub, ShiftAdd and ShiftSub with four limbs per lane: one wave per
-// chunk of 1024 limbs of one row, the chunk and flag layout of
-// addsub_chunk_kernel<K, 16> (so carry_fixup_kernel completes long rows).
-// C's rows (and B's and, for Add/Sub, A's when a_vec/b_vec) start 16-byte
-// aligned; the shifted A of ShiftAdd/ShiftSub is read a limb at a time.
+// The ops on rows of more than 512 limbs, four limbs per lane: one wave per
+// chunk of 1024 limbs of one row (carry_fixup_kernel completes longer rows).
+// Bound by HBM; the 16-byte accesses start at any limb, so row strides and
+// shifts need no alignment (R = (R1 << s) - R2 over 512 rows of 128249 limbs:
+// 271 us with a limb per lane, 158 us this way).
 template <AddSubKind K>
-__global__ void __launch_bounds__(256) addsub_vec_kernel(AddSubArgs a, bool a_vec, bool b_vec, uint32_t chunks_per_row,
-                                                         uint64_t total_chunks, uint8_t *flags) {
+__global__ void __launch_bounds__(256) addsub_vec_kernel(AddSubArgs a, uint32_t chunks_per_row, uint64_t total_chunks, uint8_t *flags) {
     constexpr bool kSub = OpTraits<K>::kSub;
     constexpr bool kShift = K == AddSubKind::ShiftAdd || K == AddSubKind::ShiftSub;
     constexpr int kSeg = 4;  // 4 x 256 limbs per wave
@@ -411,6 +399,7 @@ __global__ void __launch_bounds__(256) addsub_vec_kernel(AddSubArgs a, bool a_ve
     const uint32_t row = (uint32_t)(wave / chunks_per_row);
     const uint32_t chunk = (uint32_t)(wave - (uint64_t)row * chunks_per_row);
     uint32_t *out = a.C + (size_t)row * a.stride_C;
+    const uint32_t *ra = a.A + (size_t)row * a.stride_A, *rb = a.B + (size_t)row * a.stride_B;
     const int64_t ws = kShift ? (int64_t)(a.shift >> 5) : 0;
     const uint32_t bs = kShift ? (a.shift & 31u) : 0u;
     uint32_t d[kSeg][4], g[kSeg][4];
@@ -421,18 +410,29 @@ __global__ void __launch_bounds__(256) addsub_vec_kernel(AddSubArgs a, bool a_ve
         if constexpr (kShift) {
             // x_t = (A << shift) at limb j0 + t: A[i] << bs | A[i - 1] >> (32 - bs), i = j0 + t - ws
             uint32_t w[5];
-            const uint32_t *ra = a.A + (size_t)row * a.stride_A;
-#pragma unroll
-            for (int t = 0; t < 5; ++t) {
-                const int64_t i = j0 - ws - 1 + t;
-                w[t] = (i >= 0 && i < (int64_t)a.L_a) ? ra[i] : 0u;
-            }
+            const int64_t i = j0 - ws - 1;
+            w[0] = (i >= 0 && i < (int64_t)a.L_a) ? ra[i] : 0u;
+            load4(ra, i + 1, a.L_a, w + 1);
 #pragma unroll
             for (int t = 0; t < 4; ++t) x[t] = bs ? (w[t + 1] << bs) | (w[t] >> (32u - bs)) : w[t + 1];
+        } else if constexpr (K == AddSubKind::MulSmall) {
+            // x: low words of the limb products, y: high words of the ones below
+            const uint32_t below = j0 > 0 && j0 <= (int64_t)a.L_a ? ra[j0 - 1] : 0u;
+            load4(ra, j0, a.L_a, x);
+            y[0] = __umulhi(below, a.scalar);
+#pragma unroll
+            for (int t = 1; t < 4; ++t) y[t] = __umulhi(x[t - 1], a.scalar);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) x[t] *= a.scalar;
         } else {
-            load4(a.A, row, a.stride_A, j0, a.L_a, a_vec, x);
+            load4(ra, j0, a.L_a, x);
         }
-        load4(a.B, row, a.stride_B, j0, a.L_b, b_vec, y);
+        if constexpr (K == AddSubKind::AddSmall || K == AddSubKind::SubSmall) {
+            y[0] = j0 == 0 ? a.scalar : 0u;
+            y[1] = y[2] = y[3] = 0u;
+        } else if constexpr (K != AddSubKind::MulSmall) {
+            load4(rb, j0, a.L_b, y);
+        }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             d[s][t] = kSub ? x[t] - y[t] : x[t] + y[t];
@@ -465,7 +465,7 @@ __global__ void __launch_bounds__(256) addsub_vec_kernel(AddSubArgs a, bool a_ve
             r[t] = v;
         }
         if (j0 + 4 <= (int64_t)a.L_c) {
-            *reinterpret_cast<uint4 *>(out + j0) = make_uint4(r[0], r[1], r[2], r[3]);
+            *reinterpret_cast<Quad *>(out + j0) = Quad{{r[0], r[1], r[2], r[3]}};
         } else {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
@@ -517,23 +517,23 @@ hipError_t run_addsub(const AddSubArgs &a, const SpillArgs &sp, uint8_t *flags, 
     const uint64_t blocks = ceil_div64(total, 4);
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
     uint8_t *fl = need_fix ? flags : nullptr;
-    constexpr bool kVecKind = K == AddSubKind::Add || K == AddSubKind::Sub || K == AddSubKind::ShiftAdd ||
-                              K == AddSubKind::ShiftSub;
-    if (kVecKind && p.chunk_len == 4u * 4u * kWave && rows_aligned(a.C, a.N, a.stride_C)) {
-        // four limbs per lane (in place is fine: a lane reads the limbs it
-        // writes before writing them); 16-byte B (and A) loads where their
-        // rows allow
-        const bool a_vec = rows_aligned(a.A, a.N, a.stride_A), b_vec = rows_aligned(a.B, a.N, a.stride_B);
-        hipLaunchKernelGGL(addsub_vec_kernel<K>, dim3((uint32_t)blocks), dim3(256), 0, stream, a, a_vec, b_vec,
+    const dim3 grid((uint32_t)blocks), block(256);
+    const auto chunks = [&](auto seg) {
+        hipLaunchKernelGGL((addsub_chunk_kernel<K, decltype(seg)::value>), grid, block, 0, stream, a, sp,
                            p.chunks_per_row, total, fl);
-    } else {
+    };
     switch (p.seg) {
-        case 1: hipLaunchKernelGGL((addsub_chunk_kernel<K, 1>), dim3((uint32_t)blocks), dim3(256), 0, stream, a, sp, p.chunks_per_row, total, fl); break;
-        case 2: hipLaunchKernelGGL((addsub_chunk_kernel<K, 2>), dim3((uint32_t)blocks), dim3(256), 0, stream, a, sp, p.chunks_per_row, total, fl); break;
-        case 4: hipLaunchKernelGGL((addsub_chunk_kernel<K, 4>), dim3((uint32_t)blocks), dim3(256), 0, stream, a, sp, p.chunks_per_row, total, fl); break;
-        case 8: hipLaunchKernelGGL((addsub_chunk_kernel<K, 8>), dim3((uint32_t)blocks), dim3(256), 0, stream, a, sp, p.chunks_per_row, total, fl); break;
-        default: hipLaunchKernelGGL((addsub_chunk_kernel<K, 16>), dim3((uint32_t)blocks), dim3(256), 0, stream, a, sp, p.chunks_per_row, total, fl); break;
-    }
+        case 1: chunks(std::integral_constant<int, 1>{}); break;
+        case 2: chunks(std::integral_constant<int, 2>{}); break;
+        case 4: chunks(std::integral_constant<int, 4>{}); break;
+        case 8: chunks(std::integral_constant<int, 8>{}); break;
+        default:
+            // in place is fine: a lane reads the limbs it writes first
+            if constexpr (K == AddSubKind::SpillAdd)
+                hipLaunchKernelGGL(spill_add_vec_kernel, grid, block, 0, stream, a.C, a.stride_C, a.L_c, sp,
+                                   p.chunks_per_row, total, fl);
+            else
+                hipLaunchKernelGGL(addsub_vec_kernel<K>, grid, block, 0, stream, a, p.chunks_per_row, total, fl);
     }
     GPUPI_RETURN_IF(hipGetLastError());
     if (need_fix) {
@@ -585,28 +585,7 @@ hipError_t launch_add_spills(uint32_t *C, const uint64_t *spill, uint32_t N, uin
     a.stride_C = stride_C;
     if (run_len == 0 || (run_len & (run_len - 1)) != 0) return hipErrorInvalidValue;
     const SpillArgs sp{spill, (uint32_t)__builtin_ctz(run_len), runs_per_row};
-    const ChunkPlan p = plan_for(L_c);
-    if (N == 0 || L_c == 0) return hipSuccess;
-    if (p.thread_rows || p.chunk_len != 4u * 4u * kWave || (((uintptr_t)C) & 15u) != 0 ||
-        (N > 1 && (stride_C & 3u) != 0))
-        return run_addsub<AddSubKind::SpillAdd>(a, sp, flags, stream);
-    const uint64_t total = (uint64_t)N * p.chunks_per_row;
-    const bool need_fix = p.chunks_per_row > 1;
-    if (need_fix && flags == nullptr) return hipErrorInvalidValue;
-    const uint64_t blocks = ceil_div64(total, 4);
-    if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(spill_add_vec_kernel, dim3((uint32_t)blocks), dim3(256), 0, stream, C, stride_C, L_c, sp,
-                       p.chunks_per_row, total, need_fix ? flags : nullptr);
-    GPUPI_RETURN_IF(hipGetLastError());
-    if (need_fix) {
-        const uint64_t fix_total = (uint64_t)N * (p.chunks_per_row - 1);
-        const uint64_t fblocks = ceil_div64(fix_total, 4);
-        if (fblocks > 0x7fffffffull) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(carry_fixup_kernel<false>, dim3((uint32_t)fblocks), dim3(256), 0, stream, C, stride_C, L_c,
-                           p.chunk_len, p.chunks_per_row, fix_total, (const uint8_t *)flags);
-        GPUPI_RETURN_IF(hipGetLastError());
-    }
-    return hipSuccess;
+    return run_addsub<AddSubKind::SpillAdd>(a, sp, flags, stream);
 }
 
 hipError_t launch_ragged_assemble(const uint32_t *staging, uint64_t K, const RaggedAssembly *as, uint32_t n,

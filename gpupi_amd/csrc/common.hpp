@@ -28,6 +28,12 @@ __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
 __device__ __forceinline__ uint64_t ballot64(bool p) { return (uint64_t)__ballot(p); }
 
+// Four limbs at any limb address: one 16-byte access (global memory takes
+// them at 4-byte alignment).
+struct __attribute__((packed, aligned(4))) Quad {
+    uint32_t w[4];
+};
+
 // Resolve a 64-lane carry (or borrow) chain.  Bit l of G: lane l produces a
 // carry with no carry-in; bit l of P: lane l passes an incoming carry on
 // (G and P never share a bit).  Treating (G|P) and G as two 64-bit numbers,

@@ -44,9 +44,6 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-struct __attribute__((packed, aligned(4))) Quad {  // 16 bytes at any limb
-    uint32_t w[4];
-};
 
 constexpr uint32_t kTileLimbs = 256;
 constexpr uint32_t kMaxTiles = 32;

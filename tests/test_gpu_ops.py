@@ -210,3 +210,49 @@ def test_decimal_naive(ctx, L_limb, L_dec, n):
     Ah = np.ascontiguousarray(A)
     of.lib().o_decimal_naive(Ah.ctypes.data, want.ctypes.data, n, L_limb, L_limb, L_dec, L_dec)
     assert np.array_equal(got[:, :L_dec], want.reshape(n, L_dec))
+
+
+@pytest.mark.parametrize("la", [511, 512, 513, 1023, 1024, 1027, 2050, 3073])
+@pytest.mark.parametrize("extra", [0, 1, 2, 3])
+def test_rows_at_any_alignment(ctx, la, extra):
+    """The four-limbs-per-lane carry kernels (results of more than 512 limbs)
+    on rows and operands at every 4-byte alignment, around their 1024-limb
+    chunks: random limbs, all ones and zeros, carries and borrows through
+    whole chunks, shifts within and across words, one operation in place."""
+    n, lb = 4, la - 5
+    rng = np.random.default_rng(la * 8 + extra)
+
+    def rows(length):
+        out = rng.integers(0, 1 << 32, size=(n, length), dtype=np.uint32)
+        out[1], out[2] = 0xFFFFFFFF, 0
+        out[3, : length - 1] = 0
+        return out
+
+    def value(x):
+        return int.from_bytes(np.ascontiguousarray(x).tobytes(), "little")
+
+    A, B = rows(la), rows(lb)
+    B[1], B[2, 0] = 1, 1
+    bufa, va = g.upload_rows(A, la + extra)
+    bufb, vb = g.upload_rows(B, lb + (3 * extra) % 4)
+    a, b = [value(x) for x in A], [value(x) for x in B]
+    k, s = 0xFFFFFFFB, 32 * 7 + 5 * extra
+    cases = [("add", (va, vb), [x + y for x, y in zip(a, b)], la + 1),
+             ("sub", (va, vb), [x - y for x, y in zip(a, b)], la),
+             ("sub", (vb, va), [y - x for x, y in zip(a, b)], la + 2),
+             ("add_small", (va, k), [x + k for x in a], la + 1),
+             ("sub_small", (va, k), [x - k for x in a], la + 1),
+             ("mul_small", (va, k), [x * k for x in a], la + 1),
+             ("shift_add", (va, vb, s), [(x << s) + y for x, y in zip(a, b)], la + 9),
+             ("shift_sub", (vb, va, s), [(y << s) - x for x, y in zip(a, b)], la + 7)]
+    for op, args, want, lc in cases:
+        bufc, vc = g.upload_rows(np.full((n, lc), 7, np.uint32), lc + extra, 0x5EED5EED)
+        g.check(getattr(ctx, op)(*args, vc), op)
+        g.synchronize()
+        full = bufc.download(np.uint32).reshape(n, lc + extra)
+        assert [value(r[:lc]) for r in full] == [w % (1 << (32 * lc)) for w in want], op
+        assert (full[:, lc:] == 0x5EED5EED).all(), op
+    g.check(ctx.add(va, vb, va), "add in place")
+    g.synchronize()
+    got = g.download_rows(va, bufa)
+    assert [value(r) for r in got] == [(x + y) % (1 << (32 * la)) for x, y in zip(a, b)]
