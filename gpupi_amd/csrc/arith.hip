@@ -332,22 +332,32 @@ hipError_t batch_mp_set_ntt_threshold(BatchMPContext *ctx, uint32_t min_total_li
 
 namespace {
 
-// One-row products whose transform is mostly padding, or whose shorter
-// operand is far shorter than the longer (L the longer, S the shorter,
-// K = 2^k >= L + S the transform), run in pieces of the longer operand that
-// share the shorter one's transform.  Transform work counts 3 K for the
-// product as it is, and (2 m + 1) K' for m pieces of K' points (m forward,
-// m inverse, one of S):
-//   two pieces at K' = K/2 when L + 2 S <= K (2.5 K), s = K/2 - S;
-//   m >= 3 pieces of s = K' - S >= S limbs at a smaller K' when that costs
-//     at most 0.8 of 3 K.
+// One-row products whose shorter operand is far shorter than the longer (L
+// the longer, S the shorter, K = 2^k >= L + S the transform) run in pieces of
+// the longer operand that share the shorter one's transform.  Transform work
+// counts 3 K points for the product as it is and (2 m + 1) K' for m pieces
+// of K' points (m forward, m inverse, one of S), each times the share that
+// transforms with tau of their 16 parts in use cost (transform_share):
+//   two pieces of ceil(L / 2) limbs at K' = K/2 when L + 2 S <= K;
+//   m >= 3 equal pieces of at least S limbs at a smaller K' when even their
+//     full transforms cost at most 0.8 of 3 K.
 // Two pieces are two products sharing S's transform, the first written in
-// place.  More are the rows of one ragged launch sequence (piece_row): even
-// pieces' products land in C and odd ones in an accumulator, each at its
-// offset with zeros to the next piece of its parity.  Either way one add
-// finishes.  Transforms of 2^22 points and up for two pieces, 2^20 for more
-// (smaller products are bound by launches, not by transform size).
-constexpr int kSplitMinLog2 = 22, kSplitManyMinLog2 = 20;
+// place, and one add finishes.  More are the rows of one ragged launch
+// sequence (piece_row), staged and assembled.  Transforms of 2^22 points and
+// up for two pieces, 2^21 for more (smaller products are bound by launches,
+// not by transform size: at 2^20 points whole products take 69-78 us and
+// pieces 78-99).  Measured, whole / two / many (us): L = 6.17 S, 74 % of
+// 2^24: 638 / 652 / 826; L = 50 S: 636 / 642 / 493; L = 12 S, 53 %: 545 /
+// 504 / 480; L = 1.1 S, 60 %: 553 / 703 / -.
+constexpr int kSplitMinLog2 = 22, kSplitManyMinLog2 = 21;
+
+// Time of a transform of 2^k points of which tau of 16 parts are used, in
+// eightieths of a full one's: the first forward level and the launches do not
+// shrink (2^26 points at 10 / 12 / 14 parts: 0.70 / 0.81 / 0.92; 2^22: 0.81 /
+// 0.88 / 0.96; 2^21: 1.0).
+double transform_share(int k, uint32_t tau) {
+    return k >= 23 ? 16.0 + 4.0 * tau : k == 22 ? 40.0 + 2.5 * tau : 64.0 + tau;
+}
 
 struct SplitPlan {
     uint32_t m = 0;  // pieces: 0 = none
@@ -358,18 +368,27 @@ SplitPlan split_plan(uint32_t L, uint32_t S) {
     SplitPlan p;
     const int k = gpupi::ntt_transform_log2(L, S);
     const uint64_t K = 1ull << k;
-    double best = 3.0 * (double)K;
+    double best = 3.0 * (double)K * transform_share(k, gpupi::ntt_tau(L, S, k));
     if (k >= kSplitMinLog2 && (uint64_t)L + 2ull * S <= K && (uint64_t)S < K / 2) {
-        p.m = 2;
-        p.s = (uint32_t)(K / 2 - S);
-        best = 2.5 * (double)K;
+        // the second product's own passes and the add: 5 % where transforms
+        // are large enough to show it
+        const uint32_t s = (L + 1) / 2;
+        const double cost = (k >= 23 ? 2.625 : 2.5) * (double)K * transform_share(k - 1, gpupi::ntt_tau(s, S, k - 1));
+        if (cost < best) {
+            p.m = 2;
+            p.s = s;
+            best = cost;
+        }
     }
     if (k < kSplitManyMinLog2) return p;
     for (uint64_t Kp = K / 2; Kp >= 2ull * S && Kp >= (1ull << 13); Kp /= 2) {
-        const uint64_t s = Kp - S;
-        const uint64_t m = ((uint64_t)L + s - 1) / s;
-        const double cost = (2.0 * (double)m + 1.0) * (double)Kp;
-        if (m >= 3 && cost <= 0.8 * 3.0 * (double)K && cost < best) {
+        const uint64_t m = ((uint64_t)L + Kp - S - 1) / (Kp - S);
+        const uint64_t s = ((uint64_t)L + m - 1) / m;
+        const double points = (2.0 * (double)m + 1.0) * (double)Kp;
+        if (m < 3 || s < S || (m - 1) * s >= L || points > 0.8 * 3.0 * (double)K) continue;
+        const int kp = __builtin_ctzll(Kp);
+        const double cost = 1.1 * points * transform_share(kp, gpupi::ntt_tau((uint32_t)s, S, kp));
+        if (cost < best) {
             best = cost;
             p.m = (uint32_t)m;
             p.s = (uint32_t)s;
@@ -529,7 +548,7 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items,
         auto f = bidx.find(std::make_pair(B, LB));
         if (f == bidx.end()) {
             f = bidx.emplace(std::make_pair(B, LB), (uint32_t)l.nb++).first;
-            host_bset.push_back(gpupi::RaggedB{B, LB});
+            host_bset.push_back(gpupi::RaggedB{B, LB, 0});
         }
         return f->second;
     };
@@ -557,6 +576,10 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items,
                 for (uint32_t i = 0; i < m; ++i) host_rows.push_back(gpupi::piece_row(i, Lp, L, Sp, S, m, plans[q].s, b));
             }
             l.n += m;
+        }
+        for (size_t r = l.r0; r < l.r0 + l.n; ++r) {
+            gpupi::RaggedB &b = host_bset[l.b0 + host_rows[r].b];
+            b.tau = std::max(b.tau, gpupi::ntt_tau(host_rows[r].L_a, host_rows[r].L_b, k));
         }
         l.na = host_asms.size() - l.a0;
         ntt_bytes = std::max(ntt_bytes, gpupi::ntt_ragged_workspace_bytes((uint32_t)l.n, (uint32_t)l.nb, l.chunks, k));

@@ -110,6 +110,8 @@ hipError_t launch_mul_ntt_bounded(const uint32_t *A, const uint32_t *B, uint32_t
                                   uint32_t L_a, uint32_t L_b, uint32_t stride_A, uint32_t stride_B,
                                   uint32_t stride_C, hipStream_t stream);
 int ntt_transform_log2(uint32_t L_a, uint32_t L_b);
+// Parts (of 16) of a transform of 2^log2K points that such a product uses.
+uint32_t ntt_tau(uint32_t L_a, uint32_t L_b, int log2K);
 // The fused 17-term group stage: N rows each of P (51 limbs), Q (68), R (83).
 hipError_t launch_group_stage(uint32_t N, uint32_t *P, uint32_t *Q, uint32_t *R, hipStream_t stream);
 // Rows a ragged launch is filled to (one launch chunk of 2^log2K-point

@@ -67,6 +67,7 @@ struct NttConsts {
     double w16[2][8];
     double w16i[2][8];
     double kinv[2][kMaxLog2 + 1];
+    double inv2[2];
     double garner;  // p0^-1 mod p1, centred
 };
 __constant__ NttConsts c_ntt;
@@ -186,12 +187,39 @@ __device__ __forceinline__ void fwd_dft(double *v, double *lds, const double *ta
     }
 }
 
+// The last inverse step (step 0, radix 16) of a truncated transform: its
+// twiddles, then the radix-16 inverse from the first tau values (uniform over
+// the block); inputs tau.. are zero.  Outputs re-centred as by kDitToGarner.
+template <int T>
+__device__ __forceinline__ void itft16(double *v, int P, Mod m) {
+#pragma unroll
+    for (int j = T; j < 16; ++j) v[j] = 0.0;
+    itft<16, T>(v, c_ntt.w16[P], c_ntt.w16i[P], c_ntt.inv2[P], m);
+}
+template <int M, bool COL>
+__device__ __forceinline__ void itft_step(double *v, const StepMap<M, 0, COL> &sm, const double *tab, int P, Mod m,
+                                          uint32_t tau) {
+    using SM = StepMap<M, 0, COL>;
+    static_assert(SM::R == 16 && SM::LSS > 0, "the first step of several, radix 16");
+    const double *tw = tab + kOffStepInv + ((1u << SM::LMS) - 32u) + sm.n2[0];
+#pragma unroll
+    for (int j = 1; j < 16; ++j) v[j] = mulp(v[j], tw[j << SM::LSS], m);
+    switch (tau) {
+        case 10: itft16<10>(v, P, m); break;
+        case 12: itft16<12>(v, P, m); break;
+        case 14: itft16<14>(v, P, m); break;
+        default: itft16<16>(v, P, m); break;
+    }
+}
+
 // Inverse transform of the tile.  On entry v holds this thread's last-step
 // elements (as left by fwd_dft, so the first LDS store touches only slots
 // this thread read); on exit its step-0 elements.
-template <int M, bool COL, int FINAL = kDitLast>
+// TRUNC: the last step solves for the first `tau` inputs (the others are
+// zero) instead.
+template <int M, bool COL, int FINAL = kDitLast, bool TRUNC = false>
 __device__ __forceinline__ void inv_dft(double *v, double *lds, const double *tab, int P, Mod m,
-                                        uint32_t tid = threadIdx.x) {
+                                        uint32_t tid = threadIdx.x, uint32_t tau = kTauMax) {
     constexpr int kLast = step_count(M) - 1;
     const StepMap<M, kLast, COL> sl(tid);
     step_regs<M, kLast, true, COL, inv_kind<M, kLast>()>(v, sl, tab, P, m);
@@ -201,7 +229,8 @@ __device__ __forceinline__ void inv_dft(double *v, double *lds, const double *ta
         lds_steps<M, true, COL, kLast - 1, 1>(lds, tab, P, m, tid);
         const StepMap<M, 0, COL> s0(tid);
         lds_load(v, lds, s0);
-        step_regs<M, 0, true, COL, FINAL>(v, s0, tab, P, m);
+        if constexpr (TRUNC) itft_step<M, COL>(v, s0, tab, P, m, tau);
+        else step_regs<M, 0, true, COL, FINAL>(v, s0, tab, P, m);
     }
 }
 
@@ -335,9 +364,26 @@ struct PassArgs {
     // (device arrays), or null when the operands above describe every product
     const RaggedRow *rows;
     const RaggedB *bset;
+    // truncation (ntt_plan.hpp): the parts of every transform in use and the
+    // deeper levels' tiles that hold them (with row_tau the most of any row:
+    // each ragged row uses its own)
+    uint32_t tau, tau_tiles, row_tau;
     // log2 of the tiles each XCD takes in turn (xcd_tile)
     int xcd_log2;
 };
+
+// The parts of its transform that row `row` of forward operand (or product)
+// `seg` needs.
+__device__ __forceinline__ uint32_t fwd_tau(const PassArgs &a, uint32_t seg, uint32_t row) {
+    if (!a.row_tau) return a.tau;
+    return seg ? a.bset[row].tau : tau_of((uint64_t)a.rows[row].L_a + a.rows[row].L_b, a.plan.log2K);
+}
+__device__ __forceinline__ uint32_t prod_tau(const PassArgs &a, uint32_t row) { return fwd_tau(a, 0, row); }
+// Whether a deeper level's tile t lies past those parts (ragged rows; the
+// grid has no such tiles otherwise).
+__device__ __forceinline__ bool past_tau(const PassArgs &a, uint32_t tau, uint32_t t) {
+    return a.row_tau && t >= tau_tiles(tiles_per_product(a.plan), tau);
+}
 
 // Global memory instructions between memory_first_begin() and
 // memory_first_end() issue at raised wave priority: a wave about to wait on
@@ -448,6 +494,15 @@ struct ColThread {
     __device__ __forceinline__ uint64_t off(int u) const { return off0 + ((uint64_t)u << ustep); }
     // plane position of element u (residues)
     __device__ __forceinline__ uint64_t poff(int u) const { return poff0 + (uint64_t)u * pstep; }
+    // whether the last-step values of small DFT u (k = u R .. u R + R - 1, all
+    // in one part) lie in the first parts, rows below rows_end
+    __device__ __forceinline__ bool part_used(int u, uint32_t rows_end) const {
+        constexpr int LR = col_last_lr(M);
+        const uint32_t delta = col_last_row_delta(M, u << LR);
+        // the last row of the parts that DFT u's threads hold
+        const uint32_t top = delta + (((256u >> (kTileLog2 - M)) - 1u) << LR);
+        return top < tau_rows(M, kTauMin) || col_last_row0(M, tid) + delta < rows_end;
+    }
     // plane position of last-step value k
     __device__ __forceinline__ uint64_t plast(int k) const {
         return plast0 + (uint64_t)col_last_row_delta(M, k) * prow;
@@ -491,7 +546,8 @@ __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_fwd_kern
     using CP = ColPair<M, PAIR>;
     __shared__ double lds_tiles[CP::kLdsWords];
     double *const lds = lds_tiles + CP::half() * CP::kTileStride;
-    const BlockPos bp = block_pos(a.op_start, a.n_ops, tiles_per_product(a.plan) >> CP::kLog2, a.xcd_log2);
+    const BlockPos bp = block_pos(a.op_start, a.n_ops, a.tau_tiles >> CP::kLog2, a.xcd_log2);
+    if (past_tau(a, fwd_tau(a, bp.seg, bp.row), bp.t << CP::kLog2)) return;
     const NttOp o = a.ops[bp.seg];
     const ColThread<M> ct(a.plan, level, (bp.t << CP::kLog2) + CP::half(), CP::vtid());
     double *T0 = a.T + o.base + (size_t)bp.row * plane_row_elems(a.plan);
@@ -509,6 +565,43 @@ __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_fwd_kern
     for (int k = 0; k < 16; ++k) T0[ct.plast(k)] = v0[k];
 #pragma unroll
     for (int k = 0; k < 16; ++k) T1[ct.plast(k)] = v1[k];
+}
+
+// Stores last-step values (TRUNC: those of rows below rows_end).
+template <int M, bool TRUNC>
+__device__ __forceinline__ void col_store_last(double *T, const double *v, const ColThread<M> &ct, uint32_t rows_end) {
+    if constexpr (!TRUNC) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) T[ct.plast(k)] = v[k];
+    } else {
+        constexpr int R = 1 << col_last_lr(M);
+#pragma unroll
+        for (int u = 0; u < 16 / R; ++u) {
+            // the values are final here (not computed under the condition,
+            // which would keep their inputs live as well)
+#pragma unroll
+            for (int j = 0; j < R; ++j) __asm__ volatile("" : : "v"(v[u * R + j]));
+            if (ct.part_used(u, rows_end)) {
+#pragma unroll
+                for (int j = 0; j < R; ++j) T[ct.plast(u * R + j)] = v[u * R + j];
+            }
+        }
+    }
+}
+// Loads them (zero where TRUNC leaves them out).
+template <int M, bool TRUNC>
+__device__ __forceinline__ void col_load_last(double *v, const double *T, const ColThread<M> &ct, uint32_t rows_end) {
+    constexpr int R = 1 << col_last_lr(M);
+#pragma unroll
+    for (int u = 0; u < 16 / R; ++u) {
+        if (!TRUNC || ct.part_used(u, rows_end)) {
+#pragma unroll
+            for (int j = 0; j < R; ++j) v[u * R + j] = T[ct.plast(u * R + j)];
+        } else {
+#pragma unroll
+            for (int j = 0; j < R; ++j) v[u * R + j] = 0.0;
+        }
+    }
 }
 
 // Limbs of one tile block for the first forward level: element u of the
@@ -551,7 +644,8 @@ __device__ __forceinline__ void load_limbs(uint32_t *x, const PassArgs &a, const
 // step, against three waves).  The 2^5 and 2^9-point levels would spill
 // at four and keep three.
 constexpr int limbs_waves(int m) { return m >= 6 && m <= 8 ? 4 : 3; }
-template <int M, bool PAIR>
+// TRUNC: only the rows of the transforms' first parts are stored.
+template <int M, bool PAIR, bool TRUNC>
 __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) __attribute__((amdgpu_waves_per_eu(limbs_waves(M))))
 ntt_col_fwd_limbs_kernel(PassArgs a, uint32_t total) {
     using CP = ColPair<M, PAIR>;
@@ -568,13 +662,13 @@ ntt_col_fwd_limbs_kernel(PassArgs a, uint32_t total) {
         const NttOp o = a.ops[bp.seg];
         double *T0 = a.T + o.base + (size_t)bp.row * plane_row_elems(a.plan);
         double *T1 = T0 + o.pstride;
+        const uint32_t rows_end = TRUNC ? tau_rows(M, fwd_tau(a, bp.seg, bp.row)) : 1u << M;
         double v[16];
 #pragma unroll
         for (int u = 0; u < 16; ++u) v[u] = (double)x[u];
         col_fwd_prime_late<M, 0>(v, lds, ct, a.tables);
         memory_first_begin();
-#pragma unroll
-        for (int k = 0; k < 16; ++k) T0[ct.plast(k)] = v[k];
+        col_store_last<M, TRUNC>(T0, v, ct, rows_end);
         memory_first_end();
 #pragma unroll
         for (int u = 0; u < 16; ++u) v[u] = (double)x[u];
@@ -587,8 +681,7 @@ ntt_col_fwd_limbs_kernel(PassArgs a, uint32_t total) {
         // the barrier at its end lets the next tile block reuse `lds`
         col_fwd_prime_late<M, 1>(v, lds, ct, a.tables);
         memory_first_begin();
-#pragma unroll
-        for (int k = 0; k < 16; ++k) T1[ct.plast(k)] = v[k];
+        col_store_last<M, TRUNC>(T1, v, ct, rows_end);
         memory_first_end();
         if (!more) break;
         w = wn;
@@ -611,7 +704,8 @@ template <int M>
 __global__ void __launch_bounds__(256) ntt_row_fused_kernel(PassArgs a) {
     __shared__ double lds[kLdsSlots];
     constexpr uint32_t kJ = 1u << (M - 4);
-    const BlockPos bp = block_pos(a.prod_start, a.n_prods, tiles_per_product(a.plan), a.xcd_log2);
+    const BlockPos bp = block_pos(a.prod_start, a.n_prods, a.tau_tiles, a.xcd_log2);
+    if (past_tau(a, prod_tau(a, bp.row), bp.t)) return;
     const NttProd pr = a.prods[bp.seg];
     const NttOp oa = a.ops[pr.a], ob = a.ops[pr.b];
     const uint64_t Kp = plane_row_elems(a.plan);
@@ -675,7 +769,7 @@ template <int M>
 __global__ void __launch_bounds__(256) ntt_row_pair_kernel(PassArgs a, uint32_t rows0, uint32_t rows1) {
     __shared__ double lds[kLdsSlots];
     constexpr uint32_t kJ = 1u << (M - 4);
-    const uint32_t tiles = tiles_per_product(a.plan);
+    const uint32_t tiles = a.tau_tiles;
     const uint32_t bid = xcd_tile(blockIdx.x, gridDim.x, a.xcd_log2);
     const uint32_t row = bid / tiles, t = bid % tiles;
     const NttOp ob = a.ops[a.prods[0].b];
@@ -723,24 +817,24 @@ __global__ void __launch_bounds__(256) ntt_row_pair_kernel(PassArgs a, uint32_t 
 // loaded from ct.plast(k)): inverse twiddle, inverse DFT; leaves the
 // thread's elements tid + 256 u in v.  The caller must make sure no thread
 // still reads `lds`.
-template <int M, int P, int FINAL = kDitLast>
+template <int M, int P, int FINAL = kDitLast, bool TRUNC = false>
 __device__ __forceinline__ void col_inv_prime(double *v, double *lds, const ColThread<M> &ct, const double *tables,
-                                              const ColTw &tw) {
+                                              const ColTw &tw, uint32_t tau = kTauMax) {
     const Mod m = mod_of(P);
     const double *tab = tables + P * kPrimeTable;
     column_twiddles<M>(v, tw, m);
-    inv_dft<M, true, FINAL>(v, lds, tab, P, m, ct.tid);
+    inv_dft<M, true, FINAL, TRUNC>(v, lds, tab, P, m, ct.tid, tau);
 }
 
-// Loads both primes' values of a column tile and their inverse column
-// twiddle table entries (every load before any store).
-template <int M>
+// Loads both primes' values of a column tile (TRUNC: its rows below rows_end)
+// and their inverse column twiddle table entries (every load before any
+// store).
+template <int M, bool TRUNC = false>
 __device__ __forceinline__ void col_inv_load(double *v0, double *v1, ColTw &tw0, ColTw &tw1, const PassArgs &a,
-                                             const ColThread<M> &ct, const double *T0, const double *T1) {
-#pragma unroll
-    for (int k = 0; k < 16; ++k) v0[k] = T0[ct.plast(k)];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) v1[k] = T1[ct.plast(k)];
+                                             const ColThread<M> &ct, const double *T0, const double *T1,
+                                             uint32_t rows_end = 1u << M) {
+    col_load_last<M, TRUNC>(v0, T0, ct, rows_end);
+    col_load_last<M, TRUNC>(v1, T1, ct, rows_end);
     tw0 = col_tw_load<M>(a.tables, ct.cg, ct.B0, true);
     tw1 = col_tw_load<M>(a.tables + kPrimeTable, ct.cg, ct.B0, true);
 }
@@ -752,7 +846,8 @@ __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_inv_kern
     using CP = ColPair<M, PAIR>;
     __shared__ double lds_tiles[CP::kLdsWords];
     double *const lds = lds_tiles + CP::half() * CP::kTileStride;
-    const BlockPos bp = block_pos(a.prod_start, a.n_prods, tiles_per_product(a.plan) >> CP::kLog2, a.xcd_log2);
+    const BlockPos bp = block_pos(a.prod_start, a.n_prods, a.tau_tiles >> CP::kLog2, a.xcd_log2);
+    if (past_tau(a, prod_tau(a, bp.row), bp.t << CP::kLog2)) return;
     const NttOp oa = a.ops[a.prods[bp.seg].a];
     const ColThread<M> ct(a.plan, level, (bp.t << CP::kLog2) + CP::half(), CP::vtid());
     double *T0 = a.T + oa.base + (size_t)bp.row * plane_row_elems(a.plan);
@@ -786,8 +881,9 @@ __device__ __forceinline__ uint32_t row_shr(uint32_t x) {
 // limb column sums s_j = w0_j + w1_(j-1) + w2_(j-2), which become limbs with
 // one neighbour shift and one ballot carry resolution per run; what passes
 // the run's top goes to the spill word (the carry engine adds it).
-template <int M, bool PAIR>
-__global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_inv_limbs_kernel(PassArgs a) {
+template <int M, bool PAIR, bool TRUNC>
+__global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) __attribute__((amdgpu_waves_per_eu(4)))
+ntt_col_inv_limbs_kernel(PassArgs a) {
     using CP = ColPair<M, PAIR>;
     __shared__ double lds_tiles[CP::kLdsWords];
     double *const lds = lds_tiles + CP::half() * CP::kTileStride;
@@ -807,15 +903,16 @@ __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_inv_limb
     const double *T0 = a.T + oa.base + (size_t)prod * plane_row_elems(a.plan);
     double v0[16], v1[16];
     ColTw tw0, tw1;
-    col_inv_load<M>(v0, v1, tw0, tw1, a, ct, T0, T0 + oa.pstride);
+    const uint32_t tau = TRUNC ? prod_tau(a, prod) : kTauMax;
+    col_inv_load<M, TRUNC>(v0, v1, tw0, tw1, a, ct, T0, T0 + oa.pstride, tau_rows(M, tau));
     // 1/K rides on the column twiddles (the inverse transform is linear):
     // one product per prime instead of one per value; the last inverse step
     // re-centres its outputs (|v| < p/2 + p/1024) for the recombination
     tw0.lb = mulp(tw0.lb, c_ntt.kinv[0][log2K], mod_of(0));
     tw1.lb = mulp(tw1.lb, c_ntt.kinv[1][log2K], mod_of(1));
-    col_inv_prime<M, 0, kDitToGarner>(v0, lds, ct, a.tables, tw0);
+    col_inv_prime<M, 0, kDitToGarner, TRUNC>(v0, lds, ct, a.tables, tw0, tau);
     __syncthreads();
-    col_inv_prime<M, 1, kDitToGarner>(v1, lds, ct, a.tables, tw1);
+    col_inv_prime<M, 1, kDitToGarner, TRUNC>(v1, lds, ct, a.tables, tw1, tau);
     // prime 1's elements wait in the thread's own LDS slots while the limbs
     // are formed (registers for the carry resolution)
     __syncthreads();
@@ -833,6 +930,7 @@ __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_inv_limb
     const uint64_t n_u0 = ct.off0;  // coefficient index of element u = 0
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
+        if (TRUNC && u >= (int)kTauMin && u >= (int)tau) break;  // uniform over the block
         const unsigned __int128 c = recombine(v0[u], lds[ct.lds0 + 272u * u]);
         const uint32_t w0 = (uint32_t)c, w1 = (uint32_t)(c >> 32), w2 = (uint32_t)(c >> 64);
         const uint32_t w1a = row_shr<1>(w1), w2a = row_shr<1>(w2), w2b = row_shr<2>(w2);
@@ -1147,14 +1245,14 @@ uint32_t device_cus() {
     }
     return (uint32_t)n;
 }
-template <int M, bool PAIR>
+template <int M, bool PAIR, bool TRUNC>
 __global__ void ntt_col_fwd_limbs_kernel(PassArgs a, uint32_t total);
-template <int M, bool PAIR>
+template <int M, bool PAIR, bool TRUNC>
 uint32_t persistent_grid(uint32_t total) {
     static std::atomic<int> per_cu{0};
     int b = per_cu.load(std::memory_order_relaxed);
     if (b == 0) {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, ntt_col_fwd_limbs_kernel<M, PAIR>,
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, ntt_col_fwd_limbs_kernel<M, PAIR, TRUNC>,
                                                          ColPair<M, PAIR>::kThreads, 0) != hipSuccess || b < 1)
             b = 1;
         per_cu.store(b, std::memory_order_relaxed);
@@ -1163,17 +1261,19 @@ uint32_t persistent_grid(uint32_t total) {
     return (uint32_t)std::min<uint64_t>(total, fit < kXcds ? kXcds : fit);
 }
 
-// Calls f(std::integral_constant<bool, PAIR>) with PAIR = pair where a level
-// of 2^M points can pair its tiles, false otherwise.
+// Calls f(PAIR, TRUNC) as std::integral_constants: PAIR = pair where a level of
+// 2^M points can pair its tiles, false otherwise.
 template <int M, typename F>
-void with_pair(bool pair, F &&f) {
+void with_flags(bool pair, bool trunc, F &&f) {
     if constexpr (col_pair_log2(M) > 0) {
         if (pair) {
-            f(std::true_type{});
+            if (trunc) f(std::true_type{}, std::true_type{});
+            else f(std::true_type{}, std::false_type{});
             return;
         }
     }
-    f(std::false_type{});
+    if (trunc) f(std::false_type{}, std::true_type{});
+    else f(std::false_type{}, std::false_type{});
 }
 
 // Spill words per product for any plan of size 2^k: runs are never shorter
@@ -1230,6 +1330,7 @@ hipError_t ntt_tables_init(NTTPrecomputedTables *tables) {
             cst.w16[q][e] = centred(powmod_u64(w16, e, P), P);
             cst.w16i[q][e] = centred(powmod_u64(w16i, e, P), P);
         }
+        cst.inv2[q] = centred((P + 1) / 2, P);
         for (int k = 0; k <= kMaxLog2; ++k)
             cst.kinv[q][k] = centred(powmod_u64(powmod_u64(2, k, P), P - 2, P), P);
     }
@@ -1308,6 +1409,7 @@ struct JobShape {
     bool op_bcast[3] = {false, false, false};
     uint32_t rows = 0;
     uint32_t Lc[2] = {0, 0};
+    uint32_t tau = kTauMax;  // parts of the transforms in use (the most of any product)
 };
 
 JobShape shape_of(const NttJob &j) {
@@ -1320,7 +1422,14 @@ JobShape shape_of(const NttJob &j) {
         sh.op_rows[pr.a] = std::max(sh.op_rows[pr.a], pr.N);
         sh.op_rows[pr.b] = std::max(sh.op_rows[pr.b], pr.N);
         used_as_a[pr.a] = true;
-        sh.Lc[q] = j.ragged ? (uint32_t)K : j.ops[pr.a].L + j.ops[pr.b].L;
+        // ragged rows are staged, K words apart
+        uint64_t total = j.ragged ? 0 : (uint64_t)j.ops[pr.a].L + j.ops[pr.b].L;
+        if (j.ragged && j.host_rows == nullptr) total = K;
+        else if (j.ragged)
+            for (uint32_t i = 0; i < pr.N; ++i)
+                total = std::max<uint64_t>(total, (uint64_t)j.host_rows[i].L_a + j.host_rows[i].L_b);
+        sh.Lc[q] = (uint32_t)total;
+        sh.tau = q == 0 ? tau_of(total, j.k) : std::max(sh.tau, tau_of(total, j.k));
     }
     for (uint32_t o = 0; o < j.n_ops; ++o) {
         sh.op_bcast[o] = !j.ragged && !used_as_a[o] && j.ops[o].s == 0 && sh.op_rows[o] > 1;
@@ -1458,26 +1567,42 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
     a.spill = reinterpret_cast<uint64_t *>(ws + l.spill_off);
     a.n_ops = j.n_ops;
     a.n_prods = j.n_prods;
+    // ragged rows are truncated when that leaves out a tenth of the launch's
+    // parts (the truncating first-level kernels are 5-10 % slower: 256 ragged
+    // pairs, most of them in pieces that fill their transforms, took 37.1 ms
+    // truncated wherever a row allowed it and 36.0 ms not truncated)
+    uint32_t tau = sh.tau;
+    if (j.ragged) {
+        uint64_t parts = 0;
+        for (uint32_t i = 0; i < sh.rows; ++i)
+            parts += tau_of((uint64_t)j.host_rows[i].L_a + j.host_rows[i].L_b, k);
+        a.row_tau = 10 * parts <= 9 * (uint64_t)kTauMax * sh.rows;
+        if (!a.row_tau) tau = kTauMax;
+    }
+    a.tau = tau;
+    a.tau_tiles = tau_tiles(tiles, tau);
+    const bool trunc = a.row_tau || tau < kTauMax;
     const size_t spill_stride = align256(l.spill_elems * sizeof(uint64_t)) / sizeof(uint64_t);
     for (size_t r0 = 0; r0 < sh.rows; r0 += l.nc) {
         // operands: rows of this chunk (a broadcast row only in the first)
-        uint64_t fwd_blocks = 0, limb_reads = 0;
-        uint32_t op_rows[3] = {0, 0, 0};
+        uint64_t fwd_rows = 0, limb_reads = 0;
+        uint32_t op_row0[3] = {0, 0, 0};
         for (uint32_t o = 0; o < j.n_ops; ++o) {
             const NttJob::Op &op = j.ops[o];
-            if (sh.op_bcast[o]) op_rows[o] = r0 == 0 ? 1u : 0u;
-            else op_rows[o] = (uint32_t)std::min<size_t>(l.nc, sh.op_rows[o] > r0 ? sh.op_rows[o] - r0 : 0);
+            uint32_t op_rows;
+            if (sh.op_bcast[o]) op_rows = r0 == 0 ? 1u : 0u;
+            else op_rows = (uint32_t)std::min<size_t>(l.nc, sh.op_rows[o] > r0 ? sh.op_rows[o] - r0 : 0);
             a.ops[o].X = op.X + (sh.op_bcast[o] ? 0 : r0 * op.s);
             a.ops[o].L = op.L;
             a.ops[o].s = op.s;
             a.ops[o].base = l.op_base[o];
             a.ops[o].pstride = l.plane_elems[o];
-            if (o < 3) a.op_start[o] = (uint32_t)fwd_blocks;
-            fwd_blocks += (uint64_t)op_rows[o] * tiles;
-            if (!j.ragged) limb_reads += (uint64_t)op_rows[o] * op.L;
+            op_row0[o] = (uint32_t)fwd_rows;
+            fwd_rows += op_rows;
+            if (!j.ragged) limb_reads += (uint64_t)op_rows * op.L;
         }
-        uint64_t prod_blocks = 0, prod_rows = 0, limb_writes = 0;
-        uint32_t rows[2] = {0, 0};
+        uint64_t prod_rows = 0, limb_writes = 0;
+        uint32_t rows[2] = {0, 0}, prod_row0[2] = {0, 0};
         for (uint32_t q = 0; q < j.n_prods; ++q) {
             const NttJob::Prod &pr = j.prods[q];
             rows[q] = (uint32_t)std::min<size_t>(l.nc, pr.N > r0 ? pr.N - r0 : 0);
@@ -1489,44 +1614,45 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
             d.sC = j.ragged ? (uint32_t)K : pr.sC;
             d.Lc = sh.Lc[q];
             d.spill_base = q * spill_stride;
-            a.prod_start[q] = (uint32_t)prod_blocks;
-            prod_blocks += (uint64_t)rows[q] * tiles;
+            prod_row0[q] = (uint32_t)prod_rows;
             prod_rows += rows[q];
             limb_writes += (uint64_t)rows[q] * d.Lc;
         }
-        if (fwd_blocks > 0x7fffffffull || prod_blocks > 0x7fffffffull) return hipErrorInvalidValue;
+        if (fwd_rows * tiles > 0x7fffffffull || prod_rows * tiles > 0x7fffffffull) return hipErrorInvalidValue;
         if (j.ragged) {
             a.rows = j.rows;
             a.bset = j.bset;
             for (uint32_t i = 0; i < rows[0]; ++i) limb_reads += j.host_rows[i].L_a;
             for (uint32_t b = 0; b < j.nb; ++b) limb_reads += j.host_bset[b].L;
         }
-        // algorithmic bytes: 16 B per residue pair (one binary64 per prime),
-        // 4 B per limb
-        const double fwd_tb = 16.0 * (double)(fwd_blocks / tiles) * (double)K;
-        const double prod_tb = 16.0 * (double)prod_rows * (double)K;
-        // a column level of 2^lm points runs 2^col_pair_log2(lm) tiles per
-        // block: block starts and grid in units of such blocks
-        const auto pair_log2_for = [&](int kind, int lm) {
-            return ((pair_mask >> kind) & 1u) ? col_pair_log2(lm) : 0;
-        };
-        const auto col_args = [&](int kind, int lm) {
+        // algorithmic bytes: 16 B per residue pair in use (one binary64 per
+        // prime; ragged rows at the most of any), 4 B per limb
+        const double row_bytes = 16.0 * (double)K * tau / kTauMax;
+        const double fwd_tb = row_bytes * (double)fwd_rows;
+        const double prod_tb = row_bytes * (double)prod_rows;
+        // a launch of row_tiles tiles per row: the segments' first blocks; a
+        // column level of 2^lm points runs 2^col_pair_log2(lm) tiles per block
+        const auto args = [&](uint32_t row_tiles, int pl) {
             PassArgs c = a;
-            const int pl = pair_log2_for(kind, lm);
-            for (int o = 0; o < 3; ++o) c.op_start[o] >>= pl;
-            for (int q = 0; q < 2; ++q) c.prod_start[q] >>= pl;
+            for (int o = 0; o < 3; ++o) c.op_start[o] = op_row0[o] * (row_tiles >> pl);
+            for (int q = 0; q < 2; ++q) c.prod_start[q] = prod_row0[q] * (row_tiles >> pl);
             return c;
         };
-        if (fwd_blocks > 0) {
+        const auto blocks = [](uint64_t n_rows, uint32_t row_tiles, int pl) {
+            return dim3((uint32_t)(n_rows * (row_tiles >> pl)));
+        };
+        const uint32_t deep = a.tau_tiles;
+        if (fwd_rows > 0) {
             GPUPI_RETURN_IF(timed(kColFwdLimbs, k, 4.0 * (double)limb_reads + fwd_tb, stream, [&] {
                 dispatch_m<kColLo, kColHi>(p.log2M[0], [&](auto mc) {
                     constexpr int M = decltype(mc)::value;
-                    with_pair<M>((pair_mask >> kPairFwdLimbs) & 1u, [&](auto pc) {
-                        constexpr int pl = ColPair<M, decltype(pc)::value>::kLog2;
-                        const uint32_t total = (uint32_t)(fwd_blocks >> pl);
-                        hipLaunchKernelGGL((ntt_col_fwd_limbs_kernel<M, decltype(pc)::value>),
-                                           dim3(persistent_grid<M, decltype(pc)::value>(total)), dim3(256 << pl), 0,
-                                           stream, col_args(kPairFwdLimbs, M), total);
+                    with_flags<M>((pair_mask >> kPairFwdLimbs) & 1u, trunc, [&](auto pc, auto tc) {
+                        constexpr bool kPair = decltype(pc)::value, kTrunc = decltype(tc)::value;
+                        constexpr int pl = ColPair<M, kPair>::kLog2;
+                        const uint32_t total = blocks(fwd_rows, tiles, pl).x;
+                        hipLaunchKernelGGL((ntt_col_fwd_limbs_kernel<M, kPair, kTrunc>),
+                                           dim3(persistent_grid<M, kPair, kTrunc>(total)), dim3(256 << pl), 0, stream,
+                                           args(tiles, pl), total);
                     });
                 });
             }));
@@ -1534,26 +1660,23 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
                 GPUPI_RETURN_IF(timed(kColFwd, k, 2 * fwd_tb, stream, [&] {
                     dispatch_m<kColLo, kColHi>(p.log2M[1], [&](auto mc) {
                         constexpr int M = decltype(mc)::value;
-                        with_pair<M>((pair_mask >> kPairFwd) & 1u, [&](auto pc) {
+                        with_flags<M>((pair_mask >> kPairFwd) & 1u, false, [&](auto pc, auto) {
                             constexpr int pl = ColPair<M, decltype(pc)::value>::kLog2;
-                            hipLaunchKernelGGL((ntt_col_fwd_kernel<M, decltype(pc)::value>),
-                                               dim3((uint32_t)(fwd_blocks >> pl)), dim3(256 << pl), 0, stream,
-                                               col_args(kPairFwd, M), 1);
+                            hipLaunchKernelGGL((ntt_col_fwd_kernel<M, decltype(pc)::value>), blocks(fwd_rows, deep, pl),
+                                               dim3(256 << pl), 0, stream, args(deep, pl), 1);
                         });
                     });
                 }));
             }
         }
-        if (prod_blocks == 0) continue;
+        if (prod_rows == 0) continue;
         if (j.n_prods == 2 && j.prods[0].b == j.prods[1].b && p.log2M[p.levels - 1] <= kPairMaxM) {
             // shared B: its last-level transform once per tile for both products
             const uint32_t pair_rows = std::max(rows[0], rows[1]);
-            const double pair_tb = 16.0 * (double)pair_rows * (double)K + 2 * prod_tb;
-            GPUPI_RETURN_IF(timed(kRowPair, k, pair_tb, stream, [&] {
+            GPUPI_RETURN_IF(timed(kRowPair, k, row_bytes * (double)pair_rows + 2 * prod_tb, stream, [&] {
                 dispatch_m<kRowLo, kRowHi>(p.log2M[p.levels - 1], [&](auto mc) {
-                    hipLaunchKernelGGL((ntt_row_pair_kernel<decltype(mc)::value>),
-                                       dim3((uint32_t)((uint64_t)pair_rows * tiles)), dim3(256), 0, stream, a,
-                                       rows[0], rows[1]);
+                    hipLaunchKernelGGL((ntt_row_pair_kernel<decltype(mc)::value>), blocks(pair_rows, deep, 0),
+                                       dim3(256), 0, stream, args(deep, 0), rows[0], rows[1]);
                 });
             }));
         } else {
@@ -1561,8 +1684,8 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
             const double row_tb = (j.prods[0].a == j.prods[0].b ? 2 : 3) * prod_tb;
             GPUPI_RETURN_IF(timed(kRowFused, k, row_tb, stream, [&] {
                 dispatch_m<kRowLo, kRowHi>(p.log2M[p.levels - 1], [&](auto mc) {
-                    hipLaunchKernelGGL((ntt_row_fused_kernel<decltype(mc)::value>), dim3((uint32_t)prod_blocks),
-                                       dim3(256), 0, stream, a);
+                    hipLaunchKernelGGL((ntt_row_fused_kernel<decltype(mc)::value>), blocks(prod_rows, deep, 0),
+                                       dim3(256), 0, stream, args(deep, 0));
                 });
             }));
         }
@@ -1570,27 +1693,26 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
             GPUPI_RETURN_IF(timed(kColInv, k, 2 * prod_tb, stream, [&] {
                 dispatch_m<kColLo, kColHi>(p.log2M[1], [&](auto mc) {
                     constexpr int M = decltype(mc)::value;
-                    with_pair<M>((pair_mask >> kPairInv) & 1u, [&](auto pc) {
+                    with_flags<M>((pair_mask >> kPairInv) & 1u, false, [&](auto pc, auto) {
                         constexpr int pl = ColPair<M, decltype(pc)::value>::kLog2;
-                        hipLaunchKernelGGL((ntt_col_inv_kernel<M, decltype(pc)::value>),
-                                           dim3((uint32_t)(prod_blocks >> pl)), dim3(256 << pl), 0, stream,
-                                           col_args(kPairInv, M), 1);
+                        hipLaunchKernelGGL((ntt_col_inv_kernel<M, decltype(pc)::value>), blocks(prod_rows, deep, pl),
+                                           dim3(256 << pl), 0, stream, args(deep, pl), 1);
                     });
                 });
             }));
         }
         GPUPI_RETURN_IF(timed(kColInvLimbs, k, prod_tb + 4.0 * (double)limb_writes + 8.0 * prod_rows * runs, stream,
                               [&] {
-                                  dispatch_m<kColLo, kColHi>(p.log2M[0], [&](auto mc) {
-                                      constexpr int M = decltype(mc)::value;
-                                      with_pair<M>((pair_mask >> kPairInvLimbs) & 1u, [&](auto pc) {
-                                          constexpr int pl = ColPair<M, decltype(pc)::value>::kLog2;
-                                          hipLaunchKernelGGL((ntt_col_inv_limbs_kernel<M, decltype(pc)::value>),
-                                                             dim3((uint32_t)(prod_blocks >> pl)), dim3(256 << pl),
-                                                             0, stream, col_args(kPairInvLimbs, M));
-                                      });
-                                  });
-                              }));
+            dispatch_m<kColLo, kColHi>(p.log2M[0], [&](auto mc) {
+                constexpr int M = decltype(mc)::value;
+                with_flags<M>((pair_mask >> kPairInvLimbs) & 1u, trunc, [&](auto pc, auto tc) {
+                    constexpr bool kPair = decltype(pc)::value;
+                    constexpr int pl = ColPair<M, kPair>::kLog2;
+                    hipLaunchKernelGGL((ntt_col_inv_limbs_kernel<M, kPair, decltype(tc)::value>),
+                                       blocks(prod_rows, tiles, pl), dim3(256 << pl), 0, stream, args(tiles, pl));
+                });
+            });
+        }));
         for (uint32_t q = 0; q < j.n_prods; ++q) {
             if (rows[q] == 0) continue;
             const NttProd &d = a.prods[q];
@@ -1741,6 +1863,8 @@ hipError_t launch_mul_ntt_shared(const uint32_t *A1, uint32_t L1, uint32_t s1, u
 
 int ntt_transform_log2(uint32_t L_a, uint32_t L_b) { return transform_log2(L_a, L_b); }
 
+uint32_t ntt_tau(uint32_t L_a, uint32_t L_b, int log2K) { return tau_of((uint64_t)L_a + L_b, log2K); }
+
 namespace {
 NttJob ragged_job(const RaggedRow *rows, const RaggedRow *host_rows, uint32_t N, const RaggedB *bset,
                   const RaggedB *host_bset, uint32_t nb, const RaggedAssembly *asms,
@@ -1771,7 +1895,9 @@ bool ragged_ok(const RaggedRow *rows, uint32_t N, const RaggedB *bset, uint32_t 
     const uint64_t K = 1ull << log2K;
     for (uint32_t i = 0; i < N; ++i) {
         const RaggedRow &r = rows[i];
-        if (r.b >= nb || (uint64_t)r.L_a + r.L_b > K || bset[r.b].L != r.L_b) return false;
+        if (r.b >= nb || (uint64_t)r.L_a + r.L_b > K || bset[r.b].L != r.L_b ||
+            bset[r.b].tau < tau_of((uint64_t)r.L_a + r.L_b, log2K) || bset[r.b].tau > kTauMax)
+            return false;
         if (r.C == nullptr && log2K <= kTileLog2) return false;
     }
     uint32_t next = 0;
@@ -1799,10 +1925,10 @@ namespace {
 // assembly, written on the device (no host upload).
 __global__ void __launch_bounds__(256) piece_rows_kernel(RaggedRow *rows, RaggedB *bset, RaggedAssembly *as,
                                                          const uint32_t *L, uint32_t LL, const uint32_t *S,
-                                                         uint32_t LS, uint32_t *C, uint32_t m, uint32_t s) {
+                                                         uint32_t LS, uint32_t *C, uint32_t m, uint32_t s, uint32_t tau) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i == 0) {
-        bset[0] = RaggedB{S, LS};
+        bset[0] = RaggedB{S, LS, tau};
         as[0] = RaggedAssembly{C, LL + LS, s, LS, m, 0, 0};
     }
     if (i < m) rows[i] = piece_row(i, L, LL, S, LS, m, s, 0);
@@ -1846,13 +1972,14 @@ hipError_t launch_mul_ntt_pieces(const uint32_t *L, uint32_t LL, const uint32_t 
     auto *rows = reinterpret_cast<RaggedRow *>(ws);
     auto *bset = reinterpret_cast<RaggedB *>(ws + l.rows_bytes);
     auto *as = reinterpret_cast<RaggedAssembly *>(ws + l.rows_bytes + l.bset_bytes);
+    const uint32_t tau = tau_of((uint64_t)s + LS, l.k);  // the longest pieces' parts
     hipLaunchKernelGGL(piece_rows_kernel, dim3((m + 255) / 256), dim3(256), 0, stream, rows, bset, as, L, LL, S, LS,
-                       C, m, s);
+                       C, m, s, tau);
     GPUPI_RETURN_IF(hipGetLastError());
     // the same descriptors on the host, for the launch's bookkeeping
     std::vector<RaggedRow> host_rows(m);
     for (uint32_t i = 0; i < m; ++i) host_rows[i] = piece_row(i, L, LL, S, LS, m, s, 0);
-    const RaggedB host_b{S, LS};
+    const RaggedB host_b{S, LS, tau};
     const RaggedAssembly host_as{C, LL + LS, s, LS, m, 0, 0};
     return run_ntt(ragged_job(rows, host_rows.data(), m, bset, &host_b, 1, as, &host_as, 1, l.chunks, l.k),
                    ws + l.rows_bytes + l.bset_bytes + l.asm_bytes, l.ntt_bytes, tables, stream);

@@ -263,5 +263,48 @@ GPUPI_HD void dit(double *v, const double *w16i, Mod m) {
     }
 }
 
+// Inverse of a truncated radix-S transform (S a power of two): v[0, T) hold
+// the first T of the S bit-reversed values, v[T, S) hold S times the inputs
+// T.. (known; zero at the top), and v[0, T) are left holding S times the
+// inputs below T.  With a and b the halves of the inputs, the first half of
+// the values is the transform of a + b, the second that of (a - b) w^i:
+// where the first half is known, so is a + b, and a known b gives a = (a + b)
+// - b and one more input a - b of the second half; where it is not, the known
+// a + b complete it (van der Hoeven's truncated Fourier transform).  Values
+// are re-centred throughout (inputs: |v| <= p except v[0] <= kBoundInvMid p
+// with T >= S / 2; outputs kRedBound p).
+template <int S, int T>
+GPUPI_HD void itft(double *v, const double *w16, const double *w16i, double inv2, Mod m) {
+    if constexpr (T == S && S > 1) {
+        dit<kDitToGarner, S>(v, w16i, m);
+    } else if constexpr (T > 0 && S > 1) {
+        constexpr int H = S / 2;
+        if constexpr (T >= H) {
+            itft<H, H>(v, w16, w16i, inv2, m);
+#pragma unroll
+            for (int i = T - H; i < H; ++i) {
+                const double l = v[i], b = v[H + i];
+                const int e = i * (16 / S);
+                if (T > H) v[H + i] = e ? mulp(l - b, w16[e], m) : redp(l - b, m);
+                v[i] = redp(2.0 * l - b, m);
+            }
+            itft<H, T - H>(v + H, w16, w16i, inv2, m);
+#pragma unroll
+            for (int i = 0; i < T - H; ++i) {
+                const int e = i * (16 / S);
+                const double a = v[i], t = e ? mulp(v[H + i], w16i[e], m) : v[H + i];
+                v[i] = redp(a + t, m);
+                v[H + i] = redp(a - t, m);
+            }
+        } else {
+#pragma unroll
+            for (int i = T; i < H; ++i) v[i] = mulp(v[i] + v[H + i], inv2, m);
+            itft<H, T>(v, w16, w16i, inv2, m);
+#pragma unroll
+            for (int i = 0; i < T; ++i) v[i] = redp(2.0 * v[i] - v[H + i], m);
+        }
+    }
+}
+
 }  // namespace ntt
 }  // namespace gpupi

@@ -193,6 +193,26 @@ GPUPI_HD constexpr uint32_t col_pair_vtid(uint32_t t, int lm) {
     return (t & ((1u << (kTileLog2 - lm)) - 1u)) | ((t >> (kTileLog2 - lm + col_pair_log2(lm))) << (kTileLog2 - lm));
 }
 
+// Truncated products.  The first forward step of the first level splits a
+// transform into kTauMax parts of K / kTauMax points (part j: the polynomial
+// modulo x^(K/16) - w16^bitrev(j)), so a product of `total` coefficients is
+// determined by its first tau = ceil(total kTauMax / K) parts: only they are
+// stored, transformed, multiplied and inverted, and the last inverse step
+// solves for the tau K / 16 coefficients they determine (itft).  In steps of
+// two from kTauMin: a transform is never below half full, except the last
+// piece of a product in pieces.
+constexpr uint32_t kTauMax = 16, kTauMin = 10;
+GPUPI_HD uint32_t tau_of(uint64_t total, int log2K) {
+    const uint32_t t = (uint32_t)((total * kTauMax + ((1ull << log2K) - 1ull)) >> log2K);
+    const uint32_t even = (t + 1u) & ~1u;
+    return even < kTauMin ? kTauMin : even;
+}
+// Tiles of a deeper level that hold the first tau parts (the rows of the
+// first level's 2D view come in order, part by part).
+GPUPI_HD uint32_t tau_tiles(uint32_t tiles, uint32_t tau) { return (tiles * tau + (kTauMax - 1u)) / kTauMax; }
+// Rows of the first level's 2D view (2^lm rows) in the first tau parts.
+GPUPI_HD uint32_t tau_rows(int lm, uint32_t tau) { return tau << (lm - 4); }
+
 GPUPI_HD uint32_t tiles_per_product(const Plan &p) { return 1u << (p.log2K - kTileLog2 > 0 ? p.log2K - kTileLog2 : 0); }
 
 // Row (last) level: tile t holds G = 4096 / M consecutive slabs.

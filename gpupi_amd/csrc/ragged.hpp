@@ -26,9 +26,10 @@ struct RaggedRow {
     uint32_t *C;
     uint32_t L_a, L_b, b, pad;
 };
+// tau: the parts of its transform that its rows need (ntt_plan.hpp).
 struct RaggedB {
     const uint32_t *B;
-    uint64_t L;
+    uint32_t L, tau;
 };
 // A product L * S (c = |L| + |S| limbs) run in m pieces of s limbs of L (the
 // last one shorter) against S: its pieces are the launch's rows row0 ..

@@ -662,3 +662,64 @@ def test_matrix_core_products(la, lb, n):
         g.synchronize()
         got = g.download_rows(vc, bufc)
         assert [value(r) for r in got] == [value(A[0]) * value(b) for b in B]
+
+
+@pytest.mark.parametrize("k", [13, 14, 16, 18, 20, 21, 22, 23, 24])
+def test_truncated_transforms(ctx, k):
+    """Products whose transforms use only some of their 16 parts: totals at
+    and next to every pair of parts of 2^k points, one row and several, equal
+    and unequal lengths, a broadcast operand, a square and a shared pair with
+    different numbers of parts, against GMP; nothing is written past a row."""
+    rng = np.random.default_rng(k)
+    K = 1 << k
+    totals = sorted({min(max(K * t // 16 + d, K // 2 + 1), K) for t in (8, 10, 12, 14, 16) for d in (-1, 0, 1)})
+    if k > 20:
+        totals = totals[1::3]
+    for i, total in enumerate(totals):
+        la = total // 2 if i % 2 else total // 2 - total // 11
+        lb = total - la
+        n = 3 if k < 18 and i % 3 == 0 else 1
+        A, B = rand_rows(rng, n, la, "random" if i % 4 else "ones"), rand_rows(rng, n, lb, "random" if i % 5 else "ones")
+        assert np.array_equal(device_mul(ctx, A, B), oracle_mul(A, B)), (total, n)
+        if n > 1:
+            assert np.array_equal(device_mul(ctx, A, B, b_broadcast=True), oracle_mul(A, np.repeat(B[:1], n, axis=0)))
+        if i % 3 == 1:
+            buf, va = g.upload_rows(A)
+            bufc, vc = g.upload_rows(np.zeros((n, 2 * la), np.uint32))
+            g.check(ctx.mul(va, va, vc), "square")
+            g.synchronize()
+            assert np.array_equal(g.download_rows(vc, bufc), oracle_mul(A, A))
+    la1, la2, lb = K // 4 + 5, K // 2 - 3, K // 4 + 77
+    A1, A2, B = (rand_rows(rng, 1, n, "random") for n in (la1, la2, lb))
+    (b1, v1), (b2, v2), (bb, vb) = g.upload_rows(A1), g.upload_rows(A2), g.upload_rows(B)
+    c1, w1 = g.upload_rows(np.zeros((1, la1 + lb), np.uint32))
+    c2, w2 = g.upload_rows(np.zeros((1, la2 + lb), np.uint32))
+    g.check(ctx.mul_shared(v1, v2, vb, w1, w2), "mul_shared")
+    g.synchronize()
+    assert np.array_equal(g.download_rows(w1, c1), oracle_mul(A1, B))
+    assert np.array_equal(g.download_rows(w2, c2), oracle_mul(A2, B))
+
+
+def test_truncated_transforms_in_ragged_calls(ctx):
+    """Ragged rows of one transform size with different numbers of parts,
+    some sharing an operand, with the pieces of unbalanced products."""
+    rng = np.random.default_rng(16)
+    K = 1 << 15
+    lengths = [(K * t // 32 + d, K * t // 32) for t in range(9, 17) for d in (-1, 0)]
+    lengths += [(K - 4000, 4000), (300, K - 301), (1 << 20, 5000), ((1 << 20) + 12345, 30000), (700000, 600000)]
+    ops = [(rand_rows(rng, 1, a, "random")[0], rand_rows(rng, 1, b, "random")[0]) for a, b in lengths]
+    shared = ops[3][1]
+    ops += [(rand_rows(rng, 1, n, "random")[0], shared) for n in (K // 4 + 100, K // 2 - 1)]
+    keep, items, outs = [], [], []
+    sb = g.DeviceBuffer.from_array(shared)
+    for a, b in ops:
+        ba, bb = g.DeviceBuffer.from_array(a), sb if b is shared else g.DeviceBuffer.from_array(b)
+        bc = g.DeviceBuffer(4 * (a.size + b.size))
+        keep += [ba, bb]
+        outs.append(bc)
+        items.append((ba.ptr, bb.ptr, bc.ptr, a.size, b.size))
+    g.check(ctx.mul_ragged(items), "mul_ragged")
+    g.synchronize()
+    for (a, b), bc in zip(ops, outs):
+        want = oracle_mul(a.reshape(1, -1), b.reshape(1, -1))[0]
+        assert np.array_equal(bc.download(np.uint32, count=want.size), want), (a.size, b.size)

@@ -57,3 +57,16 @@ def test_ragged_assembly_rules(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=600)
     assert out.returncode == 0, out.stdout + out.stderr
     assert "ragged assembly check: ok" in out.stdout
+
+
+def test_truncated_transforms(tmp_path):
+    """Transforms of which only some parts are computed: the last inverse
+    step from any number of known values (gpupi_amd/csrc/ntt_arith.hpp, itft)
+    against 128-bit modular arithmetic on values at their bounds, the parts
+    every total needs, and the rows, tiles and thread values that hold them."""
+    exe = tmp_path / "itft_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-I", os.path.join(ROOT, "gpupi_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "native", "itft_check.cpp"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=600)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert "itft check: ok" in out.stdout
