@@ -48,9 +48,10 @@ typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 constexpr uint32_t kTileLimbs = 256;
 constexpr uint32_t kMaxTiles = 32;
 constexpr uint32_t kPassBias = 1u << 24;
+constexpr uint32_t kManyG = 8, kFewG = 5;  // tiles per wave at most: many rows, few rows
 
 // Blocks of 32 digits of an operand (its digits and the recoding's carry).
-inline uint32_t blocks_of(uint32_t L) { return L / 8u + 1u; }
+__host__ __device__ inline uint32_t blocks_of(uint32_t L) { return L / 8u + 1u; }
 
 // How a product runs: W groups of tiles (wave w takes the tiles w, w + W,
 // ...), and steps i0 < i0_end in each of which a wave multiplies the blocks
@@ -61,7 +62,8 @@ struct MfmaArgs {
     uint32_t *C;
     uint32_t LA, LB, sA, sB, sC;
     uint32_t W, M, E, na, nb, i0_end, m_thr;
-    uint32_t a_words, b_half, lds_words;  // LDS words: a, half of b, all but the column sums
+    uint32_t a_words, b_lead, b_half, lds_words;  // LDS words: a, zeros below b and a half of it, all but the column sums
+    const RaggedRow *rows;                        // ragged launches: a product per row
 };
 
 MfmaArgs shape_of(uint32_t LA, uint32_t LB, uint32_t W) {
@@ -77,7 +79,8 @@ MfmaArgs shape_of(uint32_t LA, uint32_t LB, uint32_t W) {
     s.m_thr = s.na + 1u - 32u * W * (s.M - 1u);
     s.E = (s.nb - 1u + s.i0_end - 1u) / (32u * W) + 1u;
     s.a_words = (8u * (s.i0_end + 32u * W * (s.M - 1u)) + 17u + 3u) & ~3u;
-    s.b_half = 4u * (32u * W * s.E + s.i0_end - 1u);
+    s.b_lead = 4u * (s.i0_end - 1u);
+    s.b_half = 4u * 32u * W * s.E + s.b_lead;
     s.lds_words = s.a_words + 2 * s.b_half + 2 * kMaxTiles;
     return s;
 }
@@ -262,12 +265,15 @@ __device__ __forceinline__ void tile_store(uint32_t *c, uint32_t l, uint32_t Lc,
     }
 }
 
+// RAGGED (S > 1, G = 5): block i multiplies row i's operands, of any lengths
+// that W takes; M and E are one of three shapes with M + E - 1 = 5 chosen per
+// block, and fragments a product does not reach are zero.
 // One product per block, W tile groups (WT: W where it is known, else 0).
 // S = 1: one wave per group, finishing its own tiles.  S > 1: S waves per
 // group, part ks of them taking the steps ks, ks + S, ...; the parts' column
 // sums meet in LDS and each wave finishes a tile or two.
 constexpr int mfma_waves(int g) { return g <= 1 ? 8 : g <= 2 ? 6 : g <= 5 ? 4 : 2; }
-template <int M, int E, int WT, int S>
+template <int M, int E, int WT, int S, bool RAGGED = false>
 __global__ void __launch_bounds__(S == 1 ? 256 : 1024) __attribute__((amdgpu_waves_per_eu(mfma_waves(M + E - 1))))
 mul_mfma_kernel(MfmaArgs a) {
     constexpr int G = M + E - 1;
@@ -277,9 +283,22 @@ mul_mfma_kernel(MfmaArgs a) {
     const uint32_t W = WT > 0 ? (uint32_t)WT : a.W;
     const uint32_t TW = W * S;  // waves per product
     const uint32_t ks = S > 1 ? wid / W : 0u, tw = wid - ks * W;
-    const size_t row = blockIdx.x;
+    const size_t row = RAGGED ? 0 : blockIdx.x;
+    if constexpr (RAGGED) {
+        const RaggedRow rr = a.rows[blockIdx.x];
+        const bool swap = rr.L_a > rr.L_b;
+        a.A = swap ? rr.B : rr.A;
+        a.B = swap ? rr.A : rr.B;
+        a.C = rr.C;
+        a.LA = swap ? rr.L_b : rr.L_a;
+        a.LB = swap ? rr.L_a : rr.L_b;
+        a.na = blocks_of(a.LA);
+        a.nb = blocks_of(a.LB);
+        a.i0_end = min(32u * W - 1u, a.na) + 1u;
+        a.m_thr = a.i0_end;
+    }
     uint32_t *const a_s = lds + 8;
-    const uint32_t b_lead = 4u * (a.i0_end - 1u);
+    const uint32_t b_lead = a.b_lead;
     uint32_t *const b_s = lds + a.a_words + b_lead;
     uint32_t *const h_s = lds + a.a_words + 2 * a.b_half;  // per tile: what it passes on
     uint32_t *const f_s = h_s + kMaxTiles;                 // per tile: carry out for a carry-in of 0, 1
@@ -293,9 +312,9 @@ mul_mfma_kernel(MfmaArgs a) {
         const uint32_t t = wid * kWave + lane, step = TW * kWave;
         zero_quads(a_s - 8, 2, t, step);
         zero_quads(a_s + 8 * a.na, (a.a_words - 8u - 8u * a.na) / 4u, t, step);
-        zero_quads(b_s - b_lead, a.i0_end - 1u, t, step);
-        zero_quads(b_s - b_lead + a.b_half, a.i0_end - 1u, t, step);
-        const uint32_t above = a.b_half / 4u - (a.i0_end - 1u) - a.nb;
+        zero_quads(b_s - b_lead, b_lead / 4u, t, step);
+        zero_quads(b_s - b_lead + a.b_half, b_lead / 4u, t, step);
+        const uint32_t above = (a.b_half - b_lead) / 4u - a.nb;
         zero_quads(b_s + 4 * a.nb, above, t, step);
         zero_quads(b_s + a.b_half + 4 * a.nb, above, t, step);
         if (S > 1) zero_quads(d_s, W * G * 256u, t, step);
@@ -316,15 +335,31 @@ mul_mfma_kernel(MfmaArgs a) {
     for (int g = 0; g < G; ++g)
 #pragma unroll
         for (int k = 0; k < 16; ++k) acc[g][k] = (k & 3) == 3 && ks == 0 ? -1 : 0;
+    uint32_t i0 = ks;
+    if constexpr (RAGGED) {
+        static_assert(S > 1 && G == (int)kFewG, "every shape has G tiles");
+        const uint32_t m_row = a.na / (32u * W) + 1u, e_row = (a.nb - 1u + a.i0_end - 1u) / (32u * W) + 1u;
+        const uint32_t first = min(a.i0_end, 32u * (tw + 1u));
+        if (m_row <= 1u) {
+            steps_mfma<1, 0, 5, S>(acc, i0, first, first, 0u, a_l, b_l, W, sh);
+            steps_mfma<1, 1, 5, S>(acc, i0, a.i0_end, a.i0_end, 0u, a_l, b_l, W, sh);
+        } else if (e_row > 3u) {
+            steps_mfma<2, 0, 4, S>(acc, i0, first, first, 0u, a_l, b_l, W, sh);
+            steps_mfma<2, 1, 4, S>(acc, i0, a.i0_end, a.i0_end, 0u, a_l, b_l, W, sh);
+        } else {
+            steps_mfma<3, 0, 3, S>(acc, i0, first, first, 0u, a_l, b_l, W, sh);
+            steps_mfma<3, 1, 3, S>(acc, i0, a.i0_end, a.i0_end, 0u, a_l, b_l, W, sh);
+        }
+    } else {
     // from e_thr on the last of the E blocks reaches digits of b; from f_thr
     // on the first one lies below them
     const uint32_t e_thr = (uint32_t)max(32 * (int)(tw + W * (E - 1)) - (int)(a.nb - 1u), 0);
-    uint32_t i0 = ks;
     if constexpr (WT == 1) {
         steps_mfma<M, 0, E, S>(acc, i0, a.i0_end, a.m_thr, e_thr, a_l, b_l, W, sh);
     } else {
         steps_mfma<M, 0, E, S>(acc, i0, min(a.i0_end, 32u * (tw + 1u)), a.m_thr, e_thr, a_l, b_l, W, sh);
         steps_mfma<M, 1, E, S>(acc, i0, a.i0_end, a.m_thr, e_thr, a_l, b_l, W, sh);
+    }
     }
 
     uint32_t *const c = a.C + row * a.sC;
@@ -408,7 +443,6 @@ mul_mfma_kernel(MfmaArgs a) {
 }
 
 typedef void (*MfmaKernel)(MfmaArgs);
-constexpr uint32_t kManyG = 8, kFewG = 5;  // tiles per wave at most
 constexpr int kParts = 4;
 // Calls f with the kernels <M, E> for M <= E, M + E - 1 <= GMAX in turn until
 // it returns true.
@@ -419,6 +453,9 @@ bool each_kernel(F &&f) {
     else if constexpr (2 * M + 1 <= (int)GMAX) return each_kernel<M + 1, M + 1, WT, S, GMAX>(f);
     else return false;
 }
+
+constexpr uint32_t kRaggedMaxW = 4;
+const MfmaKernel kRaggedKernel = mul_mfma_kernel<3, 3, 0, kParts, true>;
 
 // The kernels of several parts may take more than 64 KB of LDS; the attribute
 // is a property of the current device, set once per device (serving threads
@@ -437,6 +474,7 @@ hipError_t allow_large_lds() {
         return err != hipSuccess;
     });
     GPUPI_RETURN_IF(err);
+    GPUPI_RETURN_IF(hipFuncSetAttribute((const void *)kRaggedKernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     g_lds_done |= bit;
     return hipSuccess;
 }
@@ -483,6 +521,31 @@ hipError_t launch_mul_mfma(const uint32_t *A, const uint32_t *B, uint32_t *C, ui
     if (k == nullptr || tiles > kMaxTiles || W > 4 || lds > 160 * 1024) return hipErrorInvalidValue;
     if (lds > 65536) GPUPI_RETURN_IF(allow_large_lds());
     hipLaunchKernelGGL(k, dim3(N), dim3(kWave * W * (few ? kParts : 1)), lds, stream, a);
+    return hipGetLastError();
+}
+
+uint32_t mul_mfma_groups(uint32_t L_a, uint32_t L_b) {
+    const uint32_t LA = std::min(L_a, L_b), LB = std::max(L_a, L_b);
+    uint32_t W = 1;
+    MfmaArgs a = shape_of(LA, LB, W);
+    while (a.M + a.E - 1 > kFewG) a = shape_of(LA, LB, ++W);
+    return W;
+}
+
+hipError_t launch_mul_mfma_ragged(const RaggedRow *rows, uint32_t N, uint32_t W, hipStream_t stream) {
+    if (N == 0) return hipSuccess;
+    if (rows == nullptr || W < 1 || W > kRaggedMaxW || N > 0x7fffffffu) return hipErrorInvalidValue;
+    MfmaArgs a{};
+    a.rows = rows;
+    a.W = W;
+    // LDS for the longest operands of any shape: three blocks of a, five of b
+    a.a_words = 256u * W * 3u + 20u;
+    a.b_lead = 4u * (32u * W - 1u);
+    a.b_half = 4u * 32u * W * 5u + a.b_lead;
+    a.lds_words = a.a_words + 2 * a.b_half + 2 * kMaxTiles;
+    const size_t lds = (a.lds_words + W * kFewG * 1024u) * 4u;
+    if (lds > 65536) GPUPI_RETURN_IF(allow_large_lds());
+    hipLaunchKernelGGL(kRaggedKernel, dim3(N), dim3(kWave * W * kParts), lds, stream, a);
     return hipGetLastError();
 }
 

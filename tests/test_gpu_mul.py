@@ -723,3 +723,43 @@ def test_truncated_transforms_in_ragged_calls(ctx):
     for (a, b), bc in zip(ops, outs):
         want = oracle_mul(a.reshape(1, -1), b.reshape(1, -1))[0]
         assert np.array_equal(bc.download(np.uint32, count=want.size), want), (a.size, b.size)
+
+
+@pytest.mark.parametrize("count", [3, 40, 300])
+def test_ragged_small_products(ctx, count):
+    """Ragged calls of products the matrix cores take (1..4088 limbs in all,
+    every number of tile groups, one launch up to 256 of them and several
+    above), with empty operands, tiny ones, a shared operand and products at
+    the NTT's side of the limit, against Python integers."""
+    rng = np.random.default_rng(count)
+    lengths = [(1, 1), (0, 7), (5, 3000), (17, 17), (256, 257), (1016, 1016), (2044, 2044), (1016, 3072), (2045, 2044),
+               (3900, 188), (4000, 3), (40, 4040), (1500, 1500), (700, 3300), (5000, 4000), (6000, 5)]
+    while len(lengths) < count:
+        lengths.append(tuple(int(2 ** u) for u in rng.uniform(0, 11, size=2)))
+    lengths = lengths[:count] if count > 3 else [(300, 20), (1, 900), (4000, 88)]
+    ops = []
+    for i, (a, b) in enumerate(lengths):
+        A, B = (rng.integers(0, 1 << 32, size=n, dtype=np.uint32) for n in (a, b))
+        if i % 5 == 1:
+            A[:] = 0x7F7F7F7F
+        if i % 7 == 2:
+            B[:] = 0xFFFFFFFF
+        ops.append((A, ops[3][1] if i == 20 else B))
+    keep, items, outs = [], [], []
+    for A, B in ops:
+        ba, bb = g.DeviceBuffer.from_array(A), g.DeviceBuffer.from_array(B)
+        bc = g.DeviceBuffer.from_array(np.full(A.size + B.size + 1, PAD, dtype=np.uint32))
+        keep += [ba, bb]
+        outs.append(bc)
+        items.append((ba.ptr, bb.ptr, bc.ptr, A.size, B.size))
+    ctx.set_ntt_threshold(4089)
+    try:
+        g.check(ctx.mul_ragged(items), "mul_ragged")
+        g.synchronize()
+    finally:
+        g.check(ctx.set_ntt_threshold(384))
+    for (A, B), bc in zip(ops, outs):
+        got = bc.download(np.uint32, count=A.size + B.size + 1)
+        want = int.from_bytes(A.tobytes(), "little") * int.from_bytes(B.tobytes(), "little")
+        assert int.from_bytes(got[:-1].tobytes(), "little") == want, (A.size, B.size)
+        assert got[-1] == PAD, (A.size, B.size)
