@@ -187,42 +187,91 @@ __global__ void __launch_bounds__(256) carry_fixup_kernel(uint32_t *C, uint32_t 
     }
 }
 
+// Rows of 2..kRowWaves chunks of 1024 limbs run as one block per row (a wave
+// per chunk, ROW): the waves' (carry out, all propagate) flags meet in LDS,
+// so no second kernel settles the carries between chunks.  Short launches are
+// bound by the time of a launch: one addition of 16000 limbs takes 4.4 us
+// instead of 6.8 with carry_fixup_kernel behind it, 64 of them 5.8 instead of
+// 6.8, and full chips gain too, by one reading of the flags (8192 rows of 4000
+// limbs 73 instead of 78, 1024 of 16000 limbs 35.3 instead of 36.3 us).
+// Sixteen waves are the largest block.
+constexpr uint32_t kRowWaves = 16;
+
+// Which chunk a wave works on.
+struct ChunkPos {
+    uint32_t row, chunk;
+    bool valid;
+    uint64_t wave;
+};
+template <bool ROW>
+__device__ __forceinline__ ChunkPos chunk_pos(uint32_t chunks_per_row, uint64_t total_chunks) {
+    ChunkPos p;
+    if constexpr (ROW) {
+        p.row = blockIdx.x;
+        p.chunk = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+        p.valid = true;
+        p.wave = 0;
+    } else {
+        p.wave = (uint64_t)blockIdx.x * (256 / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+        p.valid = p.wave < total_chunks;
+        p.row = (uint32_t)(p.wave / chunks_per_row);
+        p.chunk = (uint32_t)(p.wave - (uint64_t)p.row * chunks_per_row);
+    }
+    return p;
+}
+
+// The carry into a wave of a ROW block from the waves below it: G, P are the
+// masks of its kSeg groups of 256 limbs (four per lane, settled within it).
+constexpr int kSeg = 4;
+__device__ __forceinline__ uint32_t carry_into_wave(const uint64_t *G, const uint64_t *P, uint32_t lane) {
+    __shared__ uint32_t flags[kRowWaves];
+    uint32_t cout = 0;
+    bool all_prop = true;
+#pragma unroll
+    for (int s = 0; s < kSeg; ++s) {
+        (void)resolve_carries(G[s], P[s], cout, &cout);
+        all_prop = all_prop && P[s] == ~0ull;
+    }
+    const uint32_t w = threadIdx.x / kWave;
+    if (lane == 0) flags[w] = cout | (all_prop ? 2u : 0u);
+    __syncthreads();
+    uint32_t cin = 0;
+    for (uint32_t i = 0; i < w; ++i) cin = (flags[i] & 1u) | ((flags[i] >> 1) & cin);
+    return __builtin_amdgcn_readfirstlane(cin);
+}
+
 // The spill-add of NTT products of more than 512 limbs with four limbs per
 // lane (16-byte loads and stores at any limb): one wave per chunk of 1024
 // limbs of one row.  Each lane settles its four limbs for a carry-in of zero,
 // the lanes' (generate, propagate) pairs go through one ballot resolution per
 // 256 limbs, and the lane adds its carry-in.
-__global__ void __launch_bounds__(256) spill_add_vec_kernel(uint32_t *C, uint32_t stride_C, uint32_t L_c,
-                                                            SpillArgs sp, uint32_t chunks_per_row,
-                                                            uint64_t total_chunks, uint8_t *flags) {
-    constexpr int kSeg = 4;  // 4 x 256 limbs per wave
-    const uint64_t wave = (uint64_t)blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
-    if (wave >= total_chunks) return;
+template <bool ROW>
+__global__ void __launch_bounds__(ROW ? kRowWaves * kWave : 256)
+spill_add_vec_kernel(uint32_t *C, uint32_t stride_C, uint32_t L_c, SpillArgs sp, uint32_t chunks_per_row,
+                     uint64_t total_chunks, uint8_t *flags) {
+    const ChunkPos pos = chunk_pos<ROW>(chunks_per_row, total_chunks);
+    if (!pos.valid) return;
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t row = (uint32_t)(wave / chunks_per_row);
-    const uint32_t chunk = (uint32_t)(wave - (uint64_t)row * chunks_per_row);
-    uint32_t *out = C + (size_t)row * stride_C;
-    const uint64_t *rsp = sp.spill + (size_t)row * sp.runs_per_row;
+    uint32_t *out = C + (size_t)pos.row * stride_C;
+    const uint64_t *rsp = sp.spill + (size_t)pos.row * sp.runs_per_row;
     const uint32_t run_mask = (1u << sp.run_log2) - 1u;
-    uint32_t x[kSeg][4];
+    const uint32_t base = pos.chunk * (uint32_t)(kSeg * 4 * kWave) + 4 * lane;
+    uint32_t r[kSeg][4];
+    uint64_t G[kSeg], P[kSeg];
 #pragma unroll
     for (int s = 0; s < kSeg; ++s) {
-        const uint32_t j0 = chunk * (uint32_t)(kSeg * 4 * kWave) + (uint32_t)s * (4 * kWave) + 4 * lane;
+        const uint32_t j0 = base + (uint32_t)s * (4 * kWave);
         if (j0 + 4 <= L_c) {
             const Quad v = *reinterpret_cast<const Quad *>(out + j0);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) x[s][t] = v.w[t];
+            for (int t = 0; t < 4; ++t) r[s][t] = v.w[t];
         } else {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) x[s][t] = j0 + t < L_c ? out[j0 + t] : 0u;
+            for (int t = 0; t < 4; ++t) r[s][t] = j0 + t < L_c ? out[j0 + t] : 0u;
         }
     }
-    uint32_t cin = 0;
-    bool all_prop = true;
-#pragma unroll
-    for (int s = 0; s < kSeg; ++s) {
-        const uint32_t j0 = chunk * (uint32_t)(kSeg * 4 * kWave) + (uint32_t)s * (4 * kWave) + 4 * lane;
-        uint32_t r[4];
+    const auto settle = [&](int s) {
+        const uint32_t j0 = base + (uint32_t)s * (4 * kWave);
         uint32_t c = 0;
         bool ones = true;
 #pragma unroll
@@ -234,34 +283,46 @@ __global__ void __launch_bounds__(256) spill_add_vec_kernel(uint32_t *C, uint32_
                 const uint64_t w = rsp[q - 1];
                 y = rem == 0 ? (uint32_t)w : (uint32_t)(w >> 32);
             }
-            const uint32_t d = x[s][t] + y;
+            const uint32_t d = r[s][t] + y;
             const uint32_t g = d < y ? 1u : 0u;
-            r[t] = d + c;
+            r[s][t] = d + c;
             c = g | (c & (d == 0xffffffffu ? 1u : 0u));
-            ones = ones && r[t] == 0xffffffffu && j < L_c;
+            ones = ones && r[s][t] == 0xffffffffu && j < L_c;
         }
-        const bool valid = j0 < L_c;
-        const uint64_t G = ballot64(valid && c != 0), P = ballot64(valid && ones);
+        G[s] = ballot64(j0 < L_c && c != 0);
+        P[s] = ballot64(j0 < L_c && ones);
+    };
+    uint32_t cin = 0;
+    if constexpr (ROW) {
+#pragma unroll
+        for (int s = 0; s < kSeg; ++s) settle(s);
+        cin = carry_into_wave(G, P, lane);
+    }
+    bool all_prop = true;
+#pragma unroll
+    for (int s = 0; s < kSeg; ++s) {
+        if constexpr (!ROW) settle(s);
+        const uint32_t j0 = base + (uint32_t)s * (4 * kWave);
         uint32_t cout;
-        const uint64_t cm = resolve_carries(G, P, cin, &cout);
+        const uint64_t cm = resolve_carries(G[s], P[s], cin, &cout);
         uint32_t ci = (uint32_t)(cm >> lane) & 1u;
+        Quad q;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const uint32_t v = r[t] + ci;
-            ci = ci & (r[t] == 0xffffffffu ? 1u : 0u);
-            r[t] = v;
+            q.w[t] = r[s][t] + ci;
+            ci = ci & (r[s][t] == 0xffffffffu ? 1u : 0u);
         }
         if (j0 + 4 <= L_c) {
-            *reinterpret_cast<Quad *>(out + j0) = Quad{{r[0], r[1], r[2], r[3]}};
+            *reinterpret_cast<Quad *>(out + j0) = q;
         } else {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-                if (j0 + t < L_c) out[j0 + t] = r[t];
+                if (j0 + t < L_c) out[j0 + t] = q.w[t];
         }
-        all_prop = all_prop && (P == ~0ull);
+        all_prop = all_prop && (P[s] == ~0ull);
         cin = cout;
     }
-    if (flags != nullptr && lane == 0) flags[wave] = (uint8_t)(cin | (all_prop ? 2u : 0u));
+    if (flags != nullptr && lane == 0) flags[pos.wave] = (uint8_t)(cin | (all_prop ? 2u : 0u));
 }
 
 // The assembly holding launch chunk g (assemblies in chunk order).
@@ -384,28 +445,29 @@ __device__ __forceinline__ void load4(const uint32_t *r, int64_t j0, uint32_t L,
 }
 
 // The ops on rows of more than 512 limbs, four limbs per lane: one wave per
-// chunk of 1024 limbs of one row (carry_fixup_kernel completes longer rows).
+// chunk of 1024 limbs of one row (up to 16 chunks meet in one block,
+// carry_fixup_kernel completes longer rows).
 // Bound by HBM; the 16-byte accesses start at any limb, so row strides and
 // shifts need no alignment (R = (R1 << s) - R2 over 512 rows of 128249 limbs:
 // 271 us with a limb per lane, 158 us this way).
-template <AddSubKind K>
-__global__ void __launch_bounds__(256) addsub_vec_kernel(AddSubArgs a, uint32_t chunks_per_row, uint64_t total_chunks, uint8_t *flags) {
+template <AddSubKind K, bool ROW>
+__global__ void __launch_bounds__(ROW ? kRowWaves * kWave : 256)
+addsub_vec_kernel(AddSubArgs a, uint32_t chunks_per_row, uint64_t total_chunks, uint8_t *flags) {
     constexpr bool kSub = OpTraits<K>::kSub;
     constexpr bool kShift = K == AddSubKind::ShiftAdd || K == AddSubKind::ShiftSub;
-    constexpr int kSeg = 4;  // 4 x 256 limbs per wave
-    const uint64_t wave = (uint64_t)blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
-    if (wave >= total_chunks) return;
+    const ChunkPos pos = chunk_pos<ROW>(chunks_per_row, total_chunks);
+    if (!pos.valid) return;
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t row = (uint32_t)(wave / chunks_per_row);
-    const uint32_t chunk = (uint32_t)(wave - (uint64_t)row * chunks_per_row);
+    const uint32_t row = pos.row;
     uint32_t *out = a.C + (size_t)row * a.stride_C;
     const uint32_t *ra = a.A + (size_t)row * a.stride_A, *rb = a.B + (size_t)row * a.stride_B;
     const int64_t ws = kShift ? (int64_t)(a.shift >> 5) : 0;
     const uint32_t bs = kShift ? (a.shift & 31u) : 0u;
+    const int64_t base = (int64_t)pos.chunk * (kSeg * 4 * kWave);
     uint32_t d[kSeg][4], g[kSeg][4];
 #pragma unroll
     for (int s = 0; s < kSeg; ++s) {
-        const int64_t j0 = (int64_t)chunk * (kSeg * 4 * kWave) + s * (4 * kWave) + 4 * (int64_t)lane;
+        const int64_t j0 = base + s * (4 * kWave) + 4 * (int64_t)lane;
         uint32_t x[4], y[4];
         if constexpr (kShift) {
             // x_t = (A << shift) at limb j0 + t: A[i] << bs | A[i - 1] >> (32 - bs), i = j0 + t - ws
@@ -439,42 +501,56 @@ __global__ void __launch_bounds__(256) addsub_vec_kernel(AddSubArgs a, uint32_t 
             g[s][t] = kSub ? (x[t] < y[t] ? 1u : 0u) : (d[s][t] < x[t] ? 1u : 0u);
         }
     }
-    uint32_t cin = 0;
-    bool all_prop = true;
-#pragma unroll
-    for (int s = 0; s < kSeg; ++s) {
-        const int64_t j0 = (int64_t)chunk * (kSeg * 4 * kWave) + s * (4 * kWave) + 4 * (int64_t)lane;
+    constexpr int kHeld = ROW ? kSeg : 1;  // groups settled before the first is stored
+    uint32_t r[kHeld][4];
+    uint64_t G[kHeld], P[kHeld];
+    const auto settle = [&](int s, int h) {
         // the lane's four limbs for a carry-in of zero
-        uint32_t r[4], c = 0;
+        const int64_t j0 = base + s * (4 * kWave) + 4 * (int64_t)lane;
+        uint32_t c = 0;
         bool prop = true;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            r[t] = kSub ? d[s][t] - c : d[s][t] + c;
+            r[h][t] = kSub ? d[s][t] - c : d[s][t] + c;
             c = g[s][t] | (c & (kSub ? (d[s][t] == 0u ? 1u : 0u) : (d[s][t] == 0xffffffffu ? 1u : 0u)));
-            prop = prop && (kSub ? r[t] == 0u : r[t] == 0xffffffffu) && j0 + t < (int64_t)a.L_c;
+            prop = prop && (kSub ? r[h][t] == 0u : r[h][t] == 0xffffffffu) && j0 + t < (int64_t)a.L_c;
         }
         const bool valid = j0 < (int64_t)a.L_c;
-        const uint64_t G = ballot64(valid && c != 0), P = ballot64(valid && prop);
+        G[h] = ballot64(valid && c != 0);
+        P[h] = ballot64(valid && prop);
+    };
+    uint32_t cin = 0;
+    if constexpr (ROW) {
+#pragma unroll
+        for (int s = 0; s < kSeg; ++s) settle(s, s);
+        cin = carry_into_wave(G, P, lane);
+    }
+    bool all_prop = true;
+#pragma unroll
+    for (int s = 0; s < kSeg; ++s) {
+        const int h = ROW ? s : 0;
+        if constexpr (!ROW) settle(s, 0);
+        const int64_t j0 = base + s * (4 * kWave) + 4 * (int64_t)lane;
         uint32_t cout;
-        const uint64_t cm = resolve_carries(G, P, cin, &cout);
+        const uint64_t cm = resolve_carries(G[h], P[h], cin, &cout);
         uint32_t ci = (uint32_t)(cm >> lane) & 1u;
+        Quad q;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const uint32_t v = kSub ? r[t] - ci : r[t] + ci;
-            ci = ci & (kSub ? (r[t] == 0u ? 1u : 0u) : (r[t] == 0xffffffffu ? 1u : 0u));
-            r[t] = v;
+            q.w[t] = kSub ? r[h][t] - ci : r[h][t] + ci;
+            ci = ci & (kSub ? (r[h][t] == 0u ? 1u : 0u) : (r[h][t] == 0xffffffffu ? 1u : 0u));
         }
         if (j0 + 4 <= (int64_t)a.L_c) {
-            *reinterpret_cast<Quad *>(out + j0) = Quad{{r[0], r[1], r[2], r[3]}};
+            *reinterpret_cast<Quad *>(out + j0) = q;
         } else {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-                if (j0 + t < (int64_t)a.L_c) out[j0 + t] = r[t];
+                if (j0 + t < (int64_t)a.L_c) out[j0 + t] = q.w[t];
         }
-        all_prop = all_prop && (P == ~0ull);
+        all_prop = all_prop && (P[h] == ~0ull);
         cin = cout;
     }
-    if (flags != nullptr && lane == 0) flags[wave] = (uint8_t)(cin | (all_prop ? 2u : 0u));
+    if (flags != nullptr && lane == 0) flags[pos.wave] = (uint8_t)(cin | (all_prop ? 2u : 0u));
 }
 
 struct ChunkPlan {
@@ -512,12 +588,14 @@ hipError_t run_addsub(const AddSubArgs &a, const SpillArgs &sp, uint8_t *flags, 
         return hipGetLastError();
     }
     const uint64_t total = (uint64_t)a.N * p.chunks_per_row;
-    const bool need_fix = p.chunks_per_row > 1;
-    if (need_fix && flags == nullptr) return hipErrorInvalidValue;
-    const uint64_t blocks = ceil_div64(total, 4);
+    // one block per row where a row's chunks fit it
+    const bool rows = p.chunks_per_row > 1 && p.chunks_per_row <= kRowWaves;
+    const bool need_fix = p.chunks_per_row > 1 && !rows;
+    if (p.chunks_per_row > 1 && flags == nullptr) return hipErrorInvalidValue;
+    const uint64_t blocks = rows ? a.N : ceil_div64(total, 4);
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
     uint8_t *fl = need_fix ? flags : nullptr;
-    const dim3 grid((uint32_t)blocks), block(256);
+    const dim3 grid((uint32_t)blocks), block(rows ? p.chunks_per_row * kWave : 256u);
     const auto chunks = [&](auto seg) {
         hipLaunchKernelGGL((addsub_chunk_kernel<K, decltype(seg)::value>), grid, block, 0, stream, a, sp,
                            p.chunks_per_row, total, fl);
@@ -529,11 +607,13 @@ hipError_t run_addsub(const AddSubArgs &a, const SpillArgs &sp, uint8_t *flags, 
         case 8: chunks(std::integral_constant<int, 8>{}); break;
         default:
             // in place is fine: a lane reads the limbs it writes first
-            if constexpr (K == AddSubKind::SpillAdd)
-                hipLaunchKernelGGL(spill_add_vec_kernel, grid, block, 0, stream, a.C, a.stride_C, a.L_c, sp,
-                                   p.chunks_per_row, total, fl);
-            else
-                hipLaunchKernelGGL(addsub_vec_kernel<K>, grid, block, 0, stream, a, p.chunks_per_row, total, fl);
+            if constexpr (K == AddSubKind::SpillAdd) {
+                const auto k = rows ? spill_add_vec_kernel<true> : spill_add_vec_kernel<false>;
+                hipLaunchKernelGGL(k, grid, block, 0, stream, a.C, a.stride_C, a.L_c, sp, p.chunks_per_row, total, fl);
+            } else {
+                const auto k = rows ? addsub_vec_kernel<K, true> : addsub_vec_kernel<K, false>;
+                hipLaunchKernelGGL(k, grid, block, 0, stream, a, p.chunks_per_row, total, fl);
+            }
     }
     GPUPI_RETURN_IF(hipGetLastError());
     if (need_fix) {

@@ -212,13 +212,13 @@ def test_decimal_naive(ctx, L_limb, L_dec, n):
     assert np.array_equal(got[:, :L_dec], want.reshape(n, L_dec))
 
 
-@pytest.mark.parametrize("la", [511, 512, 513, 1023, 1024, 1027, 2050, 3073])
+@pytest.mark.parametrize("la", [511, 512, 513, 1023, 1024, 1027, 2050, 3073, 16383, 16385])
 @pytest.mark.parametrize("extra", [0, 1, 2, 3])
 def test_rows_at_any_alignment(ctx, la, extra):
     """The four-limbs-per-lane carry kernels (results of more than 512 limbs)
     on rows and operands at every 4-byte alignment, around their 1024-limb
-    chunks: random limbs, all ones and zeros, carries and borrows through
-    whole chunks, shifts within and across words, one operation in place."""
+    chunks and the 16 chunks that one block takes: random limbs, all ones and
+    zeros, carries and borrows through whole chunks, shifts within and across words, one operation in place."""
     n, lb = 4, la - 5
     rng = np.random.default_rng(la * 8 + extra)
 
