@@ -54,13 +54,17 @@ constexpr uint64_t kGen0 = 3, kGen1 = 13;          // primitive roots
 //   step tables: for Ms = 2^x (x = 5..12), at (2^x - 32): [j * Ms/16 + n2] =
 //                w_Ms^(n2 * bitrev(j, 4)), j < 16, n2 < Ms/16
 //   lo/hi: w_{2^30}^e and w_{2^30}^(e 2^15), e < 2^15 (and the inverses)
+//   radix-4 step tables (thin tiles): for Ms = 2^x (x = 3..12), at (2^x - 8):
+//                [j * Ms/4 + n2] = w_Ms^(n2 * bitrev(j, 2)), j < 4, n2 < Ms/4
 constexpr size_t kOffStep = 0;
 constexpr size_t kOffStepInv = 8192;
 constexpr size_t kOffLo = 16384;
 constexpr size_t kOffHi = kOffLo + 32768;
 constexpr size_t kOffLoInv = kOffHi + 32768;
 constexpr size_t kOffHiInv = kOffLoInv + 32768;
-constexpr size_t kPrimeTable = kOffHiInv + 32768;
+constexpr size_t kOffStep4 = kOffHiInv + 32768;
+constexpr size_t kOffStep4Inv = kOffStep4 + 8192;
+constexpr size_t kPrimeTable = kOffStep4Inv + 8192;
 constexpr size_t kTableLen = 2 * kPrimeTable;
 
 struct NttConsts {
@@ -873,14 +877,43 @@ __device__ __forceinline__ uint32_t row_shr(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x110 + D, 0xf, 0xf, true);
 }
 
+// The limb at a lane's coefficient c, 2^RL adjacent lanes holding a run of
+// adjacent coefficients (lane mod 2^RL: the position in the run): coefficient
+// c = w0 + 2^32 w1 + 2^64 w2 adds to the limb column sums
+// s_j = w0_j + w1_(j-1) + w2_(j-2), which become limbs with one neighbour
+// shift and one ballot carry resolution per run; what passes the run's top
+// is left in `over` of its last lane.
+template <int RL>
+__device__ __forceinline__ uint32_t run_limb(unsigned __int128 c, uint32_t lane, uint64_t &over) {
+    constexpr uint32_t kRun = 1u << RL;
+    const uint32_t jr = lane & (kRun - 1u);
+    uint64_t last_mask = 0;  // last lanes of runs pass no carry on
+#pragma unroll
+    for (uint32_t l = kRun - 1; l < kWave; l += kRun) last_mask |= 1ull << l;
+    const uint32_t w0 = (uint32_t)c, w1 = (uint32_t)(c >> 32), w2 = (uint32_t)(c >> 64);
+    const uint32_t w1a = row_shr<1>(w1), w2a = row_shr<1>(w2), w2b = row_shr<2>(w2);
+    const uint64_t s = (uint64_t)w0 + (jr >= 1 ? w1a : 0u) + (jr >= 2 ? w2b : 0u);
+    const uint32_t lo = (uint32_t)s, hi = (uint32_t)(s >> 32);
+    const uint32_t hia = row_shr<1>(hi);
+    const uint64_t t = (uint64_t)lo + (jr >= 1 ? hia : 0u);
+    const uint32_t lo2 = (uint32_t)t;
+    const bool gen = (t >> 32) != 0, prop = lo2 == 0xffffffffu;
+    const uint64_t G = ballot64(gen) & ~last_mask, P = ballot64(prop) & ~last_mask;
+    uint32_t unused;
+    const uint64_t cm = resolve_carries(G, P, 0u, &unused);
+    const uint32_t ci = (uint32_t)(cm >> lane) & 1u;
+    // V >> 32 kRun: the carry out of the top limb, the top column's high part
+    // and the words of the last two coefficients past the run
+    const uint64_t cout = (gen || (prop && ci)) ? 1u : 0u;
+    over = cout + hi + (uint64_t)w1 + (uint64_t)w2a + ((uint64_t)w2 << 32);
+    return lo2 + ci;
+}
+
 // First inverse column level: both primes through one tile, 1/K, Garner,
 // and the limbs of each run of adjacent coefficients with the run's spill
-// word.  A thread's element u is (row r0 + u 2^(M-4), column g) and lanes
-// hold adjacent columns, so a run of 2^RL adjacent coefficients sits in
-// 2^RL adjacent lanes: coefficient c = w0 + 2^32 w1 + 2^64 w2 adds to the
-// limb column sums s_j = w0_j + w1_(j-1) + w2_(j-2), which become limbs with
-// one neighbour shift and one ballot carry resolution per run; what passes
-// the run's top goes to the spill word (the carry engine adds it).
+// word (run_limb; the carry engine adds it).  A thread's element u is (row
+// r0 + u 2^(M-4), column g) and lanes hold adjacent columns, so a run of 2^RL
+// adjacent coefficients sits in 2^RL adjacent lanes.
 template <int M, bool PAIR, bool TRUNC>
 __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) __attribute__((amdgpu_waves_per_eu(4)))
 ntt_col_inv_limbs_kernel(PassArgs a) {
@@ -921,9 +954,6 @@ ntt_col_inv_limbs_kernel(PassArgs a) {
 
     const uint32_t lane = threadIdx.x & (kWave - 1u);
     const uint32_t jr = lane & (kRun - 1u);  // position inside the run
-    uint64_t last_mask = 0;                   // last lanes of runs pass no carry on
-#pragma unroll
-    for (uint32_t l = kRun - 1; l < kWave; l += kRun) last_mask |= 1ull << l;
     uint32_t *out = pr.C + (size_t)prod * pr.sC;
     const uint32_t Lc = pr.Lc;
     uint64_t *spill = a.spill + pr.spill_base + (size_t)prod * ((1ull << log2K) >> RL);
@@ -932,26 +962,287 @@ ntt_col_inv_limbs_kernel(PassArgs a) {
     for (int u = 0; u < 16; ++u) {
         if (TRUNC && u >= (int)kTauMin && u >= (int)tau) break;  // uniform over the block
         const unsigned __int128 c = recombine(v0[u], lds[ct.lds0 + 272u * u]);
-        const uint32_t w0 = (uint32_t)c, w1 = (uint32_t)(c >> 32), w2 = (uint32_t)(c >> 64);
-        const uint32_t w1a = row_shr<1>(w1), w2a = row_shr<1>(w2), w2b = row_shr<2>(w2);
-        const uint64_t s = (uint64_t)w0 + (jr >= 1 ? w1a : 0u) + (jr >= 2 ? w2b : 0u);
-        const uint32_t lo = (uint32_t)s, hi = (uint32_t)(s >> 32);
-        const uint32_t hia = row_shr<1>(hi);
-        const uint64_t t = (uint64_t)lo + (jr >= 1 ? hia : 0u);
-        const uint32_t lo2 = (uint32_t)t;
-        const bool gen = (t >> 32) != 0, prop = lo2 == 0xffffffffu;
-        const uint64_t G = ballot64(gen) & ~last_mask, P = ballot64(prop) & ~last_mask;
-        uint32_t unused;
-        const uint64_t cm = resolve_carries(G, P, 0u, &unused);
-        const uint32_t ci = (uint32_t)(cm >> lane) & 1u;
         const uint64_t n = n_u0 + ((uint64_t)u << ct.ustep);
-        if (n < Lc) out[n] = lo2 + ci;
-        if (jr == kRun - 1) {
-            // V >> 32 kRun: the carry out of the top limb, the top column's
-            // high part and the words of the last two coefficients past the run
-            const uint64_t cout = (gen || (prop && ci)) ? 1u : 0u;
-            spill[(n - jr) >> RL] = cout + hi + (uint64_t)w1 + (uint64_t)w2a + ((uint64_t)w2 << 32);
+        uint64_t over;
+        const uint32_t limb = run_limb<RL>(c, lane, over);
+        if (n < Lc) out[n] = limb;
+        if (jr == kRun - 1) spill[(n - jr) >> RL] = over;
+    }
+}
+
+// ------------------------------------------------------------ thin tiles
+//
+// Launches of few blocks are bound by the time of one wave, not by the chip:
+// with 4096-element tiles and 16 values per thread, one product of 2^15
+// coefficients is 16 blocks on 16 of 256 CUs, each wave running both primes'
+// transforms one after the other (13..20 us per kernel).  Thin tiles put the
+// same transform on 8..16 times the waves: 1024 elements, four values per
+// thread in radix-4 steps, one prime per block (both in the halves of a
+// block where the limbs are formed), and the row level transforms A and B
+// side by side.  Plans are 2^kThinCol x 2^(k - kThinCol), every step's
+// twiddles are loaded before the data arrive, and transforms are not
+// truncated (their blocks run side by side anyway).  Values take the
+// butterfly kinds and bounds of the full tiles.  In the products of 10^6
+// digits (up to 2^17 points) the three kernels take 7.8 + 6.9..8.6 + 6.8 us
+// instead of 14 + 12.5..20 + 13.7, most of it launch and memory latency.
+
+// Step S of the 2^M-point DFTs of a tile of 2^LT elements, four values
+// v[u * R + j] per thread (StepMap with radix 4, a last step of 2 for odd M).
+template <int M, int S, bool COL, int LT>
+struct ThinMap {
+    static constexpr int LR = thin_log2radix(M, S);
+    static constexpr int R = 1 << LR;
+    static constexpr int PER = 4 / R;
+    static constexpr int LMS = M - 2 * S;
+    static constexpr int LSS = LMS - LR;
+    static constexpr uint32_t kStride = COL ? 1u << (LSS + LT - M) : 1u << LSS;
+    uint32_t base[PER];
+    uint32_t n2;  // of radix-4 steps (PER == 1)
+    __device__ __forceinline__ explicit ThinMap(uint32_t tid) {
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const ThinDft d = thin_dft(M, S, tid + ((uint32_t)u << (LT - 2)), COL, LT);
+            base[u] = d.base;
+            n2 = d.n2;
         }
+    }
+    __device__ __forceinline__ uint32_t slot(int k) const {
+        return lds_index(base[k / R]) + lds_index((k % R) * kStride);
+    }
+};
+constexpr uint32_t thin_slots(int lt) { return (1u << lt) + (1u << (lt - 4)); }
+
+// The twiddles of a transform's steps, loaded together.
+template <int M, bool COL, int LT>
+struct ThinTw {
+    static constexpr int kSteps = thin_steps(M) - 1;  // the last step has none
+    double w[kSteps][3];
+    template <int S = 0>
+    __device__ __forceinline__ void load(const double *steps, uint32_t tid) {
+        if constexpr (S < kSteps) {
+            using TM = ThinMap<M, S, COL, LT>;
+            const double *tw = steps + ((1u << TM::LMS) - 8u) + TM(tid).n2;
+#pragma unroll
+            for (int j = 1; j < 4; ++j) w[S][j - 1] = tw[j << TM::LSS];
+            load<S + 1>(steps, tid);
+        }
+    }
+};
+
+template <int M, int S, bool INV, bool COL, int LT, int KIND>
+__device__ __forceinline__ void thin_step(double *v, const ThinTw<M, COL, LT> &tw, const double *w16, Mod m) {
+    using TM = ThinMap<M, S, COL, LT>;
+#pragma unroll
+    for (int u = 0; u < TM::PER; ++u) {
+        if (!INV) dif<KIND, TM::R>(&v[u * TM::R], w16, m);
+        if constexpr (S < thin_steps(M) - 1) {
+#pragma unroll
+            for (int j = 1; j < 4; ++j) v[j] = mulp(v[j], tw.w[S][j - 1], m);
+        }
+        if (INV) dit<KIND, TM::R>(&v[u * TM::R], w16, m);
+    }
+}
+template <typename TM>
+__device__ __forceinline__ void thin_store(double *lds, const double *v, const TM &tm) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) lds[tm.slot(k)] = v[k];
+}
+template <typename TM>
+__device__ __forceinline__ void thin_load(double *v, const double *lds, const TM &tm) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = lds[tm.slot(k)];
+}
+
+// Forward transform of a tile, or of two tiles side by side (TWO: v1 in
+// lds1); step-0 values in, last-step values out.
+template <int M, bool COL, int LT, bool TWO, int FINAL0, int FINAL1, int S = 0>
+__device__ __forceinline__ void thin_fwd(double *v0, double *v1, double *lds0, double *lds1,
+                                         const ThinTw<M, COL, LT> &tw, uint32_t tid, const double *w16, Mod m) {
+    constexpr bool kLast = S == thin_steps(M) - 1;
+    const ThinMap<M, S, COL, LT> tm(tid);
+    if constexpr (S > 0) {
+        thin_load(v0, lds0, tm);
+        if (TWO) thin_load(v1, lds1, tm);
+    }
+    thin_step<M, S, false, COL, LT, kLast ? FINAL0 : kDifMid>(v0, tw, w16, m);
+    if (TWO) thin_step<M, S, false, COL, LT, kLast ? FINAL1 : kDifMid>(v1, tw, w16, m);
+    if constexpr (!kLast) {
+        thin_store(lds0, v0, tm);
+        if (TWO) thin_store(lds1, v1, tm);
+        __syncthreads();
+        thin_fwd<M, COL, LT, TWO, FINAL0, FINAL1, S + 1>(v0, v1, lds0, lds1, tw, tid, w16, m);
+    }
+}
+
+// Inverse transform: last-step values in (the thread's own slots, as thin_fwd
+// leaves them), step-0 values out.
+template <int M, bool COL, int LT, int FINAL, int S = thin_steps(M) - 1>
+__device__ __forceinline__ void thin_inv(double *v, double *lds, const ThinTw<M, COL, LT> &tw, uint32_t tid,
+                                         const double *w16i, Mod m) {
+    constexpr bool kFirst = S == thin_steps(M) - 1;
+    const ThinMap<M, S, COL, LT> tm(tid);
+    if constexpr (!kFirst) thin_load(v, lds, tm);
+    thin_step<M, S, true, COL, LT, kFirst ? kDitFirst : S == 0 ? FINAL : kDitMid>(v, tw, w16i, m);
+    if constexpr (S > 0) {
+        thin_store(lds, v, tm);
+        __syncthreads();
+        thin_inv<M, COL, LT, FINAL, S - 1>(v, lds, tw, tid, w16i, m);
+    }
+}
+
+// A column tile's thread: column col = 2^(kThinTileLog2 - kThinCol) t + g of
+// the 2^kThinCol x 2^lr view (element r 2^lr + col), step-0 rows
+// r0 + u 2^(kThinCol - 2), last-step rows thin_col_row(tid, k).
+struct ThinCol {
+    static constexpr int LC = kThinTileLog2 - kThinCol;
+    uint32_t tid, col, r0;
+    int lr;
+    __device__ __forceinline__ ThinCol(const Plan &p, uint32_t t, uint32_t tid_)
+        : tid(tid_), col((t << LC) + (tid_ & ((1u << LC) - 1u))), r0(tid_ >> LC), lr(p.log2M[1]) {}
+    __device__ __forceinline__ uint32_t off(int u) const {
+        return ((r0 + ((uint32_t)u << (kThinCol - 2))) << lr) + col;
+    }
+    __device__ __forceinline__ uint32_t last(int k) const { return (thin_col_row(tid, k) << lr) + col; }
+};
+
+// Column twiddles of last-step value k = 2 u + j: w_K^(col E) with
+// E = thin_col_e0(tid) + u + j 2^(kThinCol - 1), w_K = w_{2^30}^(2^(30 - k)).
+struct ThinColTw {
+    double lb, hb, lu, hu, sj;
+    __device__ __forceinline__ ThinColTw(const double *tab, const ThinCol &tc, int log2K, bool inv) {
+        const double *lo = tab + (inv ? kOffLoInv : kOffLo), *hi = tab + (inv ? kOffHiInv : kOffHi);
+        const uint32_t cg = tc.col << (kMaxLog2 - log2K), eb = cg * thin_col_e0(tc.tid);
+        lb = lo[eb & 32767u];
+        hb = hi[eb >> 15];
+        lu = lo[cg & 32767u];
+        hu = hi[cg >> 15];
+        sj = hi[(cg << (kThinCol - 1)) >> 15];  // a multiple of 2^15: log2K <= 21
+    }
+    __device__ __forceinline__ void apply(double *v, Mod m) const {
+        static_assert(kThinCol % 2 == 1, "a last step of radix 2");
+        const double c0 = mulp(lb, hb, m), su = mulp(lu, hu, m);
+        const double c1 = mulp(c0, sj, m), c2 = mulp(c0, su, m), c3 = mulp(c1, su, m);
+        v[0] = mulp(v[0], c0, m);
+        v[1] = mulp(v[1], c1, m);
+        v[2] = mulp(v[2], c2, m);
+        v[3] = mulp(v[3], c3, m);
+    }
+};
+
+// First level: block (operand row, tile, prime) takes limbs to twiddled
+// columns.
+__global__ void __launch_bounds__(256) ntt_thin_fwd_kernel(PassArgs a) {
+    constexpr int LT = kThinTileLog2;
+    __shared__ double lds[thin_slots(LT)];
+    const int log2K = a.plan.log2K;
+    const BlockPos bp = block_pos_of(blockIdx.x, a.op_start, a.n_ops, 2u << (log2K - LT));
+    const int P = (int)(bp.t & 1u);
+    const NttOp o = a.ops[bp.seg];
+    const ThinCol tc(a.plan, bp.t >> 1, threadIdx.x);
+    const uint32_t *X = o.X + (size_t)bp.row * o.s;
+    uint32_t x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = tc.off(u) < o.L ? X[tc.off(u)] : 0u;
+    const double *tab = a.tables + P * kPrimeTable;
+    ThinTw<kThinCol, true, LT> tw;
+    tw.load(tab + kOffStep4, tc.tid);
+    const ThinColTw ctw(tab, tc, log2K, false);
+    const Mod m = mod_of(P);
+    double v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = (double)x[u];
+    thin_fwd<kThinCol, true, LT, false, kDifToTwiddle, kDifToTwiddle>(v, v, lds, lds, tw, tc.tid, c_ntt.w16[P], m);
+    ctw.apply(v, m);
+    double *T = a.T + o.base + P * o.pstride + ((size_t)bp.row << log2K);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) T[tc.last(k)] = v[k];
+}
+
+// Last level: block (product row, tile, prime) multiplies A's rows by B's
+// (by themselves for a square), over A's plane.
+template <int M>
+__global__ void __launch_bounds__(1u << (thin_row_tile(M) - 2)) ntt_thin_row_kernel(PassArgs a) {
+    constexpr int LT = thin_row_tile(M);
+    __shared__ double lds[2 * thin_slots(LT)];
+    const int log2K = a.plan.log2K;
+    const BlockPos bp = block_pos_of(blockIdx.x, a.prod_start, a.n_prods, 2u << (log2K - LT));
+    const int P = (int)(bp.t & 1u);
+    const NttProd pr = a.prods[bp.seg];
+    const NttOp oa = a.ops[pr.a], ob = a.ops[pr.b];
+    const bool square = pr.a == pr.b;  // uniform over the launch
+    const uint32_t tid = threadIdx.x;
+    const ThinMap<M, 0, false, LT> s0(tid);
+    const size_t off = ((size_t)(bp.t >> 1) << LT) + s0.base[0];
+    double *TA = a.T + oa.base + P * oa.pstride + ((size_t)bp.row << log2K) + off;
+    const double *TB = a.T + ob.base + P * ob.pstride + ((size_t)(pr.b_bcast ? 0u : bp.row) << log2K) + off;
+    double va[4], vb[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) va[j] = TA[j << ThinMap<M, 0, false, LT>::LSS];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) vb[j] = TB[j << ThinMap<M, 0, false, LT>::LSS];
+    const double *tab = a.tables + P * kPrimeTable;
+    ThinTw<M, false, LT> tw, twi;
+    tw.load(tab + kOffStep4, tid);
+    twi.load(tab + kOffStep4Inv, tid);
+    const Mod m = mod_of(P);
+    double *ldsb = lds + thin_slots(LT);
+    if (square) {
+        thin_fwd<M, false, LT, false, kDifToPointA, kDifToPointA>(va, va, lds, lds, tw, tid, c_ntt.w16[P], m);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) va[j] = mulp(va[j], va[j], m);
+    } else {
+        thin_fwd<M, false, LT, true, kDifToPointA, kDifToPointB>(va, vb, lds, ldsb, tw, tid, c_ntt.w16[P], m);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) va[j] = mulp(vb[j], va[j], m);
+    }
+    thin_inv<M, false, LT, kDitLast>(va, lds, twi, tid, c_ntt.w16i[P], m);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) TA[j << ThinMap<M, 0, false, LT>::LSS] = va[j];
+}
+
+// First level's inverse: block (product row, tile), a prime per half of the
+// block; then each half recombines half of the coefficients.
+__global__ void __launch_bounds__(512) ntt_thin_inv_kernel(PassArgs a) {
+    constexpr int LT = kThinTileLog2, RL = ThinCol::LC;
+    static_assert(RL <= 4, "a run lies in a DPP row");
+    __shared__ double lds_tiles[2 * thin_slots(LT)];
+    const int log2K = a.plan.log2K;
+    const BlockPos bp = block_pos_of(blockIdx.x, a.prod_start, a.n_prods, 1u << (log2K - LT));
+    const int P = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    double *lds = lds_tiles + P * thin_slots(LT);
+    const NttProd pr = a.prods[bp.seg];
+    const NttOp oa = a.ops[pr.a];
+    const ThinCol tc(a.plan, bp.t, threadIdx.x & 255u);
+    const double *T = a.T + oa.base + P * oa.pstride + ((size_t)bp.row << log2K);
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = T[tc.last(k)];
+    const double *tab = a.tables + P * kPrimeTable;
+    ThinColTw ctw(tab, tc, log2K, true);
+    ThinTw<kThinCol, true, LT> tw;
+    tw.load(tab + kOffStep4Inv, tc.tid);
+    const Mod m = mod_of(P);
+    ctw.lb = mulp(ctw.lb, c_ntt.kinv[P][log2K], m);  // 1/K, as in the full tiles
+    ctw.apply(v, m);
+    thin_inv<kThinCol, true, LT, kDitToGarner>(v, lds, tw, tc.tid, c_ntt.w16i[P], m);
+    // half P keeps elements u = 2 P, 2 P + 1 and hands the others over
+    const ThinMap<kThinCol, 0, true, LT> s0(tc.tid);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) lds[P ? s0.slot(e) : s0.slot(e + 2)] = P ? v[e] : v[e + 2];
+    __syncthreads();
+    const double *other = lds_tiles + (1 - P) * thin_slots(LT);
+    uint32_t *out = pr.C + (size_t)bp.row * pr.sC;
+    uint64_t *spill = a.spill + pr.spill_base + ((size_t)bp.row << (log2K - RL));
+    const uint32_t lane = threadIdx.x & (kWave - 1u);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const double mine = P ? v[e + 2] : v[e];
+        const double theirs = other[P ? s0.slot(e + 2) : s0.slot(e)];
+        const uint32_t n = P ? tc.off(e + 2) : tc.off(e);
+        uint64_t over;
+        const uint32_t limb = run_limb<RL>(P ? recombine(theirs, mine) : recombine(mine, theirs), lane, over);
+        if (n < pr.Lc) out[n] = limb;
+        if ((lane & ((1u << RL) - 1u)) == (1u << RL) - 1u) spill[n >> RL] = over;
     }
 }
 
@@ -1112,6 +1403,7 @@ void dispatch_m(int m, F &&f) {
         else dispatch_m<LO + 1, HI>(m, f);
     }
 }
+constexpr int kThinRowLo = kThinMinLog2 - kThinCol;
 constexpr int kColLo = 5, kColHi = 9, kRowLo = 6, kRowHi = 12, kLocalLo = kMinLog2, kLocalHi = kTileLog2;
 
 // ---------------------------------------------------------------- host side
@@ -1323,6 +1615,18 @@ hipError_t ntt_tables_init(NTTPrecomputedTables *tables) {
             loi = mulmod_u64(loi, w30i, P);
             hi = mulmod_u64(hi, step_hi, P);
             hii = mulmod_u64(hii, step_hi_i, P);
+        }
+        // radix-4 step tables: powers of w_Ms are powers w_{2^30}^(e 2^15)
+        for (int x = 3; x <= kThinRowMax; ++x) {
+            const uint32_t ss = 1u << (x - 2);
+            for (uint32_t j = 0; j < 4; ++j) {
+                for (uint32_t n2 = 0; n2 < ss; ++n2) {
+                    const size_t slot = ((size_t)1 << x) - 8 + (size_t)j * ss + n2;
+                    const size_t e = ((size_t)n2 * bitrev(j, 2)) << (15 - x);
+                    tab[kOffStep4 + slot] = tab[kOffHi + e];
+                    tab[kOffStep4Inv + slot] = tab[kOffHiInv + e];
+                }
+            }
         }
         const uint64_t w16 = powmod_u64(w30, 1ull << (kMaxLog2 - 4), P);
         const uint64_t w16i = powmod_u64(w16, P - 2, P);
@@ -1541,6 +1845,21 @@ hipError_t run_local(const NttJob &j, const NTTPrecomputedTables &tables, hipStr
     return hipSuccess;
 }
 
+// Whether a job runs on thin tiles: few rows of a plan that was not set by
+// hand.  Measured (us per product call, full / thin tiles): one row of 2^13,
+// 2^15, 2^17, 2^19 points 42 / 19, 45 / 22, 53 / 25, 67 / 44; 2^20 points in
+// all, as 128 rows of 2^13 .. 4 of 2^18, 62..73 / 52..62 and half full 56 / 51;
+// 2^21 points 81..93 / 86..104 (the radix-4 steps take more twiddle products
+// and LDS passes).  Planes and spill words lie where the full tiles' would
+// (neither plan pads its planes, and the runs are the shortest the layout
+// allows for).
+constexpr int kThinMaxTotalLog2 = 20;
+bool run_thin(const NttJob &j, const JobShape &sh) {
+    if (j.ragged || j.k < kThinMinLog2 || j.k > kThinMaxLog2) return false;
+    if (g_split[j.k].load(std::memory_order_relaxed) != 0) return false;
+    return ((uint64_t)sh.rows * j.n_prods << j.k) <= 1ull << kThinMaxTotalLog2;
+}
+
 hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, const NTTPrecomputedTables &tables,
                    hipStream_t stream) {
     if (!job_ok(j)) return hipErrorInvalidValue;
@@ -1548,11 +1867,13 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
     if (sh.rows == 0) return hipSuccess;
     const int k = j.k;
     if (make_plan(k).levels == 1) return run_local(j, tables, stream);
-    const Plan p = active_plan(k);
+    const bool thin = run_thin(j, sh);
+    const Plan p = thin ? thin_plan(k) : active_plan(k);
     const size_t K = size_t(1) << k;
     const JobLayout l = layout_of(j, sh);
     if (workspace == nullptr || workspace_bytes < l.total) return hipErrorInvalidValue;
-    const size_t runs = K >> final_run_log2(p);
+    const int run_log2 = thin ? ThinCol::LC : (int)final_run_log2(p);
+    const size_t runs = K >> run_log2;
     char *ws = static_cast<char *>(workspace);
     uint8_t *flags = reinterpret_cast<uint8_t *>(ws + l.flags_off);
     uint32_t *staging = reinterpret_cast<uint32_t *>(ws + l.staging_off);
@@ -1571,7 +1892,7 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
     // parts (the truncating first-level kernels are 5-10 % slower: 256 ragged
     // pairs, most of them in pieces that fill their transforms, took 37.1 ms
     // truncated wherever a row allowed it and 36.0 ms not truncated)
-    uint32_t tau = sh.tau;
+    uint32_t tau = thin ? kTauMax : sh.tau;
     if (j.ragged) {
         uint64_t parts = 0;
         for (uint32_t i = 0; i < sh.rows; ++i)
@@ -1642,7 +1963,12 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
             return dim3((uint32_t)(n_rows * (row_tiles >> pl)));
         };
         const uint32_t deep = a.tau_tiles;
-        if (fwd_rows > 0) {
+        if (thin && fwd_rows > 0) {
+            const uint32_t n = 2u << (k - kThinTileLog2);
+            GPUPI_RETURN_IF(timed(kColFwdLimbs, k, 4.0 * (double)limb_reads + fwd_tb, stream, [&] {
+                hipLaunchKernelGGL(ntt_thin_fwd_kernel, blocks(fwd_rows, n, 0), dim3(256), 0, stream, args(n, 0));
+            }));
+        } else if (fwd_rows > 0) {
             GPUPI_RETURN_IF(timed(kColFwdLimbs, k, 4.0 * (double)limb_reads + fwd_tb, stream, [&] {
                 dispatch_m<kColLo, kColHi>(p.log2M[0], [&](auto mc) {
                     constexpr int M = decltype(mc)::value;
@@ -1670,7 +1996,22 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
             }
         }
         if (prod_rows == 0) continue;
-        if (j.n_prods == 2 && j.prods[0].b == j.prods[1].b && p.log2M[p.levels - 1] <= kPairMaxM) {
+        if (thin) {
+            const double row_tb = (j.prods[0].a == j.prods[0].b ? 2 : 3) * prod_tb;
+            GPUPI_RETURN_IF(timed(kRowFused, k, row_tb, stream, [&] {
+                dispatch_m<kThinRowLo, kThinRowMax>(p.log2M[1], [&](auto mc) {
+                    constexpr int M = decltype(mc)::value, LT = thin_row_tile(M);
+                    const uint32_t n = 2u << (k - LT);
+                    hipLaunchKernelGGL((ntt_thin_row_kernel<M>), blocks(prod_rows, n, 0), dim3(1u << (LT - 2)), 0,
+                                       stream, args(n, 0));
+                });
+            }));
+            const uint32_t n = 1u << (k - kThinTileLog2);
+            GPUPI_RETURN_IF(timed(kColInvLimbs, k, prod_tb + 4.0 * (double)limb_writes + 8.0 * prod_rows * runs,
+                                  stream, [&] {
+                hipLaunchKernelGGL(ntt_thin_inv_kernel, blocks(prod_rows, n, 0), dim3(512), 0, stream, args(n, 0));
+            }));
+        } else if (j.n_prods == 2 && j.prods[0].b == j.prods[1].b && p.log2M[p.levels - 1] <= kPairMaxM) {
             // shared B: its last-level transform once per tile for both products
             const uint32_t pair_rows = std::max(rows[0], rows[1]);
             GPUPI_RETURN_IF(timed(kRowPair, k, row_bytes * (double)pair_rows + 2 * prod_tb, stream, [&] {
@@ -1701,8 +2042,8 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
                 });
             }));
         }
-        GPUPI_RETURN_IF(timed(kColInvLimbs, k, prod_tb + 4.0 * (double)limb_writes + 8.0 * prod_rows * runs, stream,
-                              [&] {
+        if (!thin) GPUPI_RETURN_IF(timed(kColInvLimbs, k, prod_tb + 4.0 * (double)limb_writes + 8.0 * prod_rows * runs,
+                                         stream, [&] {
             dispatch_m<kColLo, kColHi>(p.log2M[0], [&](auto mc) {
                 constexpr int M = decltype(mc)::value;
                 with_flags<M>((pair_mask >> kPairInvLimbs) & 1u, trunc, [&](auto pc, auto tc) {
@@ -1717,7 +2058,7 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
             if (rows[q] == 0) continue;
             const NttProd &d = a.prods[q];
             GPUPI_RETURN_IF(launch_add_spills(d.C, a.spill + d.spill_base, rows[q], d.Lc, d.sC,
-                                              1u << final_run_log2(p), (uint32_t)runs, flags, stream));
+                                              1u << run_log2, (uint32_t)runs, flags, stream));
         }
         if (j.ragged) {
             bool copies = false;

@@ -317,6 +317,58 @@ GPUPI_HD uint64_t col_plane_row_step(const Plan &p, int level) {
     return (1ull << rs) + ((s && rs >= s) ? ((uint64_t)kPlanePad << (rs - s)) : 0ull);
 }
 
+// Thin tiles (launches of few blocks): transforms of 2^kThinMinLog2 ..
+// 2^kThinMaxLog2 points as 2^kThinCol columns and a contiguous level, tiles
+// of 2^kThinTileLog2 elements (a longer row is a tile by itself), four values
+// per thread: radix-4 steps, the last one of radix 2 when the size is odd.
+constexpr int kThinCol = 7, kThinTileLog2 = 10;
+constexpr int kThinMinLog2 = 13, kThinMaxLog2 = 19;
+constexpr int kThinRowMax = kThinMaxLog2 - kThinCol;
+GPUPI_HD Plan thin_plan(int log2K) {
+    Plan p{};
+    p.log2K = log2K;
+    p.levels = 2;
+    p.log2M[0] = kThinCol;
+    p.log2M[1] = log2K - kThinCol;
+    return p;
+}
+GPUPI_HD constexpr int thin_row_tile(int m) { return m > kThinTileLog2 ? m : kThinTileLog2; }
+GPUPI_HD constexpr int thin_steps(int m) { return (m + 1) / 2; }
+GPUPI_HD constexpr int thin_log2radix(int m, int s) { return s < m / 2 ? 2 : 1; }
+// Small DFT q (of 2^lt / R per tile) at step s, as small_dft.
+struct ThinDft {
+    uint32_t base, n2;
+};
+GPUPI_HD ThinDft thin_dft(int m, int s, uint32_t q, bool col, int lt) {
+    const int log2Ms = m - 2 * s;
+    const int log2Ss = log2Ms - thin_log2radix(m, s);
+    const int lg = lt - m;
+    ThinDft d;
+    if (col) {
+        const uint32_t g = q & ((1u << lg) - 1u), rest = q >> lg;
+        d.n2 = rest & ((1u << log2Ss) - 1u);
+        d.base = ((((rest >> log2Ss) << log2Ms) + d.n2) << lg) + g;
+    } else {
+        d.n2 = q & ((1u << log2Ss) - 1u);
+        d.base = ((q >> log2Ss) << log2Ms) + d.n2;
+    }
+    return d;
+}
+// Last-step value k = 2 u + j of a column tile's thread: its row, and the
+// row's frequency bitrev(row, kThinCol) = thin_col_e0 + u + j 2^(kThinCol - 1).
+GPUPI_HD uint32_t thin_col_row(uint32_t tid, int k) {
+    return 2u * (tid >> (kThinTileLog2 - kThinCol)) + ((uint32_t)(k >> 1) << (kThinCol - 1)) + (uint32_t)(k & 1);
+}
+GPUPI_HD uint32_t thin_col_e0(uint32_t tid) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint32_t r = __brev(tid >> (kThinTileLog2 - kThinCol)) >> (32 - (kThinCol - 2));
+#else
+    uint32_t r = 0;
+    for (int i = 0; i < kThinCol - 2; ++i) r |= ((tid >> (kThinTileLog2 - kThinCol + i)) & 1u) << (kThinCol - 3 - i);
+#endif
+    return 2u * r;
+}
+
 // Workgroups are dealt to the 8 XCDs (each with its own L2) round-robin:
 // block b runs on XCD b mod 8.  xcd_tile(b, n, c) renumbers blocks in
 // groups of 8 * 2^c: within a group each XCD gets 2^c consecutive tiles, so

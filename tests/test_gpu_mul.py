@@ -670,6 +670,15 @@ def test_truncated_transforms(ctx, k):
     and next to every pair of parts of 2^k points, one row and several, equal
     and unequal lengths, a broadcast operand, a square and a shared pair with
     different numbers of parts, against GMP; nothing is written past a row."""
+    # sizes set by hand (to the built-in ones) keep short launches on full tiles
+    g.ntt_set_split(k, *(g.ntt_get_split(k)[:-1] if k < 20 else (0,)))
+    try:
+        truncated_products(ctx, k)
+    finally:
+        g.ntt_set_split(k, 0)
+
+
+def truncated_products(ctx, k):
     rng = np.random.default_rng(k)
     K = 1 << k
     totals = sorted({min(max(K * t // 16 + d, K // 2 + 1), K) for t in (8, 10, 12, 14, 16) for d in (-1, 0, 1)})
@@ -698,6 +707,49 @@ def test_truncated_transforms(ctx, k):
     g.synchronize()
     assert np.array_equal(g.download_rows(w1, c1), oracle_mul(A1, B))
     assert np.array_equal(g.download_rows(w2, c2), oracle_mul(A2, B))
+
+
+@pytest.mark.parametrize("k", [13, 14, 15, 16, 17, 18, 19])
+def test_thin_tiles(ctx, k):
+    """Few products of 2^k points run on thin tiles, the same call with the
+    level sizes set by hand on full ones: both give GMP's product for full and
+    half-full transforms, lopsided and all-ones operands, padded rows, a
+    broadcast operand on either side, squares and shared pairs, and around
+    the number of rows where the thin tiles end."""
+    rng = np.random.default_rng(900 + k)
+    K = 1 << k
+    builtin = g.ntt_get_split(k)[:-1]
+
+    def both(run, want):
+        for sizes in ((0,), builtin):
+            g.ntt_set_split(k, *sizes)
+            try:
+                assert all(np.array_equal(x, y) for x, y in zip(run(), want)), sizes
+            finally:
+                g.ntt_set_split(k, 0)
+
+    for n, la, lb, mode in ((1, K // 2, K // 2, "ones"), (1, K // 2, K // 2, "random"), (2, K - 4090, 4090, "random"),
+                            (1, K // 4 + 1, K // 4, "random"), (1, K // 2 - 999, K // 4 + 3, "ones")):
+        A, B = rand_rows(rng, n, la, mode), rand_rows(rng, n, lb, mode)
+        want = oracle_mul(A, B)
+        both(lambda: (device_mul(ctx, A, B, sa=la + 3, sb=lb + 1), device_mul(ctx, B, A, sc_extra=5)), (want, want))
+        both(lambda: (device_mul(ctx, A, B, b_broadcast=True),), (oracle_mul(A, np.repeat(B[:1], n, axis=0)),))
+        buf, va = g.upload_rows(A)
+        if 2 * la <= K:
+            bufc, vc = g.upload_rows(np.zeros((n, 2 * la), np.uint32))
+
+            def square():
+                g.check(ctx.mul(va, va, vc), "square")
+                g.synchronize()
+                return (g.download_rows(vc, bufc),)
+            both(square, (oracle_mul(A, A),))
+    la1, la2, lb = K // 4 + 5, K // 2 - 80, K // 4 + 77
+    for n1, n2 in ((1, 1), (2, 1), (1, 2)):
+        A1, A2, B = rand_rows(rng, n1, la1), rand_rows(rng, n2, la2), rand_rows(rng, max(n1, n2), lb)
+        both(lambda: device_mul_shared(ctx, A1, A2, B), (oracle_mul(A1, B[:n1]), oracle_mul(A2, B[:n2])))
+    for n in ((1 << 20 - k), (1 << 20 - k) + 1):
+        A, B = rand_rows(rng, n, K // 2 - 1), rand_rows(rng, n, K // 2 - 4)
+        both(lambda: (device_mul(ctx, A, B),), (oracle_mul(A, B),))
 
 
 def test_truncated_transforms_in_ragged_calls(ctx):
