@@ -521,22 +521,41 @@ namespace {
 // product's pieces stay in one launch), each with the set of distinct B
 // operands its rows use.
 hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const std::vector<uint32_t> &small,
-                           const std::vector<std::pair<int, uint32_t>> &big, const std::vector<SplitPlan> &plans) {
+                           const std::vector<uint32_t> &big, const std::vector<SplitPlan> &plans) {
     // groups of rows: a whole product (one row) or a split one (its pieces)
     struct Group {
-        int k;
+        gpupi::NttShape shape;
         size_t q;
     };
     std::vector<Group> groups;
     for (size_t q = 0; q < big.size(); ++q) {
-        const GpupiMulItem &it = items[big[q].second];
-        const int k = plans[q].m < 2 ? big[q].first
-                                     : gpupi::ntt_transform_log2(plans[q].s, std::min(it.L_a, it.L_b));
-        groups.push_back(Group{k, q});
+        const GpupiMulItem &it = items[big[q]];
+        groups.push_back(Group{plans[q].m < 2 ? gpupi::ntt_shape(it.L_a, it.L_b)
+                                              : gpupi::ntt_shape(plans[q].s, std::min(it.L_a, it.L_b)), q});
     }
-    std::stable_sort(groups.begin(), groups.end(), [](const Group &x, const Group &y) { return x.k < y.k; });
+    const auto key = [](const gpupi::NttShape &s) { return std::make_pair(s.k, s.bits); };
+    std::stable_sort(groups.begin(), groups.end(),
+                     [&](const Group &x, const Group &y) { return key(x.shape) < key(y.shape); });
+    // a launch sequence of few rows takes 35-45 us whatever its size, and 2^20
+    // points more in another take 25: up to that many, rows join the next
+    // larger transform (14 pairs of 2^8..2^16 limbs: 287 -> 111 us; with
+    // 2^22 points 164 pairs of 2^8..2^18 limbs 536 -> 656 us)
+    constexpr uint64_t kJoinPoints = 1ull << 20;
+    for (size_t e = groups.size(), top = e; e > 0;) {
+        size_t b = e;
+        uint64_t rows = 0;
+        const gpupi::NttShape shape = groups[e - 1].shape;
+        for (; b > 0 && key(groups[b - 1].shape) == key(shape); --b)
+            rows += plans[groups[b - 1].q].m < 2 ? 1u : plans[groups[b - 1].q].m;
+        const bool join = top < groups.size() && shape.k > gpupi::kNttOneTileLog2 && shape.k < groups[top].shape.k &&
+                          shape.bits >= groups[top].shape.bits && rows << groups[top].shape.k <= kJoinPoints;
+        if (join)
+            for (size_t i = b; i < e; ++i) groups[i].shape = groups[top].shape;
+        top = b;
+        e = b;
+    }
     struct Launch {
-        int k;
+        gpupi::NttShape shape;
         size_t r0, n, b0, nb, a0, na;
         uint32_t chunks;
     };
@@ -555,14 +574,14 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
     };
     size_t ntt_bytes = 0;
     for (size_t g0 = 0; g0 < groups.size();) {
-        const int k = groups[g0].k;
-        const size_t cap = gpupi::ntt_ragged_max_rows(k);
-        Launch l{k, host_rows.size(), 0, host_bset.size(), 0, host_asms.size(), 0, 0};
+        const gpupi::NttShape shape = groups[g0].shape;
+        const size_t cap = gpupi::ntt_ragged_max_rows(shape.k);
+        Launch l{shape, host_rows.size(), 0, host_bset.size(), 0, host_asms.size(), 0, 0};
         bidx.clear();
         size_t g1 = g0;
-        for (; g1 < groups.size() && groups[g1].k == k; ++g1) {
+        for (; g1 < groups.size() && key(groups[g1].shape) == key(shape); ++g1) {
             const size_t q = groups[g1].q;
-            const GpupiMulItem &it = items[big[q].second];
+            const GpupiMulItem &it = items[big[q]];
             const uint32_t m = plans[q].m < 2 ? 1u : plans[q].m;
             if (l.n > 0 && l.n + m > cap) break;
             if (m == 1) {
@@ -580,10 +599,10 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
         }
         for (size_t r = l.r0; r < l.r0 + l.n; ++r) {
             gpupi::RaggedB &b = host_bset[l.b0 + host_rows[r].b];
-            b.tau = std::max(b.tau, gpupi::ntt_tau(host_rows[r].L_a, host_rows[r].L_b, k));
+            b.tau = std::max(b.tau, gpupi::ntt_tau(host_rows[r].L_a, host_rows[r].L_b, shape.k, shape.bits));
         }
         l.na = host_asms.size() - l.a0;
-        ntt_bytes = std::max(ntt_bytes, gpupi::ntt_ragged_workspace_bytes((uint32_t)l.n, (uint32_t)l.nb, l.chunks, k));
+        ntt_bytes = std::max(ntt_bytes, gpupi::ntt_ragged_workspace_bytes((uint32_t)l.n, (uint32_t)l.nb, l.chunks, shape));
         launches.push_back(l);
         g0 = g1;
     }
@@ -628,7 +647,7 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
     for (const Launch &l : launches)
         GPUPI_RETURN_IF(gpupi::launch_mul_ntt_ragged(
             d_rows + l.r0, host_rows.data() + l.r0, (uint32_t)l.n, d_bset + l.b0, host_bset.data() + l.b0,
-            (uint32_t)l.nb, d_asms + l.a0, host_asms.data() + l.a0, (uint32_t)l.na, l.chunks, l.k, ntt_ws,
+            (uint32_t)l.nb, d_asms + l.a0, host_asms.data() + l.a0, (uint32_t)l.na, l.chunks, l.shape, ntt_ws,
             ntt_bytes, ctx->ntt_tables, ctx->stream));
     return hipSuccess;
 }
@@ -637,7 +656,7 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
 hipError_t gpupi_mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint32_t count) {
     if (ctx == nullptr || (count > 0 && items == nullptr)) return hipErrorInvalidValue;
     // validate everything before launching anything
-    std::vector<std::pair<int, uint32_t>> big;  // (log2 K, item) of the NTT products
+    std::vector<uint32_t> big;  // NTT products
     for (uint32_t i = 0; i < count; ++i) {
         const GpupiMulItem &it = items[i];
         const uint64_t total = (uint64_t)it.L_a + it.L_b;
@@ -651,7 +670,7 @@ hipError_t gpupi_mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint
             if (!gpupi::mul_naive_supports(it.L_a, it.L_b) && it.L_a && it.L_b) return hipErrorInvalidValue;
         } else {
             if (!gpupi::ntt_supports(it.L_a, it.L_b)) return hipErrorInvalidValue;
-            big.emplace_back(gpupi::ntt_transform_log2(it.L_a, it.L_b), i);
+            big.push_back(i);
         }
     }
     // small products: those the matrix cores take share a few launches where
@@ -685,7 +704,7 @@ hipError_t gpupi_mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint
     std::vector<SplitPlan> plans(big.size());
     if (ctx->pipeline_form != GPUPI_FORM_PLAIN)
         for (size_t q = 0; q < big.size(); ++q) {
-            const GpupiMulItem &it = items[big[q].second];
+            const GpupiMulItem &it = items[big[q]];
             plans[q] = split_plan(std::max(it.L_a, it.L_b), std::min(it.L_a, it.L_b));
         }
     return ragged_launches(ctx, items, small, big, plans);

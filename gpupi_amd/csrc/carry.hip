@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "ntt_plan.hpp"
 
 namespace gpupi {
 namespace {
@@ -29,7 +30,7 @@ struct Digit {
 
 struct SpillArgs {
     const uint64_t *spill;
-    uint32_t run_log2;  // runs of 2^run_log2 limbs
+    ntt::RunDivisor run;  // limbs per run
     uint32_t runs_per_row;
 };
 
@@ -71,10 +72,10 @@ __device__ __forceinline__ Digit digit_at(const AddSubArgs &a, const SpillArgs &
         }
         y = load_or_zero(a.B, row, a.stride_B, j, a.L_b);
     } else {
-        // spill-add: C[j] += word of spill[run] at (run + 1) 2^run_log2 (+1)
+        // spill-add: C[j] += word of spill[run] at (run + 1) run_len (+1)
         x = load_or_zero(a.A, row, a.stride_A, j, a.L_a);
         y = 0;
-        const uint32_t q = j >> sp.run_log2, rem = j & ((1u << sp.run_log2) - 1u);
+        const uint32_t q = sp.run.run_of(j), rem = j - q * sp.run.len;
         if (q >= 1 && rem < 2) {
             const uint64_t s = sp.spill[(size_t)row * sp.runs_per_row + (q - 1)];
             y = rem == 0 ? (uint32_t)s : (uint32_t)(s >> 32);
@@ -254,7 +255,6 @@ spill_add_vec_kernel(uint32_t *C, uint32_t stride_C, uint32_t L_c, SpillArgs sp,
     const uint32_t lane = threadIdx.x & (kWave - 1);
     uint32_t *out = C + (size_t)pos.row * stride_C;
     const uint64_t *rsp = sp.spill + (size_t)pos.row * sp.runs_per_row;
-    const uint32_t run_mask = (1u << sp.run_log2) - 1u;
     const uint32_t base = pos.chunk * (uint32_t)(kSeg * 4 * kWave) + 4 * lane;
     uint32_t r[kSeg][4];
     uint64_t G[kSeg], P[kSeg];
@@ -272,17 +272,23 @@ spill_add_vec_kernel(uint32_t *C, uint32_t stride_C, uint32_t L_c, SpillArgs sp,
     }
     const auto settle = [&](int s) {
         const uint32_t j0 = base + (uint32_t)s * (4 * kWave);
+        // runs are at least 8 limbs, so the four limbs meet at most one run's
+        // start: at limb j0 + at (at = -1: its second limb is the first here)
+        uint32_t q = sp.run.run_of(j0);
+        const uint32_t rem = j0 - q * sp.run.len;
+        int at = -(int)rem;
+        if (rem > 1) {
+            ++q;
+            at += (int)sp.run.len;
+        }
+        uint64_t w = 0;
+        if (q >= 1 && at < 4 && (int64_t)j0 + at < (int64_t)L_c) w = rsp[q - 1];
         uint32_t c = 0;
         bool ones = true;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const uint32_t j = j0 + t;
-            uint32_t y = 0;
-            const uint32_t q = j >> sp.run_log2, rem = j & run_mask;
-            if (q >= 1 && rem < 2 && j < L_c) {
-                const uint64_t w = rsp[q - 1];
-                y = rem == 0 ? (uint32_t)w : (uint32_t)(w >> 32);
-            }
+            const uint32_t y = t == at ? (uint32_t)w : t == at + 1 && j < L_c ? (uint32_t)(w >> 32) : 0u;
             const uint32_t d = r[s][t] + y;
             const uint32_t g = d < y ? 1u : 0u;
             r[s][t] = d + c;
@@ -637,7 +643,7 @@ size_t carry_flags_bytes(uint32_t N, uint32_t L_c) {
 }
 
 hipError_t launch_addsub(const AddSubArgs &a, uint8_t *flags, hipStream_t stream) {
-    const SpillArgs sp{nullptr, 0, 0};
+    const SpillArgs sp{};
     switch (a.kind) {
         case AddSubKind::Add: return run_addsub<AddSubKind::Add>(a, sp, flags, stream);
         case AddSubKind::Sub: return run_addsub<AddSubKind::Sub>(a, sp, flags, stream);
@@ -663,17 +669,17 @@ hipError_t launch_add_spills(uint32_t *C, const uint64_t *spill, uint32_t N, uin
     a.L_c = L_c;
     a.stride_A = stride_C;
     a.stride_C = stride_C;
-    if (run_len == 0 || (run_len & (run_len - 1)) != 0) return hipErrorInvalidValue;
-    const SpillArgs sp{spill, (uint32_t)__builtin_ctz(run_len), runs_per_row};
+    if (run_len < 8 || L_c >= 0x80000000u) return hipErrorInvalidValue;
+    const SpillArgs sp{spill, ntt::run_divisor(run_len), runs_per_row};
     return run_addsub<AddSubKind::SpillAdd>(a, sp, flags, stream);
 }
 
-hipError_t launch_ragged_assemble(const uint32_t *staging, uint64_t K, const RaggedAssembly *as, uint32_t n,
+hipError_t launch_ragged_assemble(const uint32_t *staging, uint64_t stride, const RaggedAssembly *as, uint32_t n,
                                   uint32_t chunks, uint8_t *flags, hipStream_t stream) {
     if (n == 0 || chunks == 0) return hipSuccess;
     if (staging == nullptr || as == nullptr || flags == nullptr) return hipErrorInvalidValue;
     const uint32_t blocks = (chunks + 3) / 4;
-    hipLaunchKernelGGL(ragged_assemble_kernel, dim3(blocks), dim3(256), 0, stream, staging, K, as, n, chunks, flags);
+    hipLaunchKernelGGL(ragged_assemble_kernel, dim3(blocks), dim3(256), 0, stream, staging, stride, as, n, chunks, flags);
     GPUPI_RETURN_IF(hipGetLastError());
     hipLaunchKernelGGL(ragged_assembly_fixup_kernel, dim3(blocks), dim3(256), 0, stream, as, n, chunks,
                        (const uint8_t *)flags);

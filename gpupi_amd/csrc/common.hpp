@@ -69,7 +69,7 @@ hipError_t launch_addsub(const AddSubArgs &args, uint8_t *flags, hipStream_t str
 
 // C (limbs) += spill words: for each run r (run_len limbs), the 64-bit
 // value spill[r] is added at limb (r + 1) * run_len of the same row
-// (run_len a power of two).
+// (run_len >= 8, L_c < 2^31).
 hipError_t launch_add_spills(uint32_t *C, const uint64_t *spill, uint32_t N, uint32_t L_c,
                              uint32_t stride_C, uint32_t run_len, uint32_t runs_per_row,
                              uint8_t *flags, hipStream_t stream);
@@ -113,9 +113,17 @@ hipError_t launch_mul_ntt_bounded(const uint32_t *A, const uint32_t *B, uint32_t
                                   size_t workspace_bytes, const NTTPrecomputedTables &tables, uint32_t N,
                                   uint32_t L_a, uint32_t L_b, uint32_t stride_A, uint32_t stride_B,
                                   uint32_t stride_C, hipStream_t stream);
+// log2 of the transform that a product takes with a limb per coefficient.
 int ntt_transform_log2(uint32_t L_a, uint32_t L_b);
+// The transform that it takes: 2^k coefficients of `bits`-bit digits.
+struct NttShape {
+    int k;
+    uint32_t bits;
+};
+NttShape ntt_shape(uint32_t L_a, uint32_t L_b);
+constexpr int kNttOneTileLog2 = 12;  // transforms up to here run in one tile
 // Parts (of 16) of a transform of 2^log2K points that such a product uses.
-uint32_t ntt_tau(uint32_t L_a, uint32_t L_b, int log2K);
+uint32_t ntt_tau(uint32_t L_a, uint32_t L_b, int log2K, uint32_t bits = 32);
 // The fused 17-term group stage: N rows each of P (51 limbs), Q (68), R (83).
 hipError_t launch_group_stage(uint32_t N, uint32_t *P, uint32_t *Q, uint32_t *R, hipStream_t stream);
 // Rows a ragged launch is filled to (one launch chunk of 2^log2K-point
@@ -129,17 +137,17 @@ size_t ntt_pieces_workspace_bytes(uint32_t LL, uint32_t LS, uint32_t m, uint32_t
 hipError_t launch_mul_ntt_pieces(const uint32_t *L, uint32_t LL, const uint32_t *S, uint32_t LS, uint32_t *C,
                                  uint32_t m, uint32_t s, void *workspace, size_t workspace_bytes,
                                  const NTTPrecomputedTables &tables, hipStream_t stream);
-// The assemblies of a ragged launch from its staged rows (K limbs each):
+// The assemblies of a ragged launch from its staged rows (`stride` limbs apart):
 // n assemblies, `chunks` chunks in all; `flags` holds one byte per chunk.
-hipError_t launch_ragged_assemble(const uint32_t *staging, uint64_t K, const RaggedAssembly *as, uint32_t n,
+hipError_t launch_ragged_assemble(const uint32_t *staging, uint64_t stride, const RaggedAssembly *as, uint32_t n,
                                   uint32_t chunks, uint8_t *flags, hipStream_t stream);
-size_t ntt_ragged_workspace_bytes(uint32_t N, uint32_t nb, uint32_t chunks, int log2K);
+size_t ntt_ragged_workspace_bytes(uint32_t N, uint32_t nb, uint32_t chunks, const NttShape &shape);
 // N rows over nb B operands and n_asm assemblies of `chunks` chunks in all,
-// as device arrays with host copies: every row's L_a + L_b <= 2^log2K and
-// b < nb; rows without C (assembled) only above one tile (2^log2K > 4096).
+// as device arrays with host copies: every row's digits fit the shape and
+// b < nb; rows without C (assembled) only above one tile (2^k > 4096).
 hipError_t launch_mul_ntt_ragged(const RaggedRow *rows, const RaggedRow *host_rows, uint32_t N, const RaggedB *bset,
                                  const RaggedB *host_bset, uint32_t nb, const RaggedAssembly *asms,
-                                 const RaggedAssembly *host_asms, uint32_t n_asm, uint32_t chunks, int log2K,
+                                 const RaggedAssembly *host_asms, uint32_t n_asm, uint32_t chunks, const NttShape &shape,
                                  void *workspace, size_t workspace_bytes, const NTTPrecomputedTables &tables,
                                  hipStream_t stream);
 bool ntt_supports(uint32_t L_a, uint32_t L_b);

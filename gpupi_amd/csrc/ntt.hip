@@ -7,9 +7,9 @@
 // product is six FP64 operations (Dekker/FMA two-product + rounded quotient):
 //     h = a*b; l = fma(a,b,-h); q = rint(h/p); r = fma(-q,p,h) + l.
 // Two primes p0, p1 < 2^49 with 2^30 | p - 1 give exact coefficients up to
-// p0 p1 ~ 2^98 (a coefficient of a product of 32-bit limbs is < 2^91 for
-// lengths up to 2^27), so each limb is one coefficient and transforms reach
-// 2^30 points.  Values are kept centred (|v| <= 0.75 p) so no compare/select
+// p0 p1 ~ 2^98, room for digits wider than a limb: 40, 36 or 34 bits by the
+// length of the product (shape_for), limbs in one-tile products.  Transforms
+// reach 2^30 points.  Values are kept centred (|v| <= 0.75 p) so no compare/select
 // is needed inside butterflies; sums are re-centred every other stage.
 //
 // Residues are stored planar (one array of binary64 per prime) and every
@@ -21,7 +21,7 @@
 // adjacent columns per tile) and a final contiguous level.  The last forward
 // level, the pointwise product and the first inverse level are one kernel;
 // the final inverse level applies 1/K, recombines the primes (Garner) and
-// emits limbs with carries resolved inside runs of <= 16 adjacent
+// emits words with carries resolved inside runs of <= 16 adjacent
 // coefficients, leaving one 64-bit spill word per run for the carry pass.
 //
 // Twiddles: in-tile steps read a per-step table laid out [j][n2] so that a
@@ -305,24 +305,25 @@ __device__ __forceinline__ void column_twiddles(double *x, const ColTw &tw, Mod 
     }
 }
 
-// An integral double in [0, 2^52) as an integer: adding 2^52 puts its value
-// in the mantissa bits (exact), which one integer subtraction reads out.
+// Integral doubles as integers, by adding a power that puts their value into
+// the mantissa bits (exact), which one integer subtraction reads out: in
+// [0, 2^52), and in [-2^51, 2^51).
 __device__ __forceinline__ uint64_t small_double_to_u64(double x) {
     return (uint64_t)__double_as_longlong(x + 0x1p52) - (uint64_t)__double_as_longlong(0x1p52);
 }
+__device__ __forceinline__ int64_t small_double_to_i64(double x) {
+    return __double_as_longlong(x + 0x1.8p52) - __double_as_longlong(0x1.8p52);
+}
 
-// Garner recombination of centred residues -> exact coefficient (< 2^98):
-// r0 + p0 t with t = (r1 - r0) / p0 mod p1; p0 t is formed from shifts, since
-// p0 = 2^49 - 2^30 + 1.
+// Garner recombination of centred residues (|v| < p/2 + p/1024) -> exact
+// coefficient c, at most p0 p1 - p0: c = v0 + p0 t with t = (v1 - v0) / p0
+// mod p1.  v0 may stay negative: (c - v0) / p0 is an integer in [0, p1), since
+// v0 <= c (it is c less a multiple of p0 and below p0) and c - v0 < p0 p1.
 __device__ __forceinline__ unsigned __int128 recombine(double v0, double v1) {
-    static_assert(kPrime0 == (1ull << 49) - (1ull << 30) + 1ull, "p0 = 2^49 - 2^30 + 1");
     const Mod m1 = mod_of(1);
-    const double r0 = v0 < 0.0 ? v0 + kP0 : v0;
-    const double r1 = v1 < 0.0 ? v1 + kP1 : v1;
-    double t = mulp(r1 - r0, c_ntt.garner, m1);
+    double t = mulp(v1 - v0, c_ntt.garner, m1);
     t = t < 0.0 ? t + kP1 : t;
-    const unsigned __int128 T = small_double_to_u64(t);
-    return (T << 49) - (T << 30) + T + small_double_to_u64(r0);
+    return (unsigned __int128)small_double_to_u64(t) * kPrime0 + (unsigned __int128)(__int128)small_double_to_i64(v0);
 }
 
 // Forward operand o of a multi-level launch: limbs of row i at X + i s (the
@@ -372,6 +373,7 @@ struct PassArgs {
     // deeper levels' tiles that hold them (with row_tau the most of any row:
     // each ragged row uses its own)
     uint32_t tau, tau_tiles, row_tau;
+    uint32_t q;  // digits of 32 + q bits
     // log2 of the tiles each XCD takes in turn (xcd_tile)
     int xcd_log2;
 };
@@ -380,7 +382,9 @@ struct PassArgs {
 // `seg` needs.
 __device__ __forceinline__ uint32_t fwd_tau(const PassArgs &a, uint32_t seg, uint32_t row) {
     if (!a.row_tau) return a.tau;
-    return seg ? a.bset[row].tau : tau_of((uint64_t)a.rows[row].L_a + a.rows[row].L_b, a.plan.log2K);
+    if (seg) return a.bset[row].tau;
+    const uint32_t bits = 32u + a.q;
+    return tau_of(digits_of(a.rows[row].L_a, bits) + digits_of(a.rows[row].L_b, bits), a.plan.log2K);
 }
 __device__ __forceinline__ uint32_t prod_tau(const PassArgs &a, uint32_t row) { return fwd_tau(a, 0, row); }
 // Whether a deeper level's tile t lies past those parts (ragged rows; the
@@ -528,7 +532,7 @@ __device__ __forceinline__ void col_fwd_prime(double *v, double *lds, const ColT
 }
 
 // col_fwd_prime with the column twiddles loaded after the transform (fewer
-// registers held through it), then a barrier.
+// registers held through it), and no barrier at its end.
 template <int M, int P>
 __device__ __forceinline__ void col_fwd_prime_late(double *v, double *lds, const ColThread<M> &ct,
                                                    const double *tables) {
@@ -536,7 +540,6 @@ __device__ __forceinline__ void col_fwd_prime_late(double *v, double *lds, const
     const double *tab = tables + P * kPrimeTable;
     fwd_dft<M, true, kDifToTwiddle>(v, lds, tab, P, m, ct.tid);
     column_twiddles<M>(v, col_tw_load<M>(tab, ct.cg, ct.B0, false), m);
-    __syncthreads();
 }
 
 // Forward column level above the first: blocks cover (product, operand,
@@ -608,10 +611,45 @@ __device__ __forceinline__ void col_load_last(double *v, const double *T, const 
     }
 }
 
-// Limbs of one tile block for the first forward level: element u of the
-// thread's column (zero past the operand's length).
+// Words w and w + 1 of an operand, which hold a digit (its low end in a, its
+// high end in b), zero past the operand's end: buffer loads, whose range
+// check is the hardware's, so that no load is under a branch.  Byte offsets
+// stay below 2^32 (kWideMaxLog2), but for b of the last digit of 2^30 points,
+// which has 32 bits and no use of it.
+struct DigitWords {
+    uint32_t a, b;
+};
+struct Words {
+    __amdgpu_buffer_rsrc_t rsrc;
+    // X, L: uniform
+    __device__ __forceinline__ Words(const uint32_t *X, uint32_t L) {
+        const uint64_t p = reinterpret_cast<uint64_t>(X);
+        const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32)) << 32 |
+                           (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
+        const int bytes = __builtin_amdgcn_readfirstlane((int)(L < 0x40000000u ? 4u * L : 0xffffffffu));
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(u), 0, bytes, 0x00020000);
+    }
+    __device__ __forceinline__ DigitWords load(uint32_t w) const {
+        return DigitWords{(uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(4u * w), 0, 0),
+                          (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(4u * w + 4u), 0, 0)};
+    }
+};
+// A digit of 32 + q bits (shift: its digit_shift): low word and the rest.
+__device__ __forceinline__ uint32_t digit_lo(const DigitWords &d, uint32_t shift) {
+    return __builtin_amdgcn_alignbit(d.b, d.a, shift);
+}
+__device__ __forceinline__ uint32_t digit_hi(const DigitWords &d, uint32_t shift, uint32_t q) {
+    return (d.b >> shift) & ((1u << q) - 1u);
+}
+// 2^32 hi + lo, hi < 2^20, exactly: the mantissa of 2^52 + that.
+__device__ __forceinline__ double digit_value(uint32_t lo, uint32_t hi) {
+    return __hiloint2double((int)(0x43300000u | hi), (int)lo) - 0x1p52;
+}
+
+// The words of one tile block's digits for the first forward level: element u
+// of the thread's column.
 template <int M>
-__device__ __forceinline__ void load_limbs(uint32_t *x, const PassArgs &a, const BlockPos &bp, const ColThread<M> &ct) {
+__device__ __forceinline__ void load_words(DigitWords *x, const PassArgs &a, const BlockPos &bp, const ColThread<M> &ct) {
     const NttOp o = a.ops[bp.seg];
     const uint32_t *X = o.X + (size_t)bp.row * o.s;
     uint32_t LX = o.L;
@@ -626,70 +664,84 @@ __device__ __forceinline__ void load_limbs(uint32_t *x, const PassArgs &a, const
             LX = rr.L_a;
         }
     }
+    // 2^ustep is a multiple of 512: the elements' shifts are equal, and element
+    // u's words lie u step words on
+    const Words words(X, LX);
+    const uint32_t w0 = (uint32_t)digit_word(ct.off0, a.q);
+    const uint32_t step = (uint32_t)digit_word(1ull << (a.plan.log2K - 4), a.q);
     memory_first_begin();
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        const uint64_t off = ct.off(u);
-        x[u] = off < LX ? X[off] : 0u;
-    }
+    for (int u = 0; u < 16; ++u) x[u] = words.load(w0 + (uint32_t)u * step);
     memory_first_end();
 }
 
-// First forward column level, persistent: block b works through the tile
-// blocks w = b, b + gridDim.x, ... (numbered and XCD-ordered as one block per
-// tile block would be; gridDim.x is a multiple of the XCD count).  The limbs
-// stay in registers as 32-bit words and each prime converts them; once the
-// second prime has, the next tile block's limbs are loaded into the same
-// registers, so that their latency (and the completion of the first
-// prime's stores before them) overlaps the second prime's transform and
-// stores.  Each prime's column twiddles are loaded after its transform (not
-// held through it), which brings the 2^6..2^8-point levels to 121-125 VGPRs:
-// four waves per SIMD without spills (at 10^9 digits 179 -> 165 ms per
-// step, against three waves).  The 2^5 and 2^9-point levels would spill
-// at four and keep three.
-constexpr int limbs_waves(int m) { return m >= 6 && m <= 8 ? 4 : 3; }
-// TRUNC: only the rows of the transforms' first parts are stored.
+// A thread's digits: low words, and the rest of four digits to a word.
+struct Digits {
+    uint32_t lo[16], hi[4];
+    __device__ __forceinline__ void set(const DigitWords *x, uint32_t shift, uint32_t q) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) lo[u] = digit_lo(x[u], shift);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            hi[i] = 0;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) hi[i] |= digit_hi(x[4 * i + b], shift, q) << (8 * b);
+        }
+    }
+    __device__ __forceinline__ void opaque() {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) __asm__ volatile("" : "+v"(lo[u]));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) __asm__ volatile("" : "+v"(hi[i]));
+    }
+    __device__ __forceinline__ double value(int u) const {
+        return digit_value(lo[u], (hi[u >> 2] >> (8 * (u & 3))) & 255u);
+    }
+};
+
+// First forward column level: a block per tile block (or pair).  The words of
+// the tile are loaded once and stay in registers as packed digits, which each
+// prime converts.  Each prime's column twiddles are loaded after its transform
+// (fewer registers held through it); 110-122 VGPRs and a 34.8 KB tile give
+// four waves per SIMD.  Bound by the latency of transform -> scattered stores:
+// 3.2 TB/s at 10^9 digits (144 ms per step).  Slower there: persistent blocks
+// that load the next tile's words before the second prime's stores (169 ms, no
+// spills), the second prime's tables loaded before the first prime's stores
+// (167 ms), both primes stored at the end (244 ms, spills).  TRUNC: only the
+// rows of the transforms' first parts are stored.
 template <int M, bool PAIR, bool TRUNC>
-__global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) __attribute__((amdgpu_waves_per_eu(limbs_waves(M))))
-ntt_col_fwd_limbs_kernel(PassArgs a, uint32_t total) {
+__global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) __attribute__((amdgpu_waves_per_eu(4)))
+ntt_col_fwd_limbs_kernel(PassArgs a) {
     using CP = ColPair<M, PAIR>;
     __shared__ double lds_tiles[CP::kLdsWords];
     double *const lds = lds_tiles + CP::half() * CP::kTileStride;
-    const uint32_t tiles = tiles_per_product(a.plan) >> CP::kLog2;
-    uint32_t w = blockIdx.x;
-    if (w >= total) return;  // uniform over the block
-    BlockPos bp = block_pos_of(xcd_tile(w, total, a.xcd_log2), a.op_start, a.n_ops, tiles);
-    uint32_t x[16];
-    load_limbs<M>(x, a, bp, ColThread<M>(a.plan, 0, (bp.t << CP::kLog2) + CP::half(), CP::vtid()));
-    for (;;) {
-        const ColThread<M> ct(a.plan, 0, (bp.t << CP::kLog2) + CP::half(), CP::vtid());
-        const NttOp o = a.ops[bp.seg];
-        double *T0 = a.T + o.base + (size_t)bp.row * plane_row_elems(a.plan);
-        double *T1 = T0 + o.pstride;
-        const uint32_t rows_end = TRUNC ? tau_rows(M, fwd_tau(a, bp.seg, bp.row)) : 1u << M;
-        double v[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = (double)x[u];
-        col_fwd_prime_late<M, 0>(v, lds, ct, a.tables);
-        memory_first_begin();
-        col_store_last<M, TRUNC>(T0, v, ct, rows_end);
-        memory_first_end();
-#pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = (double)x[u];
-        const uint32_t wn = w + gridDim.x;
-        const bool more = wn < total;  // uniform over the block
-        if (more) {
-            bp = block_pos_of(xcd_tile(wn, total, a.xcd_log2), a.op_start, a.n_ops, tiles);
-            load_limbs<M>(x, a, bp, ColThread<M>(a.plan, 0, (bp.t << CP::kLog2) + CP::half(), CP::vtid()));
-        }
-        // the barrier at its end lets the next tile block reuse `lds`
-        col_fwd_prime_late<M, 1>(v, lds, ct, a.tables);
-        memory_first_begin();
-        col_store_last<M, TRUNC>(T1, v, ct, rows_end);
-        memory_first_end();
-        if (!more) break;
-        w = wn;
+    const BlockPos bp = block_pos(a.op_start, a.n_ops, tiles_per_product(a.plan) >> CP::kLog2, a.xcd_log2);
+    const ColThread<M> ct(a.plan, 0, (bp.t << CP::kLog2) + CP::half(), CP::vtid());
+    Digits d;
+    {
+        DigitWords x[16];
+        load_words<M>(x, a, bp, ct);
+        d.set(x, digit_shift(ct.off0, a.q), a.q);
     }
+    const NttOp o = a.ops[bp.seg];
+    double *T0 = a.T + o.base + (size_t)bp.row * plane_row_elems(a.plan);
+    double *T1 = T0 + o.pstride;
+    const uint32_t rows_end = TRUNC ? tau_rows(M, fwd_tau(a, bp.seg, bp.row)) : 1u << M;
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = d.value(u);
+    col_fwd_prime_late<M, 0>(v, lds, ct, a.tables);
+    memory_first_begin();
+    col_store_last<M, TRUNC>(T0, v, ct, rows_end);
+    memory_first_end();
+    __syncthreads();
+    d.opaque();  // converted again, not kept as doubles
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = d.value(u);
+    col_fwd_prime_late<M, 1>(v, lds, ct, a.tables);
+    memory_first_begin();
+    col_store_last<M, TRUNC>(T1, v, ct, rows_end);
+    memory_first_end();
 }
 
 // Step-0 elements of a row tile (DFT size 2^M): v[j] is tile index
@@ -877,41 +929,73 @@ __device__ __forceinline__ uint32_t row_shr(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x110 + D, 0xf, 0xf, true);
 }
 
-// The limb at a lane's coefficient c, 2^RL adjacent lanes holding a run of
-// adjacent coefficients (lane mod 2^RL: the position in the run): coefficient
-// c = w0 + 2^32 w1 + 2^64 w2 adds to the limb column sums
-// s_j = w0_j + w1_(j-1) + w2_(j-2), which become limbs with one neighbour
-// shift and one ballot carry resolution per run; what passes the run's top
-// is left in `over` of its last lane.
+template <int D>
+__device__ __forceinline__ uint32_t row_shl(uint32_t x) {
+    static_assert(D >= 1 && D <= 15, "row_shl:1..15");
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x100 + D, 0xf, 0xf, true);
+}
+
+// The product words of a run of 2^RL adjacent coefficients in 2^RL adjacent
+// lanes (lane mod 2^RL: the position in the run).  With d = 32 + q bits per
+// digit, coefficient c = e0 + 2^d e1 + 2^2d e2 adds to the digit column sums
+// s_j = e0_j + e1_(j-1) + e2_(j-2), which become digits with one neighbour
+// shift and one ballot carry resolution per run; what passes the run's top is
+// left in `over` of its last lane (below 2^64: 2^2d times the terms of a
+// coefficient stays below 2^98).  The lane's words start in its digit
+// (lane_word): `word` from bit `shift` of the digit on, `next` from bit 32 on,
+// both with the low end of the next lane's digit.
+struct RunWords {
+    uint32_t word, next;
+};
 template <int RL>
-__device__ __forceinline__ uint32_t run_limb(unsigned __int128 c, uint32_t lane, uint64_t &over) {
+__device__ __forceinline__ RunWords run_digits(unsigned __int128 c, uint32_t lane, uint32_t q, uint32_t shift,
+                                               uint64_t &over) {
     constexpr uint32_t kRun = 1u << RL;
     const uint32_t jr = lane & (kRun - 1u);
     uint64_t last_mask = 0;  // last lanes of runs pass no carry on
 #pragma unroll
     for (uint32_t l = kRun - 1; l < kWave; l += kRun) last_mask |= 1ull << l;
-    const uint32_t w0 = (uint32_t)c, w1 = (uint32_t)(c >> 32), w2 = (uint32_t)(c >> 64);
-    const uint32_t w1a = row_shr<1>(w1), w2a = row_shr<1>(w2), w2b = row_shr<2>(w2);
-    const uint64_t s = (uint64_t)w0 + (jr >= 1 ? w1a : 0u) + (jr >= 2 ? w2b : 0u);
-    const uint32_t lo = (uint32_t)s, hi = (uint32_t)(s >> 32);
-    const uint32_t hia = row_shr<1>(hi);
-    const uint64_t t = (uint64_t)lo + (jr >= 1 ? hia : 0u);
-    const uint32_t lo2 = (uint32_t)t;
-    const bool gen = (t >> 32) != 0, prop = lo2 == 0xffffffffu;
-    const uint64_t G = ballot64(gen) & ~last_mask, P = ballot64(prop) & ~last_mask;
-    uint32_t unused;
-    const uint64_t cm = resolve_carries(G, P, 0u, &unused);
-    const uint32_t ci = (uint32_t)(cm >> lane) & 1u;
-    // V >> 32 kRun: the carry out of the top limb, the top column's high part
-    // and the words of the last two coefficients past the run
-    const uint64_t cout = (gen || (prop && ci)) ? 1u : 0u;
-    over = cout + hi + (uint64_t)w1 + (uint64_t)w2a + ((uint64_t)w2 << 32);
-    return lo2 + ci;
+    // neighbours' words: zero below the run (a run of 16 is a DPP row)
+    const auto below1 = [&](uint32_t x) {
+        const uint32_t y = row_shr<1>(x);
+        return RL == 4 || jr >= 1 ? y : 0u;
+    };
+    const auto below2 = [&](uint32_t x) {
+        const uint32_t y = row_shr<2>(x);
+        return RL == 4 || jr >= 2 ? y : 0u;
+    };
+    const uint32_t w0 = (uint32_t)c, w1 = (uint32_t)(c >> 32), w2 = (uint32_t)(c >> 64), w3 = (uint32_t)(c >> 96);
+    const uint32_t mq = (1u << q) - 1u;
+    const uint64_t e0 = (uint64_t)(w1 & mq) << 32 | w0;
+    const uint32_t e1l = __builtin_amdgcn_alignbit(w2, w1, q), e1h = __builtin_amdgcn_alignbit(w3, w2, q) & mq;
+    const uint32_t e2 = __builtin_amdgcn_alignbit(w3, w2, 2u * q);
+    const uint64_t s = e0 + ((uint64_t)below1(e1h) << 32 | below1(e1l)) + below2(e2);
+    const uint32_t hi = (uint32_t)(s >> 32) >> q;
+    uint32_t tc;
+    const uint32_t tl = __builtin_addc((uint32_t)s, below1(hi), 0u, &tc), th = ((uint32_t)(s >> 32) & mq) + tc;
+    // a digit that carries, or passes a carry on, is rare (2^-32): only a wave
+    // with one resolves its carries
+    uint64_t f = (uint64_t)th << 32 | tl;
+    uint32_t cout = 0;
+    const uint64_t ones = (uint64_t)mq << 32 | 0xffffffffu;
+    const uint64_t GP = ballot64(f >= ones);
+    if (__builtin_expect(GP != 0, 0)) {
+        const uint64_t P = ballot64(f == ones);
+        uint32_t unused;
+        const uint64_t cm = resolve_carries((GP ^ P) & ~last_mask, P & ~last_mask, 0u, &unused);
+        f += (cm >> lane) & 1u;
+        cout = f > ones ? 1u : 0u;
+    }
+    // V >> d kRun: the carry out of the top digit, the top column's high part
+    // and the digits of the last two coefficients past the run
+    over = ((uint64_t)e1h << 32 | e1l) + ((uint64_t)(e2 << q) << 32 | (hi + cout)) + below1(e2);
+    const uint32_t fl = (uint32_t)f, next = ((uint32_t)(f >> 32) & mq) | row_shl<1>(fl) << q;
+    return RunWords{__builtin_amdgcn_alignbit(next, fl, shift), next};
 }
 
 // First inverse column level: both primes through one tile, 1/K, Garner,
-// and the limbs of each run of adjacent coefficients with the run's spill
-// word (run_limb; the carry engine adds it).  A thread's element u is (row
+// and the words of each run of adjacent coefficients with the run's spill
+// word (run_digits; the carry engine adds it).  A thread's element u is (row
 // r0 + u 2^(M-4), column g) and lanes hold adjacent columns, so a run of 2^RL
 // adjacent coefficients sits in 2^RL adjacent lanes.
 template <int M, bool PAIR, bool TRUNC>
@@ -955,18 +1039,24 @@ ntt_col_inv_limbs_kernel(PassArgs a) {
     const uint32_t lane = threadIdx.x & (kWave - 1u);
     const uint32_t jr = lane & (kRun - 1u);  // position inside the run
     uint32_t *out = pr.C + (size_t)prod * pr.sC;
-    const uint32_t Lc = pr.Lc;
     uint64_t *spill = a.spill + pr.spill_base + (size_t)prod * ((1ull << log2K) >> RL);
-    const uint64_t n_u0 = ct.off0;  // coefficient index of element u = 0
+    const uint32_t shift = lane_shift(jr, a.q);
+    const bool two = a.q != 0 && shift == 0;  // the lane starts two words
+    // byte offsets (below 2^32) of the lane's word and its run's spill word
+    // from uniform bases; adjacent elements are a whole number of runs apart
+    const uint32_t words = run_words(RL, a.q), run0 = (uint32_t)(ct.off0 >> RL), runs = 1u << (log2K - 4 - RL);
+    const uint32_t n0 = 4u * (run0 * words + lane_word(jr, a.q)), n_step = 4u * words * runs, n_last = 4u * (pr.Lc - 1u);
+    const auto at = [](void *p, uint32_t bytes) { return static_cast<char *>(p) + bytes; };
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
         if (TRUNC && u >= (int)kTauMin && u >= (int)tau) break;  // uniform over the block
         const unsigned __int128 c = recombine(v0[u], lds[ct.lds0 + 272u * u]);
-        const uint64_t n = n_u0 + ((uint64_t)u << ct.ustep);
         uint64_t over;
-        const uint32_t limb = run_limb<RL>(c, lane, over);
-        if (n < Lc) out[n] = limb;
-        if (jr == kRun - 1) spill[(n - jr) >> RL] = over;
+        const RunWords rw = run_digits<RL>(c, lane, a.q, shift, over);
+        const uint32_t n = n0 + (uint32_t)u * n_step;
+        if (n <= n_last) *reinterpret_cast<uint32_t *>(at(out, n)) = rw.word;
+        if (two && n < n_last) *reinterpret_cast<uint32_t *>(at(out, n + 4u)) = rw.next;
+        if (jr == kRun - 1) *reinterpret_cast<uint64_t *>(at(spill, 8u * (run0 + (uint32_t)u * runs))) = over;
     }
 }
 
@@ -1139,10 +1229,10 @@ __global__ void __launch_bounds__(256) ntt_thin_fwd_kernel(PassArgs a) {
     const int P = (int)(bp.t & 1u);
     const NttOp o = a.ops[bp.seg];
     const ThinCol tc(a.plan, bp.t >> 1, threadIdx.x);
-    const uint32_t *X = o.X + (size_t)bp.row * o.s;
-    uint32_t x[4];
+    const Words words(o.X + (size_t)bp.row * o.s, o.L);
+    DigitWords x[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) x[u] = tc.off(u) < o.L ? X[tc.off(u)] : 0u;
+    for (int u = 0; u < 4; ++u) x[u] = words.load((uint32_t)digit_word(tc.off(u), a.q));
     const double *tab = a.tables + P * kPrimeTable;
     ThinTw<kThinCol, true, LT> tw;
     tw.load(tab + kOffStep4, tc.tid);
@@ -1150,7 +1240,10 @@ __global__ void __launch_bounds__(256) ntt_thin_fwd_kernel(PassArgs a) {
     const Mod m = mod_of(P);
     double v[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = (double)x[u];
+    for (int u = 0; u < 4; ++u) {
+        const uint32_t shift = digit_shift(tc.off(u), a.q);
+        v[u] = digit_value(digit_lo(x[u], shift), digit_hi(x[u], shift, a.q));
+    }
     thin_fwd<kThinCol, true, LT, false, kDifToTwiddle, kDifToTwiddle>(v, v, lds, lds, tw, tc.tid, c_ntt.w16[P], m);
     ctw.apply(v, m);
     double *T = a.T + o.base + P * o.pstride + ((size_t)bp.row << log2K);
@@ -1233,16 +1326,20 @@ __global__ void __launch_bounds__(512) ntt_thin_inv_kernel(PassArgs a) {
     const double *other = lds_tiles + (1 - P) * thin_slots(LT);
     uint32_t *out = pr.C + (size_t)bp.row * pr.sC;
     uint64_t *spill = a.spill + pr.spill_base + ((size_t)bp.row << (log2K - RL));
-    const uint32_t lane = threadIdx.x & (kWave - 1u);
+    const uint32_t lane = threadIdx.x & (kWave - 1u), jr = lane & ((1u << RL) - 1u);
+    const uint32_t words = run_words(RL, a.q), shift = lane_shift(jr, a.q);
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
         const double mine = P ? v[e + 2] : v[e];
         const double theirs = other[P ? s0.slot(e + 2) : s0.slot(e)];
-        const uint32_t n = P ? tc.off(e + 2) : tc.off(e);
+        const uint32_t run = (P ? tc.off(e + 2) : tc.off(e)) >> RL;
         uint64_t over;
-        const uint32_t limb = run_limb<RL>(P ? recombine(theirs, mine) : recombine(mine, theirs), lane, over);
-        if (n < pr.Lc) out[n] = limb;
-        if ((lane & ((1u << RL) - 1u)) == (1u << RL) - 1u) spill[n >> RL] = over;
+        const RunWords rw =
+            run_digits<RL>(P ? recombine(theirs, mine) : recombine(mine, theirs), lane, a.q, shift, over);
+        const uint32_t n = run * words + lane_word(jr, a.q);
+        if (n < pr.Lc) out[n] = rw.word;
+        if (a.q != 0 && shift == 0 && n + 1 < pr.Lc) out[n + 1] = rw.next;
+        if (jr == (1u << RL) - 1u) spill[run] = over;
     }
 }
 
@@ -1434,6 +1531,13 @@ int transform_log2(uint32_t L_a, uint32_t L_b) {
     return k < kMinLog2 ? kMinLog2 : k;
 }
 
+// Whether digits of `bits` bits keep the coefficients of a product whose
+// shorter operand has n digits below p0 p1.
+bool digits_exact(uint64_t n, uint32_t bits) {
+    // n (2^bits - 1)^2 then also stays p0 below (recombine)
+    return (unsigned __int128)n << (2u * bits) < (unsigned __int128)kPrime0 * kPrime1;
+}
+
 size_t chunk_products(uint32_t N, int log2K) {
     size_t n = kChunkElems >> log2K;
     if (n < 1) n = 1;
@@ -1516,42 +1620,40 @@ Plan active_plan(int k) {
     return make_plan_split(k, (int)(s & 0xffu), (int)(s >> 8));
 }
 
+// Digits are wider than limbs up to transforms of 2^29 points: there the byte
+// offsets of their words fit 32 bits.
+constexpr int kWideMaxLog2 = 29;
+
+static_assert(kNttOneTileLog2 == kTileLog2, "as the callers know it");
+
+// The widest digits of the products A1 B and A2 B (L2 = 0: of A1 B alone)
+// that keep their coefficients exact, and the transform that holds either
+// product: 40 bits up to 2^18 digits in the shorter operand, 36 up to 2^26,
+// else 34.  A coefficient costs the same whatever its digits, so the widest
+// ones take the fewest: 20, 11 and 6 % fewer than limbs.  Limbs / wide digits:
+// 96 products of 24007 x 20011 limbs 157 / 141 us, 24000001 x 20000003 limbs
+// 2.70 / 2.33 ms, 3 of 158864 x 120218 limbs 75 / 50 us, 10^9 digits of pi
+// 787 / 734 ms.  One-tile products (limbs as digits) stay so: their kernel
+// forms limbs in place.
+NttShape shape_for(uint32_t L1, uint32_t L2, uint32_t Lb) {
+    const int k32 = transform_log2(std::max(L1, L2), Lb);
+    if (k32 <= kTileLog2) return NttShape{k32, 32u};
+    for (const uint32_t bits : {40u, 36u, 34u}) {
+        const uint64_t d = digits_of(std::max(L1, L2), bits), db = digits_of(Lb, bits);
+        if (!digits_exact(std::min(d, db), bits)) continue;
+        const int k = std::max(log2_ceil(d + db), kTileLog2 + 1);
+        if (k > kWideMaxLog2) continue;
+        const int rl = std::min(run_log2_for(active_plan(k).log2M[0]), k <= kThinMaxLog2 ? kThinTileLog2 - kThinCol : 4);
+        if (run_fits(rl, bits - 32u)) return NttShape{k, bits};
+    }
+    return NttShape{k32, 32u};
+}
+
 // Launch shape (gpupi_ntt_set_launch): which column level kinds pair their
 // tiles, and the XCD chunk of the block order.  Read once per product
 // launch sequence.
 std::atomic<uint32_t> g_pair_mask{kPairMaskDefault};
 std::atomic<int> g_xcd_log2{kXcdChunkLog2};
-
-// Blocks of the persistent first-level kernel: as many as fit on the device
-// at once (a multiple of the XCD count), or one per tile block when there
-// are fewer.
-uint32_t device_cus() {
-    static std::atomic<int> cus{0};
-    int n = cus.load(std::memory_order_relaxed);
-    if (n == 0) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1)
-            n = 1;
-        cus.store(n, std::memory_order_relaxed);
-    }
-    return (uint32_t)n;
-}
-template <int M, bool PAIR, bool TRUNC>
-__global__ void ntt_col_fwd_limbs_kernel(PassArgs a, uint32_t total);
-template <int M, bool PAIR, bool TRUNC>
-uint32_t persistent_grid(uint32_t total) {
-    static std::atomic<int> per_cu{0};
-    int b = per_cu.load(std::memory_order_relaxed);
-    if (b == 0) {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, ntt_col_fwd_limbs_kernel<M, PAIR, TRUNC>,
-                                                         ColPair<M, PAIR>::kThreads, 0) != hipSuccess || b < 1)
-            b = 1;
-        per_cu.store(b, std::memory_order_relaxed);
-    }
-    const uint64_t fit = ((uint64_t)b * device_cus()) / kXcds * kXcds;
-    return (uint32_t)std::min<uint64_t>(total, fit < kXcds ? kXcds : fit);
-}
 
 // Calls f(PAIR, TRUNC) as std::integral_constants: PAIR = pair where a level of
 // 2^M points can pair its tiles, false otherwise.
@@ -1573,6 +1675,10 @@ void with_flags(bool pair, bool trunc, F &&f) {
 size_t spill_runs_bound(int k) { return (size_t(1) << k) >> run_log2_for(kColMaxLog2); }
 
 }  // namespace
+
+uint32_t ntt_tau(uint32_t L_a, uint32_t L_b, int log2K, uint32_t bits) {
+    return tau_of(digits_of(L_a, bits) + digits_of(L_b, bits), log2K);
+}
 
 void ntt_stats_suspend(bool suspend) { t_stats_off = suspend; }
 
@@ -1661,16 +1767,16 @@ void ntt_tables_release(NTTPrecomputedTables *tables) {
 
 namespace {
 
-// Copies limbs [0, L_a + L_b) of each staged product row (stride K) to its
+// Copies limbs [0, L_a + L_b) of each staged product row to its
 // row's C (rows without C stay staged for their assembly).  Blocks: (row,
 // 1024-limb slice).
-__global__ void __launch_bounds__(256) ragged_copy_kernel(const uint32_t *staging, uint64_t K,
+__global__ void __launch_bounds__(256) ragged_copy_kernel(const uint32_t *staging, uint64_t stride,
                                                           const RaggedRow *rows, uint32_t slices) {
     const uint32_t row = blockIdx.x / slices, slice = blockIdx.x % slices;
     const RaggedRow it = rows[row];
     if (it.C == nullptr) return;
     const uint32_t Lc = it.L_a + it.L_b;
-    const uint32_t *src = staging + (size_t)row * K;
+    const uint32_t *src = staging + (size_t)row * stride;
     for (uint32_t i = slice * 1024u + threadIdx.x; i < Lc && i < (slice + 1) * 1024u; i += 256u) it.C[i] = src[i];
 }
 
@@ -1703,6 +1809,7 @@ struct NttJob {
     const RaggedAssembly *host_asms = nullptr;
     uint32_t n_asm = 0, asm_chunks = 0;
     int k = 0;
+    uint32_t bits = 32;    // of a digit
     size_t max_chunk = 0;  // rows per launch chunk at most (0: the default)
 };
 
@@ -1716,6 +1823,9 @@ struct JobShape {
     uint32_t tau = kTauMax;  // parts of the transforms in use (the most of any product)
 };
 
+// Limbs from one staged product of a ragged launch to the next.
+uint64_t staging_stride(const NttJob &j) { return ((1ull << j.k) * j.bits) >> 5; }
+
 JobShape shape_of(const NttJob &j) {
     JobShape sh;
     const size_t K = size_t(1) << j.k;
@@ -1726,14 +1836,20 @@ JobShape shape_of(const NttJob &j) {
         sh.op_rows[pr.a] = std::max(sh.op_rows[pr.a], pr.N);
         sh.op_rows[pr.b] = std::max(sh.op_rows[pr.b], pr.N);
         used_as_a[pr.a] = true;
-        // ragged rows are staged, K words apart
-        uint64_t total = j.ragged ? 0 : (uint64_t)j.ops[pr.a].L + j.ops[pr.b].L;
-        if (j.ragged && j.host_rows == nullptr) total = K;
-        else if (j.ragged)
-            for (uint32_t i = 0; i < pr.N; ++i)
-                total = std::max<uint64_t>(total, (uint64_t)j.host_rows[i].L_a + j.host_rows[i].L_b);
-        sh.Lc[q] = (uint32_t)total;
-        sh.tau = q == 0 ? tau_of(total, j.k) : std::max(sh.tau, tau_of(total, j.k));
+        uint64_t limbs = 0, digits = 0;
+        const auto row = [&](uint32_t L_a, uint32_t L_b) {
+            limbs = std::max(limbs, (uint64_t)L_a + L_b);
+            digits = std::max(digits, digits_of(L_a, j.bits) + digits_of(L_b, j.bits));
+        };
+        if (!j.ragged) row(j.ops[pr.a].L, j.ops[pr.b].L);
+        else if (j.host_rows != nullptr)
+            for (uint32_t i = 0; i < pr.N; ++i) row(j.host_rows[i].L_a, j.host_rows[i].L_b);
+        else {
+            limbs = staging_stride(j);
+            digits = K;
+        }
+        sh.Lc[q] = (uint32_t)limbs;
+        sh.tau = q == 0 ? tau_of(digits, j.k) : std::max(sh.tau, tau_of(digits, j.k));
     }
     for (uint32_t o = 0; o < j.n_ops; ++o) {
         sh.op_bcast[o] = !j.ragged && !used_as_a[o] && j.ops[o].s == 0 && sh.op_rows[o] > 1;
@@ -1743,8 +1859,17 @@ JobShape shape_of(const NttJob &j) {
     return sh;
 }
 
+// Whether a product of these lengths fits a transform of 2^k digits, exactly.
+bool row_fits(uint32_t L_a, uint32_t L_b, int k, uint32_t bits) {
+    const uint64_t da = digits_of(L_a, bits), db = digits_of(L_b, bits);
+    return da + db <= 1ull << k && digits_exact(std::min(da, db), bits);
+}
+
 // Whether the operands and products describe a job run_ntt can do.
 bool job_ok(const NttJob &j) {
+    if ((j.bits != 32u && j.bits != 34u && j.bits != 36u && j.bits != 40u) || j.k < kMinLog2 || j.k > kMaxLog2 ||
+        (j.bits != 32u && (j.k <= kTileLog2 || j.k > kWideMaxLog2)))
+        return false;
     if (j.n_ops < 1 || j.n_ops > 3 || j.n_prods < 1 || j.n_prods > 2) return false;
     if (j.ragged && (j.rows == nullptr || j.host_rows == nullptr || j.bset == nullptr || j.host_bset == nullptr ||
                      j.nb == 0 || j.nb > j.prods[0].N || j.n_ops != 2 || j.n_prods != 1 ||
@@ -1756,7 +1881,7 @@ bool job_ok(const NttJob &j) {
         if (pr.a == pr.b && (j.ragged || j.n_prods != 1)) return false;  // squares: one product
         for (uint32_t r = 0; r < j.n_prods; ++r)
             if (r != q && (j.prods[r].a == pr.a || j.prods[r].b == pr.a)) return false;
-        if (!j.ragged && transform_log2(j.ops[pr.a].L, j.ops[pr.b].L) != j.k) return false;
+        if (!j.ragged && !row_fits(j.ops[pr.a].L, j.ops[pr.b].L, j.k, j.bits)) return false;
     }
     return true;
 }
@@ -1771,7 +1896,6 @@ struct JobLayout {
 
 JobLayout layout_of(const NttJob &j, const JobShape &sh) {
     JobLayout l;
-    const size_t K = size_t(1) << j.k;
     // a ragged launch is one chunk (its B set and staged pieces stay resident)
     l.nc = j.ragged ? sh.rows : chunk_products(sh.rows, j.k);
     if (j.max_chunk != 0 && l.nc > j.max_chunk) l.nc = j.max_chunk;
@@ -1790,7 +1914,7 @@ JobLayout layout_of(const NttJob &j, const JobShape &sh) {
     for (uint32_t q = 0; q < j.n_prods; ++q) fl = std::max(fl, carry_flags_bytes((uint32_t)l.nc, sh.Lc[q]));
     off += align256(fl);
     l.staging_off = off;
-    if (j.ragged) off += align256(l.nc * K * sizeof(uint32_t));
+    if (j.ragged) off += align256(l.nc * staging_stride(j) * sizeof(uint32_t));
     l.asm_flags_off = off;
     if (j.ragged) off += align256(j.asm_chunks);
     l.total = off;
@@ -1873,6 +1997,7 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
     const JobLayout l = layout_of(j, sh);
     if (workspace == nullptr || workspace_bytes < l.total) return hipErrorInvalidValue;
     const int run_log2 = thin ? ThinCol::LC : (int)final_run_log2(p);
+    if (!run_fits(run_log2, j.bits - 32u)) return hipErrorInvalidValue;
     const size_t runs = K >> run_log2;
     char *ws = static_cast<char *>(workspace);
     uint8_t *flags = reinterpret_cast<uint8_t *>(ws + l.flags_off);
@@ -1882,6 +2007,7 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
     PassArgs a{};
     a.plan = p;
     a.tables = tables.roots;
+    a.q = j.bits - 32u;
     a.xcd_log2 = g_xcd_log2.load(std::memory_order_relaxed);
     const uint32_t pair_mask = g_pair_mask.load(std::memory_order_relaxed);
     a.T = reinterpret_cast<double *>(ws);
@@ -1896,7 +2022,7 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
     if (j.ragged) {
         uint64_t parts = 0;
         for (uint32_t i = 0; i < sh.rows; ++i)
-            parts += tau_of((uint64_t)j.host_rows[i].L_a + j.host_rows[i].L_b, k);
+            parts += ntt_tau(j.host_rows[i].L_a, j.host_rows[i].L_b, k, j.bits);
         a.row_tau = 10 * parts <= 9 * (uint64_t)kTauMax * sh.rows;
         if (!a.row_tau) tau = kTauMax;
     }
@@ -1932,7 +2058,7 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
             d.b = pr.b;
             d.b_bcast = sh.op_bcast[pr.b] ? 1u : 0u;
             d.C = j.ragged ? staging : pr.C + r0 * pr.sC;
-            d.sC = j.ragged ? (uint32_t)K : pr.sC;
+            d.sC = j.ragged ? (uint32_t)staging_stride(j) : pr.sC;
             d.Lc = sh.Lc[q];
             d.spill_base = q * spill_stride;
             prod_row0[q] = (uint32_t)prod_rows;
@@ -1975,10 +2101,8 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
                     with_flags<M>((pair_mask >> kPairFwdLimbs) & 1u, trunc, [&](auto pc, auto tc) {
                         constexpr bool kPair = decltype(pc)::value, kTrunc = decltype(tc)::value;
                         constexpr int pl = ColPair<M, kPair>::kLog2;
-                        const uint32_t total = blocks(fwd_rows, tiles, pl).x;
-                        hipLaunchKernelGGL((ntt_col_fwd_limbs_kernel<M, kPair, kTrunc>),
-                                           dim3(persistent_grid<M, kPair, kTrunc>(total)), dim3(256 << pl), 0, stream,
-                                           args(tiles, pl), total);
+                        hipLaunchKernelGGL((ntt_col_fwd_limbs_kernel<M, kPair, kTrunc>), blocks(fwd_rows, tiles, pl),
+                                           dim3(256 << pl), 0, stream, args(tiles, pl));
                     });
                 });
             }));
@@ -2058,23 +2182,29 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
             if (rows[q] == 0) continue;
             const NttProd &d = a.prods[q];
             GPUPI_RETURN_IF(launch_add_spills(d.C, a.spill + d.spill_base, rows[q], d.Lc, d.sC,
-                                              1u << run_log2, (uint32_t)runs, flags, stream));
+                                              run_words(run_log2, a.q), (uint32_t)runs, flags, stream));
         }
         if (j.ragged) {
             bool copies = false;
             for (uint32_t i = 0; i < rows[0] && !copies; ++i) copies = j.host_rows[i].C != nullptr;
-            const uint32_t slices = (uint32_t)ceil_div64(K, 1024);
+            const uint64_t stride = staging_stride(j);
+            const uint32_t slices = (uint32_t)ceil_div64(stride, 1024);
             if ((uint64_t)rows[0] * slices > 0x7fffffffull) return hipErrorInvalidValue;
             if (copies) {
                 hipLaunchKernelGGL(ragged_copy_kernel, dim3(rows[0] * slices), dim3(256), 0, stream, staging,
-                                   (uint64_t)K, a.rows, slices);
+                                   stride, a.rows, slices);
                 GPUPI_RETURN_IF(hipGetLastError());
             }
-            GPUPI_RETURN_IF(launch_ragged_assemble(staging, K, j.asms, j.n_asm, j.asm_chunks,
+            GPUPI_RETURN_IF(launch_ragged_assemble(staging, stride, j.asms, j.n_asm, j.asm_chunks,
                                                    reinterpret_cast<uint8_t *>(ws + l.asm_flags_off), stream));
         }
     }
     return hipSuccess;
+}
+
+void set_shape(NttJob &j, const NttShape &s) {
+    j.k = s.k;
+    j.bits = s.bits;
 }
 
 // A uniform product C = A B of N rows; a broadcast A (stride 0) is swapped
@@ -2092,7 +2222,7 @@ NttJob uniform_job(const uint32_t *A, const uint32_t *B, uint32_t *C, uint32_t N
         j.prods[0].C = C;
         j.prods[0].sC = stride_C;
         j.prods[0].N = N;
-        j.k = transform_log2(L_a, L_b);
+        set_shape(j, shape_for(L_a, 0, L_b));
         return j;
     }
     if (stride_A == 0 && stride_B != 0) {
@@ -2109,7 +2239,7 @@ NttJob uniform_job(const uint32_t *A, const uint32_t *B, uint32_t *C, uint32_t N
     j.prods[0].C = C;
     j.prods[0].sC = stride_C;
     j.prods[0].N = N;
-    j.k = transform_log2(L_a, L_b);
+    set_shape(j, shape_for(L_a, 0, L_b));
     return j;
 }
 
@@ -2133,7 +2263,7 @@ NttJob shared_job(const uint32_t *A1, uint32_t L1, uint32_t s1, uint32_t N1, uin
     j.prods[1].C = C2;
     j.prods[1].sC = sC2;
     j.prods[1].N = N2;
-    j.k = transform_log2(L1, Lb);
+    set_shape(j, shape_for(L1, L2, Lb));
     return j;
 }
 
@@ -2163,6 +2293,11 @@ hipError_t launch_mul_ntt_bounded(const uint32_t *A, const uint32_t *B, uint32_t
     if (!ntt_supports(L_a, L_b) || tables.roots == nullptr) return hipErrorInvalidValue;
     NttJob j = uniform_job(A, B, C, N, L_a, L_b, stride_A, stride_B, stride_C);
     if (make_plan(j.k).levels > 1) {
+        // what fits does not depend on the digits: one row of limbs has to
+        NttJob limbs = j;
+        set_shape(limbs, NttShape{transform_log2(L_a, L_b), 32u});
+        limbs.max_chunk = 1;
+        if (layout_of(limbs, shape_of(limbs)).total > workspace_bytes) return hipErrorInvalidValue;
         // the most rows per chunk whose planes, spills and flags fit
         const JobShape sh = shape_of(j);
         size_t nc = chunk_products(sh.rows, j.k);
@@ -2204,12 +2339,13 @@ hipError_t launch_mul_ntt_shared(const uint32_t *A1, uint32_t L1, uint32_t s1, u
 
 int ntt_transform_log2(uint32_t L_a, uint32_t L_b) { return transform_log2(L_a, L_b); }
 
-uint32_t ntt_tau(uint32_t L_a, uint32_t L_b, int log2K) { return tau_of((uint64_t)L_a + L_b, log2K); }
+NttShape ntt_shape(uint32_t L_a, uint32_t L_b) { return shape_for(L_a, 0, L_b); }
+
 
 namespace {
 NttJob ragged_job(const RaggedRow *rows, const RaggedRow *host_rows, uint32_t N, const RaggedB *bset,
                   const RaggedB *host_bset, uint32_t nb, const RaggedAssembly *asms,
-                  const RaggedAssembly *host_asms, uint32_t n_asm, uint32_t asm_chunks, int log2K) {
+                  const RaggedAssembly *host_asms, uint32_t n_asm, uint32_t asm_chunks, const NttShape &shape) {
     NttJob j;
     j.n_ops = 2;
     j.n_prods = 1;
@@ -2224,7 +2360,7 @@ NttJob ragged_job(const RaggedRow *rows, const RaggedRow *host_rows, uint32_t N,
     j.host_asms = host_asms;
     j.n_asm = n_asm;
     j.asm_chunks = asm_chunks;
-    j.k = log2K;
+    set_shape(j, shape);
     return j;
 }
 
@@ -2232,14 +2368,13 @@ NttJob ragged_job(const RaggedRow *rows, const RaggedRow *host_rows, uint32_t N,
 // transform and B set, assembled rows only above one tile, each assembly's
 // pieces rows without C in its range, chunks numbered in order.
 bool ragged_ok(const RaggedRow *rows, uint32_t N, const RaggedB *bset, uint32_t nb, const RaggedAssembly *asms,
-               uint32_t n_asm, uint32_t chunks, int log2K) {
-    const uint64_t K = 1ull << log2K;
+               uint32_t n_asm, uint32_t chunks, const NttShape &shape) {
     for (uint32_t i = 0; i < N; ++i) {
         const RaggedRow &r = rows[i];
-        if (r.b >= nb || (uint64_t)r.L_a + r.L_b > K || bset[r.b].L != r.L_b ||
-            bset[r.b].tau < tau_of((uint64_t)r.L_a + r.L_b, log2K) || bset[r.b].tau > kTauMax)
+        if (r.b >= nb || !row_fits(r.L_a, r.L_b, shape.k, shape.bits) || bset[r.b].L != r.L_b ||
+            bset[r.b].tau < ntt_tau(r.L_a, r.L_b, shape.k, shape.bits) || bset[r.b].tau > kTauMax)
             return false;
-        if (r.C == nullptr && log2K <= kTileLog2) return false;
+        if (r.C == nullptr && shape.k <= kTileLog2) return false;
     }
     uint32_t next = 0;
     for (uint32_t q = 0; q < n_asm; ++q) {
@@ -2278,17 +2413,17 @@ __global__ void __launch_bounds__(256) piece_rows_kernel(RaggedRow *rows, Ragged
 struct PiecesLayout {
     size_t rows_bytes, bset_bytes, asm_bytes, ntt_bytes;
     uint32_t chunks;
-    int k;
+    NttShape shape;
 };
 PiecesLayout pieces_layout(uint32_t LL, uint32_t LS, uint32_t m, uint32_t s) {
     PiecesLayout l;
-    l.k = transform_log2(s, LS);
+    l.shape = ntt_shape(s, LS);
     l.chunks = assembly_chunks(LL + LS);
     l.rows_bytes = align256((size_t)m * sizeof(RaggedRow));
     l.bset_bytes = align256(sizeof(RaggedB));
     l.asm_bytes = align256(sizeof(RaggedAssembly));
     l.ntt_bytes =
-        job_workspace_bytes(ragged_job(nullptr, nullptr, m, nullptr, nullptr, 1, nullptr, nullptr, 1, l.chunks, l.k));
+        job_workspace_bytes(ragged_job(nullptr, nullptr, m, nullptr, nullptr, 1, nullptr, nullptr, 1, l.chunks, l.shape));
     return l;
 }
 }  // namespace
@@ -2306,14 +2441,14 @@ hipError_t launch_mul_ntt_pieces(const uint32_t *L, uint32_t LL, const uint32_t 
         (uint64_t)LL + LS > 0xffffffffull || tables.roots == nullptr)
         return hipErrorInvalidValue;
     const PiecesLayout l = pieces_layout(LL, LS, m, s);
-    if (l.k <= kTileLog2 || l.k > kMaxLog2 || workspace == nullptr ||
+    if (l.shape.k <= kTileLog2 || l.shape.k > kMaxLog2 || workspace == nullptr ||
         workspace_bytes < l.rows_bytes + l.bset_bytes + l.asm_bytes + l.ntt_bytes)
         return hipErrorInvalidValue;
     char *ws = static_cast<char *>(workspace);
     auto *rows = reinterpret_cast<RaggedRow *>(ws);
     auto *bset = reinterpret_cast<RaggedB *>(ws + l.rows_bytes);
     auto *as = reinterpret_cast<RaggedAssembly *>(ws + l.rows_bytes + l.bset_bytes);
-    const uint32_t tau = tau_of((uint64_t)s + LS, l.k);  // the longest pieces' parts
+    const uint32_t tau = ntt_tau(s, LS, l.shape.k, l.shape.bits);  // the longest pieces' parts
     hipLaunchKernelGGL(piece_rows_kernel, dim3((m + 255) / 256), dim3(256), 0, stream, rows, bset, as, L, LL, S, LS,
                        C, m, s, tau);
     GPUPI_RETURN_IF(hipGetLastError());
@@ -2322,26 +2457,26 @@ hipError_t launch_mul_ntt_pieces(const uint32_t *L, uint32_t LL, const uint32_t 
     for (uint32_t i = 0; i < m; ++i) host_rows[i] = piece_row(i, L, LL, S, LS, m, s, 0);
     const RaggedB host_b{S, LS, tau};
     const RaggedAssembly host_as{C, LL + LS, s, LS, m, 0, 0};
-    return run_ntt(ragged_job(rows, host_rows.data(), m, bset, &host_b, 1, as, &host_as, 1, l.chunks, l.k),
+    return run_ntt(ragged_job(rows, host_rows.data(), m, bset, &host_b, 1, as, &host_as, 1, l.chunks, l.shape),
                    ws + l.rows_bytes + l.bset_bytes + l.asm_bytes, l.ntt_bytes, tables, stream);
 }
 
-size_t ntt_ragged_workspace_bytes(uint32_t N, uint32_t nb, uint32_t chunks, int log2K) {
+size_t ntt_ragged_workspace_bytes(uint32_t N, uint32_t nb, uint32_t chunks, const NttShape &shape) {
     return job_workspace_bytes(
-        ragged_job(nullptr, nullptr, N, nullptr, nullptr, nb, nullptr, nullptr, chunks ? 1u : 0u, chunks, log2K));
+        ragged_job(nullptr, nullptr, N, nullptr, nullptr, nb, nullptr, nullptr, chunks ? 1u : 0u, chunks, shape));
 }
 
 hipError_t launch_mul_ntt_ragged(const RaggedRow *rows, const RaggedRow *host_rows, uint32_t N, const RaggedB *bset,
                                  const RaggedB *host_bset, uint32_t nb, const RaggedAssembly *asms,
-                                 const RaggedAssembly *host_asms, uint32_t n_asm, uint32_t chunks, int log2K,
+                                 const RaggedAssembly *host_asms, uint32_t n_asm, uint32_t chunks, const NttShape &shape,
                                  void *workspace, size_t workspace_bytes, const NTTPrecomputedTables &tables,
                                  hipStream_t stream) {
     if (N == 0) return hipSuccess;
-    if (tables.roots == nullptr || log2K < kMinLog2 || log2K > kMaxLog2 || rows == nullptr || host_rows == nullptr ||
+    if (tables.roots == nullptr || shape.k < kMinLog2 || shape.k > kMaxLog2 || rows == nullptr || host_rows == nullptr ||
         bset == nullptr || host_bset == nullptr || (n_asm > 0 && (asms == nullptr || host_asms == nullptr)) ||
-        !ragged_ok(host_rows, N, host_bset, nb, host_asms, n_asm, chunks, log2K))
+        !ragged_ok(host_rows, N, host_bset, nb, host_asms, n_asm, chunks, shape))
         return hipErrorInvalidValue;
-    return run_ntt(ragged_job(rows, host_rows, N, bset, host_bset, nb, asms, host_asms, n_asm, chunks, log2K),
+    return run_ntt(ragged_job(rows, host_rows, N, bset, host_bset, nb, asms, host_asms, n_asm, chunks, shape),
                    workspace, workspace_bytes, tables, stream);
 }
 

@@ -398,5 +398,34 @@ GPUPI_HD uint32_t final_run_log2(const Plan &p) {
     return p.levels == 1 ? 4u : (uint32_t)run_log2_for(p.log2M[0]);
 }
 
+// Digits.  A coefficient is one digit of 32 + q bits of the operands' limbs
+// (q = 0, 2, 4, 8: digit j lies in at most two words).  The 2^rl adjacent
+// coefficients of a run are a whole number of product words (run_words; with
+// q = 2 only runs of 16).
+GPUPI_HD uint64_t digits_of(uint64_t limbs, uint32_t bits) { return (32u * limbs + bits - 1u) / bits; }
+GPUPI_HD uint64_t digit_word(uint64_t j, uint32_t q) { return j + ((j * q) >> 5); }
+GPUPI_HD uint32_t digit_shift(uint64_t j, uint32_t q) { return (uint32_t)(j * q) & 31u; }
+GPUPI_HD bool run_fits(int rl, uint32_t q) { return ((q << rl) & 31u) == 0; }
+GPUPI_HD uint32_t run_words(int rl, uint32_t q) { return (1u << rl) + ((q << rl) >> 5); }
+// Lane jr of a run writes the words that start in its digit: word
+// lane_word(jr) of the run from bit lane_shift(jr) of the digit on, and the
+// next word too where lane_shift(jr) = 0 and q > 0.
+GPUPI_HD uint32_t lane_shift(uint32_t jr, uint32_t q) { return (0u - jr * q) & 31u; }
+GPUPI_HD uint32_t lane_word(uint32_t jr, uint32_t q) { return jr + ((jr * q + 31u) >> 5); }
+
+// Division of a limb index by a run's length: j / len = (j magic >> 32) >>
+// shift for j < 2^31, 2 <= len < 2^31 (magic = ceil(2^(32 + shift) / len) is
+// below 2^32, and its excess times j below 2^(32 + shift)).
+struct RunDivisor {
+    uint32_t len, magic, shift;
+    GPUPI_HD uint32_t run_of(uint32_t j) const { return (uint32_t)(((uint64_t)j * magic) >> 32) >> shift; }
+};
+inline RunDivisor run_divisor(uint32_t len) {
+    RunDivisor d{len, 0, 0};
+    while ((2u << d.shift) < len) ++d.shift;
+    d.magic = (uint32_t)(((1ull << (32 + d.shift)) + len - 1u) / len);
+    return d;
+}
+
 }  // namespace ntt
 }  // namespace gpupi

@@ -815,3 +815,71 @@ def test_ragged_small_products(ctx, count):
         want = int.from_bytes(A.tobytes(), "little") * int.from_bytes(B.tobytes(), "little")
         assert int.from_bytes(got[:-1].tobytes(), "little") == want, (A.size, B.size)
         assert got[-1] == PAD, (A.size, B.size)
+
+
+# p0 p1 / 2^80: the digits of 40 bits whose products' sums stay below p0 p1
+P0P1 = ((1 << 49) - (1 << 30) + 1) * 0x1FFFE00000001
+FORTY = P0P1 >> 80
+
+
+@pytest.mark.parametrize("n,la,lb,mode", [
+    (1, 4090, 7, "ones"), (1, 4096, 1, "random"), (2, 2049, 2049, "ones"), (3, 3276, 3277, "ones"),
+    (1, 3277, 3277, "ones"), (1, 6553, 1, "ones"), (300, 3000, 3553, "random"), (300, 3001, 3553, "top"),
+    (1, 20479, 20481, "ones"), (40, 20480, 20481, "ones"), (1, 163840, 163840, "ones"),
+    # the longest operands of 40-bit digits, all of their bits set, and one limb more
+    (1, FORTY * 40 // 32, FORTY * 40 // 32, "ones"), (1, FORTY * 40 // 32 + 1, FORTY * 40 // 32 + 1, "ones"),
+    (1, 500000, FORTY * 40 // 32 - 1, "top"), (1, 1179647, 1179649, "ones"), (1, 1179649, 1179649, "ones"),
+    (1, 4718593, 4718592, "random"),
+])
+def test_wide_digits(n, la, lb, mode):
+    """Products with digits wider than a limb around the lengths where their
+    number of bits or the transform changes, both ways round, padded rows, a
+    square and a shared pair: GMP's product, and nothing past a row."""
+    rng = np.random.default_rng(la * 3 + lb)
+    with g.Context() as ctx:
+        A, B = rand_rows(rng, n, la, mode), rand_rows(rng, n, lb, mode)
+        want = oracle_mul(A, B)
+        assert np.array_equal(device_mul(ctx, A, B, sa=la + 3, sb=lb + 1, sc_extra=5), want)
+        assert np.array_equal(device_mul(ctx, B, A), want)
+        if la < 200000:
+            buf, va = g.upload_rows(A)
+            bufc, vc = g.upload_rows(np.zeros((n, 2 * la), np.uint32))
+            g.check(ctx.mul(va, va, vc), "square")
+            g.synchronize()
+            assert np.array_equal(g.download_rows(vc, bufc), oracle_mul(A, A))
+            A2 = rand_rows(rng, n, max(1, la - la // 7), mode)
+            got = device_mul_shared(ctx, A, A2, B)
+            assert np.array_equal(got[0], want) and np.array_equal(got[1], oracle_mul(A2, B))
+        # the same pairs as ragged rows
+        outs, items = [], []
+        bufs = [(g.DeviceBuffer.from_array(a), g.DeviceBuffer.from_array(b)) for a, b in zip(A[:5], B[:5])]
+        for a, b in bufs:
+            c = g.DeviceBuffer.from_array(np.full(la + lb + 1, PAD, dtype=np.uint32))
+            outs.append(c)
+            items.append((a.ptr, b.ptr, c.ptr, la, lb))
+        g.check(ctx.mul_ragged(items), "mul_ragged")
+        g.synchronize()
+        for c, w in zip(outs, want):
+            got = c.download(np.uint32, count=la + lb + 1)
+            assert got[-1] == PAD and np.array_equal(got[:-1], w)
+
+
+@pytest.mark.parametrize("seed,count,lo,hi", [(1, 12, 11.5, 17.0), (2, 5, 12.0, 19.5), (3, 40, 12.0, 14.0), (4, 9, 11.9, 20.5)])
+def test_ragged_rows_of_several_sizes(ctx, seed, count, lo, hi):
+    """Ragged pairs of few rows per transform size, which share launches, next
+    to sizes of their own and unbalanced pairs in pieces: GMP's products."""
+    rng = np.random.default_rng(seed)
+    pairs, items = [], []
+    for i in range(count):
+        la, lb = (int(2.0 ** x) for x in rng.uniform(lo, hi, size=2))
+        mode = ("random", "ones", "top")[i % 3]
+        a, b = rand_rows(rng, 1, la, mode)[0], rand_rows(rng, 1, lb, mode)[0]
+        bufs = (g.DeviceBuffer.from_array(a), g.DeviceBuffer.from_array(b),
+                g.DeviceBuffer.from_array(np.full(la + lb + 1, PAD, dtype=np.uint32)))
+        pairs.append((a, b, bufs))
+        items.append((bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, la, lb))
+    g.check(ctx.mul_ragged(items), "mul_ragged")
+    g.synchronize()
+    for a, b, bufs in pairs:
+        got = bufs[2].download(np.uint32, count=len(a) + len(b) + 1)
+        assert got[-1] == PAD and np.array_equal(got[:-1], oracle_mul(a.reshape(1, -1), b.reshape(1, -1))[0])

@@ -70,3 +70,16 @@ def test_truncated_transforms(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=600)
     assert out.returncode == 0, out.stdout + out.stderr
     assert "itft check: ok" in out.stdout
+
+
+def test_digits_and_runs(tmp_path):
+    """Digits of 32 to 40 bits (gpupi_amd/csrc/ntt_plan.hpp): every digit of
+    an operand lies in two of its words and none past them, the lanes of a
+    run write each word of it once, and limb indexes are divided by a run's
+    length exactly."""
+    exe = tmp_path / "digit_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "gpupi_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "native", "digit_check.cpp"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=600)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert "digit check: ok" in out.stdout
