@@ -338,7 +338,7 @@ namespace {
 // counts 3 K points for the product as it is and (2 m + 1) K' for m pieces
 // of K' points (m forward, m inverse, one of S), each times the share that
 // transforms with tau of their 16 parts in use cost (transform_share):
-//   two pieces of ceil(L / 2) limbs at K' = K/2 when L + 2 S <= K;
+//   two pieces of ceil(L / 2) limbs at K' = K/2 when their digits fit;
 //   m >= 3 equal pieces of at least S limbs at a smaller K' when even their
 //     full transforms cost at most 0.8 of 3 K.
 // Two pieces are two products sharing S's transform, the first written in
@@ -346,9 +346,12 @@ namespace {
 // sequence (piece_row), staged and assembled.  Transforms of 2^22 points and
 // up for two pieces, 2^21 for more (smaller products are bound by launches,
 // not by transform size: at 2^20 points whole products take 69-78 us and
-// pieces 78-99).  Measured, whole / two / many (us): L = 6.17 S, 74 % of
-// 2^24: 638 / 652 / 826; L = 50 S: 636 / 642 / 493; L = 12 S, 53 %: 545 /
-// 504 / 480; L = 1.1 S, 60 %: 553 / 703 / -.
+// pieces 78-99).  Pieces fill their transforms by digits, not limbs (256
+// ragged pairs, most of them in pieces: 33.5 -> 31.1 ms).  Measured, whole /
+// pieces (us): 24000000 x 4000000 limbs 1347 / 1326 (two), 48000000 x 9000000
+// 3036 / 2709 (two), 10000000 x 1000000 546 / 504 (two), 3000000 x 300000
+// 165 / 122, 4194309 x 3000 181 / 133; 12000000 x 2000000 641 / 653 (two),
+// 24000001 x 20000003 2329 / 2682 (two).
 constexpr int kSplitMinLog2 = 22, kSplitManyMinLog2 = 21;
 
 // Time of a transform of 2^k points of which tau of 16 parts are used, in
@@ -368,12 +371,17 @@ SplitPlan split_plan(uint32_t L, uint32_t S) {
     SplitPlan p;
     const int k = gpupi::ntt_transform_log2(L, S);
     const uint64_t K = 1ull << k;
-    double best = 3.0 * (double)K * transform_share(k, gpupi::ntt_tau(L, S, k));
-    if (k >= kSplitMinLog2 && (uint64_t)L + 2ull * S <= K && (uint64_t)S < K / 2) {
-        // the second product's own passes and the add: 5 % where transforms
+    // (where the digits halve the whole product's transform, its parts are
+    // counted in limbs, at the transform it would else take)
+    const gpupi::NttShape whole = gpupi::ntt_shape(L, S);
+    double best = 3.0 * (double)K * transform_share(k, gpupi::ntt_tau(L, S, k, whole.k == k ? whole.bits : 32u));
+    // a piece of s limbs fits 2^kp points by its digits
+    const uint32_t s2 = (L + 1) / 2;
+    if (k >= kSplitMinLog2 && gpupi::ntt_piece_max(k - 1, S) >= s2 && (uint64_t)S < K / 2) {
+        // the second product's own passes and the add: 2 % where transforms
         // are large enough to show it
-        const uint32_t s = (L + 1) / 2;
-        const double cost = (k >= 23 ? 2.625 : 2.5) * (double)K * transform_share(k - 1, gpupi::ntt_tau(s, S, k - 1));
+        const uint32_t s = s2;
+        const double cost = (k >= 23 ? 2.55 : 2.5) * (double)K * transform_share(k - 1, gpupi::ntt_piece_tau(k - 1, s, S));
         if (cost < best) {
             p.m = 2;
             p.s = s;
@@ -382,12 +390,13 @@ SplitPlan split_plan(uint32_t L, uint32_t S) {
     }
     if (k < kSplitManyMinLog2) return p;
     for (uint64_t Kp = K / 2; Kp >= 2ull * S && Kp >= (1ull << 13); Kp /= 2) {
-        const uint64_t m = ((uint64_t)L + Kp - S - 1) / (Kp - S);
+        const int kp = __builtin_ctzll(Kp);
+        const uint64_t most = gpupi::ntt_piece_max(kp, S);
+        const uint64_t m = ((uint64_t)L + most - 1) / most;
         const uint64_t s = ((uint64_t)L + m - 1) / m;
         const double points = (2.0 * (double)m + 1.0) * (double)Kp;
         if (m < 3 || s < S || (m - 1) * s >= L || points > 0.8 * 3.0 * (double)K) continue;
-        const int kp = __builtin_ctzll(Kp);
-        const double cost = 1.1 * points * transform_share(kp, gpupi::ntt_tau((uint32_t)s, S, kp));
+        const double cost = 1.1 * points * transform_share(kp, gpupi::ntt_piece_tau(kp, (uint32_t)s, S));
         if (cost < best) {
             best = cost;
             p.m = (uint32_t)m;

@@ -121,6 +121,10 @@ struct NttShape {
     uint32_t bits;
 };
 NttShape ntt_shape(uint32_t L_a, uint32_t L_b);
+// The longest piece that a transform of 2^k points takes against a shorter
+// operand of S limbs (2 S <= 2^k), and the parts of it that one of s limbs uses.
+uint32_t ntt_piece_max(int k, uint32_t S);
+uint32_t ntt_piece_tau(int k, uint32_t s, uint32_t S);
 constexpr int kNttOneTileLog2 = 12;  // transforms up to here run in one tile
 // Parts (of 16) of a transform of 2^log2K points that such a product uses.
 uint32_t ntt_tau(uint32_t L_a, uint32_t L_b, int log2K, uint32_t bits = 32);

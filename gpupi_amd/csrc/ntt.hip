@@ -1626,6 +1626,15 @@ constexpr int kWideMaxLog2 = 29;
 
 static_assert(kNttOneTileLog2 == kTileLog2, "as the callers know it");
 
+// Whether a transform of 2^k points takes digits of `bits` bits whose shorter
+// operand has n of them.
+bool digits_ok(uint64_t n, uint32_t bits, int k) {
+    if (bits == 32u) return true;
+    if (k <= kTileLog2 || k > kWideMaxLog2 || !digits_exact(n, bits)) return false;
+    const int rl = std::min(run_log2_for(active_plan(k).log2M[0]), k <= kThinMaxLog2 ? kThinTileLog2 - kThinCol : 4);
+    return run_fits(rl, bits - 32u);
+}
+
 // The widest digits of the products A1 B and A2 B (L2 = 0: of A1 B alone)
 // that keep their coefficients exact, and the transform that holds either
 // product: 40 bits up to 2^18 digits in the shorter operand, 36 up to 2^26,
@@ -1640,11 +1649,8 @@ NttShape shape_for(uint32_t L1, uint32_t L2, uint32_t Lb) {
     if (k32 <= kTileLog2) return NttShape{k32, 32u};
     for (const uint32_t bits : {40u, 36u, 34u}) {
         const uint64_t d = digits_of(std::max(L1, L2), bits), db = digits_of(Lb, bits);
-        if (!digits_exact(std::min(d, db), bits)) continue;
         const int k = std::max(log2_ceil(d + db), kTileLog2 + 1);
-        if (k > kWideMaxLog2) continue;
-        const int rl = std::min(run_log2_for(active_plan(k).log2M[0]), k <= kThinMaxLog2 ? kThinTileLog2 - kThinCol : 4);
-        if (run_fits(rl, bits - 32u)) return NttShape{k, bits};
+        if (digits_ok(std::min(d, db), bits, k)) return NttShape{k, bits};
     }
     return NttShape{k32, 32u};
 }
@@ -2340,6 +2346,21 @@ hipError_t launch_mul_ntt_shared(const uint32_t *A1, uint32_t L1, uint32_t s1, u
 int ntt_transform_log2(uint32_t L_a, uint32_t L_b) { return transform_log2(L_a, L_b); }
 
 NttShape ntt_shape(uint32_t L_a, uint32_t L_b) { return shape_for(L_a, 0, L_b); }
+
+namespace {
+uint32_t piece_bits(int k, uint32_t S) {
+    for (const uint32_t bits : {40u, 36u, 34u})
+        if (digits_ok(digits_of(S, bits), bits, k)) return bits;
+    return 32u;
+}
+}  // namespace
+
+uint32_t ntt_piece_max(int k, uint32_t S) {
+    const uint32_t bits = piece_bits(k, S);
+    return (uint32_t)((((1ull << k) - digits_of(S, bits)) * bits) / 32u);
+}
+
+uint32_t ntt_piece_tau(int k, uint32_t s, uint32_t S) { return ntt_tau(s, S, k, piece_bits(k, S)); }
 
 
 namespace {
