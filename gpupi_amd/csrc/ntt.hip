@@ -374,6 +374,7 @@ struct PassArgs {
     // each ragged row uses its own)
     uint32_t tau, tau_tiles, row_tau;
     uint32_t q;  // digits of 32 + q bits
+    uint32_t streaming;  // plane_put, plane_get: past the caches
     // log2 of the tiles each XCD takes in turn (xcd_tile)
     int xcd_log2;
 };
@@ -404,6 +405,31 @@ __device__ __forceinline__ bool past_tau(const PassArgs &a, uint32_t tau, uint32
 // (first inverse 123 -> 137 ms), around the row levels' stores neutral.
 __device__ __forceinline__ void memory_first_begin() { __builtin_amdgcn_s_setprio(1); }
 __device__ __forceinline__ void memory_first_end() { __builtin_amdgcn_s_setprio(0); }
+
+// Residues of planes that no cache holds until the next kernel reads them are
+// written, and by the column levels read, with the non-temporal hint
+// (kStreamBytes): at 10^9 digits the first forward level 143 -> 136 ms per
+// step (3.27 -> 3.44 TB/s), the second levels 83 -> 76 and 52 -> 49 (4.9 ->
+// 5.4), the first inverse level 132 -> 120, the row levels' stores about 1 %.
+// The row levels' loads are without (31.8 -> 33 ms).
+template <bool NT>
+__device__ __forceinline__ void plane_put(double *p, double v) {
+    if (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+template <bool NT>
+__device__ __forceinline__ double plane_get(const double *p) {
+    return NT ? __builtin_nontemporal_load(p) : *p;
+}
+// f(std::integral_constant<bool, streaming>), the choice uniform over the
+// launch: for accesses that no arithmetic is to be interleaved with.  Kernels
+// whose last products are interleaved with their stores take the choice as a
+// template parameter (a branch there costs what the hint gives).
+template <typename F>
+__device__ __forceinline__ void with_streaming(const PassArgs &a, F &&f) {
+    if (a.streaming) f(std::true_type{});
+    else f(std::false_type{});
+}
 
 // The (segment, row, tile) a block works on: segments are operands (forward
 // launches) or products (the others), each `rows x tiles` blocks in turn.
@@ -548,7 +574,7 @@ __device__ __forceinline__ void col_fwd_prime_late(double *v, double *lds, const
 // twiddles) is issued before the first store and both primes' results are
 // stored at the end: loads and stores share one in-order counter, so a
 // load issued after a store also waits for the store.
-template <int M, bool PAIR>
+template <int M, bool PAIR, bool NT>
 __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_fwd_kernel(PassArgs a, int level) {
     using CP = ColPair<M, PAIR>;
     __shared__ double lds_tiles[CP::kLdsWords];
@@ -561,25 +587,25 @@ __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_fwd_kern
     double *T1 = T0 + o.pstride;
     double v0[16], v1[16];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v0[u] = T0[ct.poff(u)];
+    for (int u = 0; u < 16; ++u) v0[u] = plane_get<NT>(T0 + ct.poff(u));
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v1[u] = T1[ct.poff(u)];
+    for (int u = 0; u < 16; ++u) v1[u] = plane_get<NT>(T1 + ct.poff(u));
     const ColTw tw0 = col_tw_load<M>(a.tables, ct.cg, ct.B0, false);
     const ColTw tw1 = col_tw_load<M>(a.tables + kPrimeTable, ct.cg, ct.B0, false);
     col_fwd_prime<M, 0, true>(v0, lds, ct, a.tables, tw0);
     col_fwd_prime<M, 1, false>(v1, lds, ct, a.tables, tw1);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) T0[ct.plast(k)] = v0[k];
+    for (int k = 0; k < 16; ++k) plane_put<NT>(T0 + ct.plast(k), v0[k]);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) T1[ct.plast(k)] = v1[k];
+    for (int k = 0; k < 16; ++k) plane_put<NT>(T1 + ct.plast(k), v1[k]);
 }
 
 // Stores last-step values (TRUNC: those of rows below rows_end).
-template <int M, bool TRUNC>
+template <int M, bool TRUNC, bool NT>
 __device__ __forceinline__ void col_store_last(double *T, const double *v, const ColThread<M> &ct, uint32_t rows_end) {
     if constexpr (!TRUNC) {
 #pragma unroll
-        for (int k = 0; k < 16; ++k) T[ct.plast(k)] = v[k];
+        for (int k = 0; k < 16; ++k) plane_put<NT>(T + ct.plast(k), v[k]);
     } else {
         constexpr int R = 1 << col_last_lr(M);
 #pragma unroll
@@ -590,20 +616,20 @@ __device__ __forceinline__ void col_store_last(double *T, const double *v, const
             for (int j = 0; j < R; ++j) __asm__ volatile("" : : "v"(v[u * R + j]));
             if (ct.part_used(u, rows_end)) {
 #pragma unroll
-                for (int j = 0; j < R; ++j) T[ct.plast(u * R + j)] = v[u * R + j];
+                for (int j = 0; j < R; ++j) plane_put<NT>(T + ct.plast(u * R + j), v[u * R + j]);
             }
         }
     }
 }
 // Loads them (zero where TRUNC leaves them out).
-template <int M, bool TRUNC>
+template <int M, bool TRUNC, bool NT>
 __device__ __forceinline__ void col_load_last(double *v, const double *T, const ColThread<M> &ct, uint32_t rows_end) {
     constexpr int R = 1 << col_last_lr(M);
 #pragma unroll
     for (int u = 0; u < 16 / R; ++u) {
         if (!TRUNC || ct.part_used(u, rows_end)) {
 #pragma unroll
-            for (int j = 0; j < R; ++j) v[u * R + j] = T[ct.plast(u * R + j)];
+            for (int j = 0; j < R; ++j) v[u * R + j] = plane_get<NT>(T + ct.plast(u * R + j));
         } else {
 #pragma unroll
             for (int j = 0; j < R; ++j) v[u * R + j] = 0.0;
@@ -704,12 +730,13 @@ struct Digits {
 // prime converts.  Each prime's column twiddles are loaded after its transform
 // (fewer registers held through it); 110-122 VGPRs and a 34.8 KB tile give
 // four waves per SIMD.  Bound by the latency of transform -> scattered stores:
-// 3.2 TB/s at 10^9 digits (144 ms per step).  Slower there: persistent blocks
+// 3.4 TB/s at 10^9 digits (136 ms per step; the following before
+// plane_put, against 144).  Slower there: persistent blocks
 // that load the next tile's words before the second prime's stores (169 ms, no
 // spills), the second prime's tables loaded before the first prime's stores
 // (167 ms), both primes stored at the end (244 ms, spills).  TRUNC: only the
 // rows of the transforms' first parts are stored.
-template <int M, bool PAIR, bool TRUNC>
+template <int M, bool PAIR, bool TRUNC, bool NT>
 __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) __attribute__((amdgpu_waves_per_eu(4)))
 ntt_col_fwd_limbs_kernel(PassArgs a) {
     using CP = ColPair<M, PAIR>;
@@ -732,7 +759,7 @@ ntt_col_fwd_limbs_kernel(PassArgs a) {
     for (int u = 0; u < 16; ++u) v[u] = d.value(u);
     col_fwd_prime_late<M, 0>(v, lds, ct, a.tables);
     memory_first_begin();
-    col_store_last<M, TRUNC>(T0, v, ct, rows_end);
+    col_store_last<M, TRUNC, NT>(T0, v, ct, rows_end);
     memory_first_end();
     __syncthreads();
     d.opaque();  // converted again, not kept as doubles
@@ -740,7 +767,7 @@ ntt_col_fwd_limbs_kernel(PassArgs a) {
     for (int u = 0; u < 16; ++u) v[u] = d.value(u);
     col_fwd_prime_late<M, 1>(v, lds, ct, a.tables);
     memory_first_begin();
-    col_store_last<M, TRUNC>(T1, v, ct, rows_end);
+    col_store_last<M, TRUNC, NT>(T1, v, ct, rows_end);
     memory_first_end();
 }
 
@@ -806,8 +833,10 @@ __global__ void __launch_bounds__(256) ntt_row_fused_kernel(PassArgs a) {
             memory_first_end();
         }
         inv_dft<M, false>(v, lds, tab, P, m);
+        with_streaming(a, [&](auto nt) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) TA[j * kJ] = v[j];
+            for (int j = 0; j < 16; ++j) plane_put<nt.value>(TA + j * kJ, v[j]);
+        });
         __syncthreads();
     }
 }
@@ -862,8 +891,10 @@ __global__ void __launch_bounds__(256) ntt_row_pair_kernel(PassArgs a, uint32_t 
 #pragma unroll
             for (int j = 0; j < 16; ++j) v[j] = mulp(rb[j], v[j], m);
             inv_dft<M, false>(v, lds, tabq, P, m);
+            with_streaming(a, [&](auto nt) {
 #pragma unroll
-            for (int j = 0; j < 16; ++j) TA[j * kJ] = v[j];
+                for (int j = 0; j < 16; ++j) plane_put<nt.value>(TA + j * kJ, v[j]);
+            });
         }
         __syncthreads();
     }
@@ -885,19 +916,19 @@ __device__ __forceinline__ void col_inv_prime(double *v, double *lds, const ColT
 // Loads both primes' values of a column tile (TRUNC: its rows below rows_end)
 // and their inverse column twiddle table entries (every load before any
 // store).
-template <int M, bool TRUNC = false>
+template <int M, bool TRUNC, bool NT>
 __device__ __forceinline__ void col_inv_load(double *v0, double *v1, ColTw &tw0, ColTw &tw1, const PassArgs &a,
                                              const ColThread<M> &ct, const double *T0, const double *T1,
                                              uint32_t rows_end = 1u << M) {
-    col_load_last<M, TRUNC>(v0, T0, ct, rows_end);
-    col_load_last<M, TRUNC>(v1, T1, ct, rows_end);
+    col_load_last<M, TRUNC, NT>(v0, T0, ct, rows_end);
+    col_load_last<M, TRUNC, NT>(v1, T1, ct, rows_end);
     tw0 = col_tw_load<M>(a.tables, ct.cg, ct.B0, true);
     tw1 = col_tw_load<M>(a.tables + kPrimeTable, ct.cg, ct.B0, true);
 }
 
 // Inverse column level above the first: both primes through one tile,
 // stored together at the end.
-template <int M, bool PAIR>
+template <int M, bool PAIR, bool NT>
 __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_inv_kernel(PassArgs a, int level) {
     using CP = ColPair<M, PAIR>;
     __shared__ double lds_tiles[CP::kLdsWords];
@@ -910,14 +941,14 @@ __global__ void __launch_bounds__((ColPair<M, PAIR>::kThreads)) ntt_col_inv_kern
     double *T1 = T0 + oa.pstride;
     double v0[16], v1[16];
     ColTw tw0, tw1;
-    col_inv_load<M>(v0, v1, tw0, tw1, a, ct, T0, T1);
+    col_inv_load<M, false, NT>(v0, v1, tw0, tw1, a, ct, T0, T1);
     col_inv_prime<M, 0>(v0, lds, ct, a.tables, tw0);
     __syncthreads();
     col_inv_prime<M, 1>(v1, lds, ct, a.tables, tw1);
 #pragma unroll
-    for (int u = 0; u < 16; ++u) T0[ct.poff(u)] = v0[u];
+    for (int u = 0; u < 16; ++u) plane_put<NT>(T0 + ct.poff(u), v0[u]);
 #pragma unroll
-    for (int u = 0; u < 16; ++u) T1[ct.poff(u)] = v1[u];
+    for (int u = 0; u < 16; ++u) plane_put<NT>(T1 + ct.poff(u), v1[u]);
 }
 
 // x of lane - D inside the lane's row of 16 lanes (DPP row_shr; 0 where that
@@ -1021,7 +1052,9 @@ ntt_col_inv_limbs_kernel(PassArgs a) {
     double v0[16], v1[16];
     ColTw tw0, tw1;
     const uint32_t tau = TRUNC ? prod_tau(a, prod) : kTauMax;
-    col_inv_load<M, TRUNC>(v0, v1, tw0, tw1, a, ct, T0, T0 + oa.pstride, tau_rows(M, tau));
+    with_streaming(a, [&](auto nt) {
+        col_inv_load<M, TRUNC, nt.value>(v0, v1, tw0, tw1, a, ct, T0, T0 + oa.pstride, tau_rows(M, tau));
+    });
     // 1/K rides on the column twiddles (the inverse transform is linear):
     // one product per prime instead of one per value; the last inverse step
     // re-centres its outputs (|v| < p/2 + p/1024) for the recombination
@@ -1661,18 +1694,18 @@ NttShape shape_for(uint32_t L1, uint32_t L2, uint32_t Lb) {
 std::atomic<uint32_t> g_pair_mask{kPairMaskDefault};
 std::atomic<int> g_xcd_log2{kXcdChunkLog2};
 
-// Calls f(PAIR, TRUNC) as std::integral_constants: PAIR = pair where a level of
+// Calls f(PAIR, FLAG) as std::integral_constants: PAIR = pair where a level of
 // 2^M points can pair its tiles, false otherwise.
 template <int M, typename F>
-void with_flags(bool pair, bool trunc, F &&f) {
+void with_flags(bool pair, bool flag, F &&f) {
     if constexpr (col_pair_log2(M) > 0) {
         if (pair) {
-            if (trunc) f(std::true_type{}, std::true_type{});
+            if (flag) f(std::true_type{}, std::true_type{});
             else f(std::true_type{}, std::false_type{});
             return;
         }
     }
-    if (trunc) f(std::false_type{}, std::true_type{});
+    if (flag) f(std::false_type{}, std::true_type{});
     else f(std::false_type{}, std::false_type{});
 }
 
@@ -1990,6 +2023,12 @@ bool run_thin(const NttJob &j, const JobShape &sh) {
     return ((uint64_t)sh.rows * j.n_prods << j.k) <= 1ull << kThinMaxTotalLog2;
 }
 
+// Planes above this size go past the caches (plane_put): 256 MB is the size of
+// the last one.  96 products of 24007 x 20011 limbs (126 MB) with the hint at
+// any size 142 -> 152 us; 1 of 7000000 x 7000000 (380 MB) 642 -> 638, of
+// 10000000 x 10000000 1160 -> 1108.
+constexpr uint64_t kStreamBytes = 256ull << 20;
+
 hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, const NTTPrecomputedTables &tables,
                    hipStream_t stream) {
     if (!job_ok(j)) return hipErrorInvalidValue;
@@ -2032,6 +2071,9 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
         a.row_tau = 10 * parts <= 9 * (uint64_t)kTauMax * sh.rows;
         if (!a.row_tau) tau = kTauMax;
     }
+    uint64_t plane_bytes = 0;
+    for (uint32_t o = 0; o < j.n_ops; ++o) plane_bytes += 2 * sizeof(double) * l.plane_elems[o] / kTauMax * tau;
+    a.streaming = plane_bytes > kStreamBytes;
     a.tau = tau;
     a.tau_tiles = tau_tiles(tiles, tau);
     const bool trunc = a.row_tau || tau < kTauMax;
@@ -2107,8 +2149,10 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
                     with_flags<M>((pair_mask >> kPairFwdLimbs) & 1u, trunc, [&](auto pc, auto tc) {
                         constexpr bool kPair = decltype(pc)::value, kTrunc = decltype(tc)::value;
                         constexpr int pl = ColPair<M, kPair>::kLog2;
-                        hipLaunchKernelGGL((ntt_col_fwd_limbs_kernel<M, kPair, kTrunc>), blocks(fwd_rows, tiles, pl),
-                                           dim3(256 << pl), 0, stream, args(tiles, pl));
+                        const auto kernel = a.streaming ? ntt_col_fwd_limbs_kernel<M, kPair, kTrunc, true>
+                                                        : ntt_col_fwd_limbs_kernel<M, kPair, kTrunc, false>;
+                        hipLaunchKernelGGL(kernel, blocks(fwd_rows, tiles, pl), dim3(256 << pl), 0, stream,
+                                           args(tiles, pl));
                     });
                 });
             }));
@@ -2116,10 +2160,10 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
                 GPUPI_RETURN_IF(timed(kColFwd, k, 2 * fwd_tb, stream, [&] {
                     dispatch_m<kColLo, kColHi>(p.log2M[1], [&](auto mc) {
                         constexpr int M = decltype(mc)::value;
-                        with_flags<M>((pair_mask >> kPairFwd) & 1u, false, [&](auto pc, auto) {
+                        with_flags<M>((pair_mask >> kPairFwd) & 1u, a.streaming, [&](auto pc, auto nt) {
                             constexpr int pl = ColPair<M, decltype(pc)::value>::kLog2;
-                            hipLaunchKernelGGL((ntt_col_fwd_kernel<M, decltype(pc)::value>), blocks(fwd_rows, deep, pl),
-                                               dim3(256 << pl), 0, stream, args(deep, pl), 1);
+                            hipLaunchKernelGGL((ntt_col_fwd_kernel<M, decltype(pc)::value, decltype(nt)::value>),
+                                               blocks(fwd_rows, deep, pl), dim3(256 << pl), 0, stream, args(deep, pl), 1);
                         });
                     });
                 }));
@@ -2164,10 +2208,10 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
             GPUPI_RETURN_IF(timed(kColInv, k, 2 * prod_tb, stream, [&] {
                 dispatch_m<kColLo, kColHi>(p.log2M[1], [&](auto mc) {
                     constexpr int M = decltype(mc)::value;
-                    with_flags<M>((pair_mask >> kPairInv) & 1u, false, [&](auto pc, auto) {
+                    with_flags<M>((pair_mask >> kPairInv) & 1u, a.streaming, [&](auto pc, auto nt) {
                         constexpr int pl = ColPair<M, decltype(pc)::value>::kLog2;
-                        hipLaunchKernelGGL((ntt_col_inv_kernel<M, decltype(pc)::value>), blocks(prod_rows, deep, pl),
-                                           dim3(256 << pl), 0, stream, args(deep, pl), 1);
+                        hipLaunchKernelGGL((ntt_col_inv_kernel<M, decltype(pc)::value, decltype(nt)::value>),
+                                           blocks(prod_rows, deep, pl), dim3(256 << pl), 0, stream, args(deep, pl), 1);
                     });
                 });
             }));
