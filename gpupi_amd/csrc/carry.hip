@@ -345,12 +345,15 @@ __device__ __forceinline__ RaggedAssembly assembly_of(const RaggedAssembly *as, 
 // Ragged assembly (RaggedAssembly): one wave per 1024-limb chunk, the
 // layout of addsub_vec_kernel (flags per chunk for the fixup).  Limb x of C
 // is piece i's staged word x - i s plus, when x - i s < S, piece i - 1's
-// word x - i s + s, i = min(x / s, m - 1).
-__global__ void __launch_bounds__(256) ragged_assemble_kernel(const uint32_t *staging, uint64_t K,
+// word x - i s + s, i = min(x / s, m - 1).  Bound by HBM; four limbs per lane
+// and access where they share both pieces (256 ragged pairs with it and the
+// copies of whole products: 30.9 -> 29.6 ms; a division and two loads per limb
+// took 2.3 ms of them).
+__global__ void __launch_bounds__(256) ragged_assemble_kernel(const uint32_t *staging, uint64_t stride,
                                                               const RaggedAssembly *as, uint32_t n,
                                                               uint32_t chunks, uint8_t *flags) {
     constexpr int kSeg = 4;  // 4 x 256 limbs per wave
-    const uint32_t g = blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
+    const uint32_t g = blockIdx.x * (256 / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (g >= chunks) return;
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const RaggedAssembly a = assembly_of(as, n, g);
@@ -361,19 +364,35 @@ __global__ void __launch_bounds__(256) ragged_assemble_kernel(const uint32_t *st
     for (int sg = 0; sg < kSeg; ++sg) {
         const uint32_t j0 = chunk * kAssembleChunk + (uint32_t)sg * (4 * kWave) + 4 * lane;
         uint32_t d[4], gen[4];
+        // the lane's four limbs lie in one piece, and all or none of them in
+        // the overlap with the piece below, but at the pieces' ends
+        uint32_t i0, off0;
+        bool below0;
+        assembly_source(a, j0, &i0, &off0, &below0);
+        if (j0 + 4 <= a.c && (i0 + 1 == a.m || off0 + 4 <= a.s) && (!below0 || off0 + 4 <= a.S)) {
+            const Quad u = *reinterpret_cast<const Quad *>(staging + (size_t)(a.row0 + i0) * stride + off0);
+            Quad v{};
+            if (below0) v = *reinterpret_cast<const Quad *>(staging + (size_t)(a.row0 + i0 - 1) * stride + off0 + a.s);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const uint32_t x = j0 + t;
-            d[t] = 0;
-            gen[t] = 0;
-            if (x < a.c) {
-                uint32_t i, off;
-                bool below;
-                assembly_source(a, x, &i, &off, &below);
-                const uint32_t u = staging[(size_t)(a.row0 + i) * K + off];
-                const uint32_t v = below ? staging[(size_t)(a.row0 + i - 1) * K + off + a.s] : 0u;
-                d[t] = u + v;
-                gen[t] = d[t] < u ? 1u : 0u;
+            for (int t = 0; t < 4; ++t) {
+                d[t] = u.w[t] + v.w[t];
+                gen[t] = d[t] < u.w[t] ? 1u : 0u;
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const uint32_t x = j0 + t;
+                d[t] = 0;
+                gen[t] = 0;
+                if (x < a.c) {
+                    uint32_t i, off;
+                    bool below;
+                    assembly_source(a, x, &i, &off, &below);
+                    const uint32_t u = staging[(size_t)(a.row0 + i) * stride + off];
+                    const uint32_t v = below ? staging[(size_t)(a.row0 + i - 1) * stride + off + a.s] : 0u;
+                    d[t] = u + v;
+                    gen[t] = d[t] < u ? 1u : 0u;
+                }
             }
         }
         // the lane's four limbs for a carry-in of zero
@@ -390,11 +409,18 @@ __global__ void __launch_bounds__(256) ragged_assemble_kernel(const uint32_t *st
         uint32_t cout;
         const uint64_t cm = resolve_carries(G, P, cin, &cout);
         uint32_t ci = (uint32_t)(cm >> lane) & 1u;
+        Quad q;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const uint32_t v = r[t] + ci;
+            q.w[t] = r[t] + ci;
             ci = ci & (r[t] == 0xffffffffu ? 1u : 0u);
-            if (j0 + t < a.c) a.C[j0 + t] = v;
+        }
+        if (j0 + 4 <= a.c) {
+            *reinterpret_cast<Quad *>(a.C + j0) = q;
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                if (j0 + t < a.c) a.C[j0 + t] = q.w[t];
         }
         all_prop = all_prop && (P == ~0ull);
         cin = cout;
@@ -407,7 +433,7 @@ __global__ void __launch_bounds__(256) ragged_assemble_kernel(const uint32_t *st
 // over ragged rows).
 __global__ void __launch_bounds__(256) ragged_assembly_fixup_kernel(const RaggedAssembly *as, uint32_t n,
                                                                     uint32_t chunks, const uint8_t *flags) {
-    const uint32_t g = blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
+    const uint32_t g = blockIdx.x * (256 / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (g >= chunks) return;
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const RaggedAssembly a = assembly_of(as, n, g);

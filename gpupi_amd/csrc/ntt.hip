@@ -1816,7 +1816,12 @@ __global__ void __launch_bounds__(256) ragged_copy_kernel(const uint32_t *stagin
     if (it.C == nullptr) return;
     const uint32_t Lc = it.L_a + it.L_b;
     const uint32_t *src = staging + (size_t)row * stride;
-    for (uint32_t i = slice * 1024u + threadIdx.x; i < Lc && i < (slice + 1) * 1024u; i += 256u) it.C[i] = src[i];
+    const uint32_t i = slice * 1024u + 4u * threadIdx.x;
+    if (i + 4u <= Lc) {
+        *reinterpret_cast<Quad *>(it.C + i) = *reinterpret_cast<const Quad *>(src + i);
+    } else {
+        for (uint32_t t = i; t < Lc; ++t) it.C[t] = src[t];
+    }
 }
 
 // One NTT launch sequence over products of one transform size 2^k: up to
