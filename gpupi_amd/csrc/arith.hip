@@ -523,14 +523,13 @@ hipError_t batch_mp_mul_shared(BatchMPContext *ctx, BatchMPArray A1, BatchMPArra
 }
 
 namespace {
-// The launches of a ragged call that take descriptors: the matrix-core
-// products `small`; and the NTT's: rows of whole
-// products, and the pieces of split ones (plans[q].m >= 2) with their assemblies, grouped by
+// The NTT launches of a ragged call: rows of whole products, and the
+// pieces of split ones (plans[q].m >= 2) with their assemblies, grouped by
 // transform size into launches filled to ntt_ragged_max_rows rows (a
 // product's pieces stay in one launch), each with the set of distinct B
 // operands its rows use.
-hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const std::vector<uint32_t> &small,
-                           const std::vector<uint32_t> &big, const std::vector<SplitPlan> &plans) {
+hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const std::vector<uint32_t> &big,
+                           const std::vector<SplitPlan> &plans) {
     // groups of rows: a whole product (one row) or a split one (its pieces)
     struct Group {
         gpupi::NttShape shape;
@@ -615,19 +614,6 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
         launches.push_back(l);
         g0 = g1;
     }
-    // the small products after the NTT rows: up to one per CU in one launch
-    // (the blocks run side by side whatever their size), more by the tile
-    // groups they need
-    std::vector<std::pair<uint32_t, uint32_t>> classes;  // (tile groups, item)
-    for (uint32_t i : small) classes.emplace_back(gpupi::mul_mfma_groups(items[i].L_a, items[i].L_b), i);
-    std::sort(classes.begin(), classes.end());
-    if (classes.size() <= 256)
-        for (auto &c : classes) c.first = classes.back().first;
-    const size_t small_r0 = host_rows.size();
-    for (const auto &c : classes) {
-        const GpupiMulItem &it = items[c.second];
-        host_rows.push_back(gpupi::RaggedRow{it.A, it.B, it.C, it.L_a, it.L_b, 0, 0});
-    }
     // the descriptors at the head of the workspace, then the largest
     // launch's NTT scratch
     const size_t row_bytes = (host_rows.size() * sizeof(gpupi::RaggedRow) + 255) & ~(size_t)255;
@@ -641,18 +627,12 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
     char *ntt_ws = ws + row_bytes + b_bytes + a_bytes;
     GPUPI_RETURN_IF(hipMemcpyAsync(d_rows, host_rows.data(), host_rows.size() * sizeof(gpupi::RaggedRow),
                                    hipMemcpyHostToDevice, ctx->stream));
-    if (!host_bset.empty())
-        GPUPI_RETURN_IF(hipMemcpyAsync(d_bset, host_bset.data(), host_bset.size() * sizeof(gpupi::RaggedB),
-                                       hipMemcpyHostToDevice, ctx->stream));
+    GPUPI_RETURN_IF(hipMemcpyAsync(d_bset, host_bset.data(), host_bset.size() * sizeof(gpupi::RaggedB),
+                                   hipMemcpyHostToDevice, ctx->stream));
     if (!host_asms.empty())
         GPUPI_RETURN_IF(hipMemcpyAsync(d_asms, host_asms.data(), host_asms.size() * sizeof(gpupi::RaggedAssembly),
                                        hipMemcpyHostToDevice, ctx->stream));
     GPUPI_RETURN_IF(hipStreamSynchronize(ctx->stream));
-    for (size_t c0 = 0, c1 = 0; c0 < classes.size(); c0 = c1) {
-        while (c1 < classes.size() && classes[c1].first == classes[c0].first) ++c1;
-        GPUPI_RETURN_IF(gpupi::launch_mul_mfma_ragged(d_rows + small_r0 + c0, (uint32_t)(c1 - c0), classes[c0].first,
-                                                      ctx->stream));
-    }
     for (const Launch &l : launches)
         GPUPI_RETURN_IF(gpupi::launch_mul_ntt_ragged(
             d_rows + l.r0, host_rows.data() + l.r0, (uint32_t)l.n, d_bset + l.b0, host_bset.data() + l.b0,
@@ -660,10 +640,8 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
             ntt_bytes, ctx->ntt_tables, ctx->stream));
     return hipSuccess;
 }
-}  // namespace
 
-hipError_t gpupi_mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint32_t count) {
-    if (ctx == nullptr || (count > 0 && items == nullptr)) return hipErrorInvalidValue;
+hipError_t mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint32_t count) {
     // validate everything before launching anything
     std::vector<uint32_t> big;  // NTT products
     for (uint32_t i = 0; i < count; ++i) {
@@ -682,29 +660,28 @@ hipError_t gpupi_mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint
             big.push_back(i);
         }
     }
-    // small products: those the matrix cores take share a few launches where
-    // there are enough of them to pay for their descriptors' upload (124 pairs
-    // of 2^7..2^11 limbs: 98 us, 1021 us with a launch each)
-    std::vector<uint32_t> small, alone;
+    // small products: those the matrix cores take share a few launches
+    std::vector<gpupi::MfmaRow> small;
     for (uint32_t i = 0; i < count; ++i) {
         const GpupiMulItem &it = items[i];
         const uint64_t total = (uint64_t)it.L_a + it.L_b;
         if (total == 0) continue;
         const bool empty = it.L_a == 0 || it.L_b == 0;
         if (!empty && !((int64_t)total < ctx->ntt_min_limbs && gpupi::mul_naive_supports(it.L_a, it.L_b))) continue;
-        if (!empty && total <= gpupi::kMulMfmaMaxTotal) small.push_back(i);
-        else alone.push_back(i);
+        if (!empty && total <= gpupi::kMulMfmaMaxTotal)
+            small.push_back(gpupi::MfmaRow{it.A, it.B, it.C, it.L_a, it.L_b});
+        else
+            GPUPI_RETURN_IF(gpupi::launch_mul_naive(it.A, it.B, it.C, 1, it.L_a, it.L_b, it.L_a, it.L_b,
+                                                    (uint32_t)total, ctx->stream));
     }
-    if (small.size() < 4 && big.empty()) {
-        alone.insert(alone.end(), small.begin(), small.end());
-        small.clear();
+    if (small.size() == 1) {
+        const gpupi::MfmaRow &r = small[0];
+        GPUPI_RETURN_IF(gpupi::launch_mul_naive(r.A, r.B, r.C, 1, r.L_a, r.L_b, r.L_a, r.L_b, r.L_a + r.L_b,
+                                                ctx->stream));
+    } else {
+        GPUPI_RETURN_IF(gpupi::launch_mul_mfma_ragged(small, *ctx->cache, ctx->stream));
     }
-    for (uint32_t i : alone) {
-        const GpupiMulItem &it = items[i];
-        GPUPI_RETURN_IF(gpupi::launch_mul_naive(it.A, it.B, it.C, 1, it.L_a, it.L_b, it.L_a, it.L_b,
-                                                it.L_a + it.L_b, ctx->stream));
-    }
-    if (big.empty() && small.empty()) return hipSuccess;
+    if (big.empty()) return hipSuccess;
     // NTT rows, one launch sequence per transform size (and row chunk):
     // whole products, and in the batched form the pieces of the products
     // that gain from running in pieces (split_plan), which share the
@@ -716,7 +693,17 @@ hipError_t gpupi_mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint
             const GpupiMulItem &it = items[big[q]];
             plans[q] = split_plan(std::max(it.L_a, it.L_b), std::min(it.L_a, it.L_b));
         }
-    return ragged_launches(ctx, items, small, big, plans);
+    return ragged_launches(ctx, items, big, plans);
+}
+}  // namespace
+
+hipError_t gpupi_mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint32_t count) {
+    if (ctx == nullptr || (count > 0 && items == nullptr)) return hipErrorInvalidValue;
+    try {
+        return mul_ragged(ctx, items, count);
+    } catch (const std::bad_alloc &) {
+        return hipErrorOutOfMemory;  // no exception leaves a C entry
+    }
 }
 
 hipError_t batch_mp_mul_small(BatchMPContext *ctx, BatchMPArray A, uint32_t B, BatchMPArray C) {

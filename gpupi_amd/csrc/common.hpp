@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include <map>
+#include <vector>
 
 #include "batch_arith.h"
 #include "batch_kernels.h"
@@ -95,10 +96,16 @@ hipError_t launch_mul_naive(const uint32_t *A, const uint32_t *B, uint32_t *C, u
 constexpr uint32_t kMulMfmaMaxTotal = 4088;
 hipError_t launch_mul_mfma(const uint32_t *A, const uint32_t *B, uint32_t *C, uint32_t N, uint32_t LA, uint32_t LB,
                            uint32_t sA, uint32_t sB, uint32_t sC, hipStream_t stream);
-// Such products of mixed lengths, one per row (device descriptors), in W >=
-// mul_mfma_groups(L_a, L_b) tile groups (1..4) each.
-uint32_t mul_mfma_groups(uint32_t L_a, uint32_t L_b);
-hipError_t launch_mul_mfma_ragged(const RaggedRow *rows, uint32_t N, uint32_t W, hipStream_t stream);
+// Such products of mixed lengths, several to a launch.  Up to about a thousand
+// of them, or any number under capture, are launches only; more take a block of
+// the cache for their descriptors and wait for its upload.
+struct MfmaRow {
+    const uint32_t *A, *B;
+    uint32_t *C;
+    uint32_t L_a, L_b;
+};
+class BlockCache;
+hipError_t launch_mul_mfma_ragged(const std::vector<MfmaRow> &products, BlockCache &cache, hipStream_t stream);
 bool mul_naive_supports(uint32_t L_a, uint32_t L_b);
 
 hipError_t launch_mul_ntt(const uint32_t *A, const uint32_t *B, uint32_t *C, void *workspace,

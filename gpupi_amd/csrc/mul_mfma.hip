@@ -34,7 +34,9 @@
 // limbs 277 against 300 us, one row 17 against 27 us).
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <utility>
+#include <vector>
 
 #include "common.hpp"
 
@@ -63,8 +65,51 @@ struct MfmaArgs {
     uint32_t LA, LB, sA, sB, sC;
     uint32_t W, M, E, na, nb, i0_end, m_thr;
     uint32_t a_words, b_lead, b_half, lds_words;  // LDS words: a, zeros below b and a half of it, all but the column sums
-    const RaggedRow *rows;                        // ragged launches: a product per row
 };
+
+// A ragged launch carries its products in the kernel's arguments: no device
+// memory to fill, nothing to wait for, and a captured launch holds its own
+// copy.  A product is three words, its limb addresses (multiples of four) over
+// the lengths, so that as many as possible go into the 4 KB that a launch's
+// arguments may take: launches follow each other, and with rows of 32 bytes,
+// 96 to a launch, 600 products of 2^9..2^11 limbs took 156 us instead of 87.
+// Above six launches the same rows go into a block of device memory, one
+// launch per number of tile groups (600 products of 2^9..2^11 limbs 87 us from
+// arguments against 98 from memory, 1500 of them 186 against 155, 12000 2042
+// against 879).
+constexpr uint32_t kArgRows = 168, kArgRowsMost = 6 * kArgRows;
+constexpr int kLengthBits = 12;
+struct ArgRow {
+    uint64_t a, b, c;
+};
+static_assert(kMulMfmaMaxTotal <= 1u << kLengthBits, "a length fits its bits");
+inline uint64_t arg_word(const uint32_t *p, uint32_t length) { return (uint64_t)(uintptr_t)p << (kLengthBits - 2) | length; }
+__device__ __forceinline__ uint32_t *arg_limbs(uint64_t w) { return reinterpret_cast<uint32_t *>(w >> kLengthBits << 2); }
+__device__ __forceinline__ uint32_t arg_length(uint64_t w) { return (uint32_t)w & ((1u << kLengthBits) - 1u); }
+struct MfmaRaggedArgs {
+    uint32_t W;
+    ArgRow rows[kArgRows];
+};
+static_assert(sizeof(MfmaRaggedArgs) <= 4096, "a launch's arguments");
+struct MfmaListArgs {
+    uint32_t W;
+    const ArgRow *rows;
+};
+
+// What of MfmaArgs a ragged launch's W decides: LDS for the longest operands
+// of any of its shapes, three blocks of a and five of b.
+__host__ __device__ inline MfmaArgs ragged_base(uint32_t W) {
+    MfmaArgs s{};
+    s.W = W;
+    s.a_words = 256u * W * 3u + 20u;
+    s.b_lead = 4u * (32u * W - 1u);
+    s.b_half = 4u * 32u * W * 5u + s.b_lead;
+    s.lds_words = s.a_words + 2 * s.b_half + 2 * kMaxTiles;
+    return s;
+}
+__device__ inline MfmaArgs base_of(const MfmaArgs &a) { return a; }
+__device__ inline MfmaArgs base_of(const MfmaRaggedArgs &a) { return ragged_base(a.W); }
+__device__ inline MfmaArgs base_of(const MfmaListArgs &a) { return ragged_base(a.W); }
 
 MfmaArgs shape_of(uint32_t LA, uint32_t LB, uint32_t W) {
     MfmaArgs s{};
@@ -265,7 +310,7 @@ __device__ __forceinline__ void tile_store(uint32_t *c, uint32_t l, uint32_t Lc,
     }
 }
 
-// RAGGED (S > 1, G = 5): block i multiplies row i's operands, of any lengths
+// RAGGED (its own ARGS; S > 1, G = 5): block i multiplies row i's operands, of any lengths
 // that W takes; M and E are one of three shapes with M + E - 1 = 5 chosen per
 // block, and fragments a product does not reach are zero.
 // One product per block, W tile groups (WT: W where it is known, else 0).
@@ -273,10 +318,12 @@ __device__ __forceinline__ void tile_store(uint32_t *c, uint32_t l, uint32_t Lc,
 // group, part ks of them taking the steps ks, ks + S, ...; the parts' column
 // sums meet in LDS and each wave finishes a tile or two.
 constexpr int mfma_waves(int g) { return g <= 1 ? 8 : g <= 2 ? 6 : g <= 5 ? 4 : 2; }
-template <int M, int E, int WT, int S, bool RAGGED = false>
+template <int M, int E, int WT, int S, typename ARGS = MfmaArgs>
 __global__ void __launch_bounds__(S == 1 ? 256 : 1024) __attribute__((amdgpu_waves_per_eu(mfma_waves(M + E - 1))))
-mul_mfma_kernel(MfmaArgs a) {
+mul_mfma_kernel(ARGS args) {
+    constexpr bool RAGGED = !std::is_same_v<ARGS, MfmaArgs>;
     constexpr int G = M + E - 1;
+    MfmaArgs a = base_of(args);
     extern __shared__ __align__(16) uint32_t lds[];
     const uint32_t lane = threadIdx.x & (kWave - 1u);
     const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -285,13 +332,12 @@ mul_mfma_kernel(MfmaArgs a) {
     const uint32_t ks = S > 1 ? wid / W : 0u, tw = wid - ks * W;
     const size_t row = RAGGED ? 0 : blockIdx.x;
     if constexpr (RAGGED) {
-        const RaggedRow rr = a.rows[blockIdx.x];
-        const bool swap = rr.L_a > rr.L_b;
-        a.A = swap ? rr.B : rr.A;
-        a.B = swap ? rr.A : rr.B;
-        a.C = rr.C;
-        a.LA = swap ? rr.L_b : rr.L_a;
-        a.LB = swap ? rr.L_a : rr.L_b;
+        const ArgRow rr = args.rows[blockIdx.x];
+        a.A = arg_limbs(rr.a);
+        a.B = arg_limbs(rr.b);
+        a.C = arg_limbs(rr.c);
+        a.LA = arg_length(rr.a);
+        a.LB = arg_length(rr.b);
         a.na = blocks_of(a.LA);
         a.nb = blocks_of(a.LB);
         a.i0_end = min(32u * W - 1u, a.na) + 1u;
@@ -455,7 +501,10 @@ bool each_kernel(F &&f) {
 }
 
 constexpr uint32_t kRaggedMaxW = 4;
-const MfmaKernel kRaggedKernel = mul_mfma_kernel<3, 3, 0, kParts, true>;
+template <typename ARGS>
+using RaggedKernel = void (*)(ARGS);
+const RaggedKernel<MfmaRaggedArgs> kRaggedKernel = mul_mfma_kernel<3, 3, 0, kParts, MfmaRaggedArgs>;
+const RaggedKernel<MfmaListArgs> kListKernel = mul_mfma_kernel<3, 3, 0, kParts, MfmaListArgs>;
 
 // The kernels of several parts may take more than 64 KB of LDS; the attribute
 // is a property of the current device, set once per device (serving threads
@@ -474,7 +523,8 @@ hipError_t allow_large_lds() {
         return err != hipSuccess;
     });
     GPUPI_RETURN_IF(err);
-    GPUPI_RETURN_IF(hipFuncSetAttribute((const void *)kRaggedKernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    for (const void *k : {(const void *)kRaggedKernel, (const void *)kListKernel})
+        GPUPI_RETURN_IF(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     g_lds_done |= bit;
     return hipSuccess;
 }
@@ -524,29 +574,73 @@ hipError_t launch_mul_mfma(const uint32_t *A, const uint32_t *B, uint32_t *C, ui
     return hipGetLastError();
 }
 
-uint32_t mul_mfma_groups(uint32_t L_a, uint32_t L_b) {
-    const uint32_t LA = std::min(L_a, L_b), LB = std::max(L_a, L_b);
+namespace {
+// Tile groups that a product of these lengths takes (LA <= LB) in a ragged launch.
+uint32_t ragged_groups(uint32_t LA, uint32_t LB) {
     uint32_t W = 1;
     MfmaArgs a = shape_of(LA, LB, W);
     while (a.M + a.E - 1 > kFewG) a = shape_of(LA, LB, ++W);
     return W;
 }
 
-hipError_t launch_mul_mfma_ragged(const RaggedRow *rows, uint32_t N, uint32_t W, hipStream_t stream) {
-    if (N == 0) return hipSuccess;
-    if (rows == nullptr || W < 1 || W > kRaggedMaxW || N > 0x7fffffffu) return hipErrorInvalidValue;
-    MfmaArgs a{};
-    a.rows = rows;
-    a.W = W;
-    // LDS for the longest operands of any shape: three blocks of a, five of b
-    a.a_words = 256u * W * 3u + 20u;
-    a.b_lead = 4u * (32u * W - 1u);
-    a.b_half = 4u * 32u * W * 5u + a.b_lead;
-    a.lds_words = a.a_words + 2 * a.b_half + 2 * kMaxTiles;
-    const size_t lds = (a.lds_words + W * kFewG * 1024u) * 4u;
+template <typename ARGS>
+hipError_t launch_ragged(RaggedKernel<ARGS> kernel, const ARGS &args, uint32_t n, hipStream_t stream) {
+    const size_t lds = (ragged_base(args.W).lds_words + args.W * kFewG * 1024u) * 4u;
     if (lds > 65536) GPUPI_RETURN_IF(allow_large_lds());
-    hipLaunchKernelGGL(kRaggedKernel, dim3(N), dim3(kWave * W * kParts), lds, stream, a);
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(kWave * args.W * kParts), lds, stream, args);
     return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_mul_mfma_ragged(const std::vector<MfmaRow> &products, BlockCache &cache, hipStream_t stream) {
+    const size_t n = products.size();
+    // in the order of their tile groups: a launch takes those of its last
+    size_t start[kRaggedMaxW + 2] = {};  // start[w]: products of fewer than w groups
+    std::vector<uint8_t> groups(n);
+    for (size_t i = 0; i < n; ++i) {
+        const MfmaRow &r = products[i];
+        if (r.L_a == 0 || r.L_b == 0 || (uint64_t)r.L_a + r.L_b > kMulMfmaMaxTotal) return hipErrorInvalidValue;
+        const uint32_t w = ragged_groups(std::min(r.L_a, r.L_b), std::max(r.L_a, r.L_b));
+        if (w > kRaggedMaxW) return hipErrorInvalidValue;
+        groups[i] = (uint8_t)w;
+        ++start[w + 1];
+    }
+    for (uint32_t w = 1; w < kRaggedMaxW + 2; ++w) start[w] += start[w - 1];
+    std::vector<ArgRow> rows(n);
+    {
+        size_t at[kRaggedMaxW + 1];
+        std::copy_n(start, kRaggedMaxW + 1, at);
+        for (size_t i = 0; i < n; ++i) {
+            const MfmaRow &r = products[i];
+            uint64_t a = arg_word(r.A, r.L_a), b = arg_word(r.B, r.L_b);
+            if (r.L_a > r.L_b) std::swap(a, b);
+            rows[at[groups[i]]++] = ArgRow{a, b, arg_word(r.C, 0)};
+        }
+    }
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (n > kArgRowsMost) GPUPI_RETURN_IF(hipStreamIsCapturing(stream, &capturing));
+    if (n > kArgRowsMost && capturing == hipStreamCaptureStatusNone) {
+        void *list = nullptr;
+        size_t got = 0;
+        GPUPI_RETURN_IF(cache.acquire(stream, n * sizeof(ArgRow), &list, &got));
+        const ArgRow *const d = static_cast<const ArgRow *>(list);
+        hipError_t err = hipMemcpyAsync(list, rows.data(), n * sizeof(ArgRow), hipMemcpyHostToDevice, stream);
+        if (err == hipSuccess) err = hipStreamSynchronize(stream);
+        for (uint32_t w = 1; w <= kRaggedMaxW && err == hipSuccess; ++w) {
+            const size_t m = start[w + 1] - start[w];
+            if (m > 0) err = launch_ragged(kListKernel, MfmaListArgs{w, d + start[w]}, (uint32_t)m, stream);
+        }
+        cache.give_back(list, got, stream);
+        return err;
+    }
+    for (size_t r0 = 0; r0 < n; r0 += kArgRows) {
+        const size_t m = std::min<size_t>(kArgRows, n - r0);
+        MfmaRaggedArgs a{};
+        for (a.W = 1; start[a.W + 1] < r0 + m;) ++a.W;
+        std::copy_n(rows.begin() + r0, m, a.rows);
+        GPUPI_RETURN_IF(launch_ragged(kRaggedKernel, a, (uint32_t)m, stream));
+    }
+    return hipSuccess;
 }
 
 }  // namespace gpupi

@@ -71,7 +71,13 @@ hipError_t batch_mp_mul(BatchMPContext *ctx, BatchMPArray A, BatchMPArray B, Bat
  * transform, and items passing the same B (pointer and length) share its
  * transform.  Descriptors are read from host memory before the call
  * returns.  No item's C may overlap any item's operands, and distinct
- * items' C must not overlap. */
+ * items' C must not overlap.  A call whose items all lie below the NTT's
+ * threshold leaves the context's workspace alone and can be captured into a
+ * graph; it only launches, unless it has over a thousand items (and is not
+ * being captured): then it waits for the upload of their descriptors.  Any
+ * other call uploads descriptors to the context's workspace (growing it if
+ * need be), waits for that upload, and reads them there until its kernels
+ * end. */
 typedef struct GpupiMulItem {
     const uint32_t *A;
     const uint32_t *B;

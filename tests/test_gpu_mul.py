@@ -5,6 +5,8 @@ Shapes: the schoolbook size classes, every NTT plan class (one tile; column +
 row; two columns + row), the 1024-limb boundary of the reference
 (batch_arith_test.cu:99-103), random shapes with random strides in the style
 of batch_mul_ntt_test.cu:531-556, and broadcast operands."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -883,3 +885,59 @@ def test_ragged_rows_of_several_sizes(ctx, seed, count, lo, hi):
     for a, b, bufs in pairs:
         got = bufs[2].download(np.uint32, count=len(a) + len(b) + 1)
         assert got[-1] == PAD and np.array_equal(got[:-1], oracle_mul(a.reshape(1, -1), b.reshape(1, -1))[0])
+
+
+@pytest.mark.parametrize("count", [2, 5, 168, 169, 400, 1200])
+def test_small_ragged_calls_only_launch(count):
+    """A ragged call of products below the NTT's threshold takes nothing of the
+    context's workspace, and a capture of it replays on new operands (around
+    the numbers of products that one launch's arguments hold, and above the
+    number from which an eager call uploads a list)."""
+    rng = np.random.default_rng(count)
+    hip = g.hip()
+    stream, graph, gexec = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    lengths = [(17, 17), (1, 4000), (2044, 2044)] + [tuple(int(2 ** u) for u in rng.uniform(0, 10.9, size=2))
+                                                     for _ in range(count)]
+    lengths = lengths[:count]
+    at, items = [], []
+    total = sum(2 * (a + b) for a, b in lengths)
+    buf = g.DeviceBuffer(4 * total)
+    word = 0
+    for a, b in lengths:
+        at.append(word)
+        items.append((buf.ptr + 4 * word, buf.ptr + 4 * (word + a), buf.ptr + 4 * (word + a + b), a, b))
+        word += 2 * (a + b)
+
+    def fill():
+        host = rng.integers(0, 1 << 32, size=total, dtype=np.uint32)
+        g.check(hip.hipMemcpy(buf.ptr, host.ctypes.data, host.nbytes, 1), "hipMemcpy")
+        return host
+
+    def check(host):
+        out = buf.download(np.uint32, count=total)
+        for w, (a, b) in zip(at, lengths):
+            x, y = (int.from_bytes(host[i:j].tobytes(), "little") for i, j in ((w, w + a), (w + a, w + a + b)))
+            assert int.from_bytes(out[w + a + b:w + 2 * (a + b)].tobytes(), "little") == x * y, (a, b)
+
+    with g.Context() as c:
+        host = fill()
+        g.check(c.mul_ragged(items), "mul_ragged")
+        g.synchronize()
+        check(host)
+        assert c.workspace_size() == 0
+        g.check(hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1), "hipStreamCreateWithFlags")
+        g.check(c.set_stream(stream), "set_stream")
+        g.check(hip.hipStreamBeginCapture(stream, 1), "hipStreamBeginCapture")  # thread-local
+        err = c.mul_ragged(items)
+        g.check(hip.hipStreamEndCapture(stream, ctypes.byref(graph)), "hipStreamEndCapture")
+        g.check(err, "mul_ragged under capture")
+        g.check(hip.hipGraphInstantiate(ctypes.byref(gexec), graph, None, None, ctypes.c_size_t(0)), "instantiate")
+        for _ in range(3):
+            host = fill()
+            g.check(hip.hipGraphLaunch(gexec, stream), "hipGraphLaunch")
+            g.synchronize()
+            check(host)
+        g.check(hip.hipGraphExecDestroy(gexec), "hipGraphExecDestroy")
+        g.check(hip.hipGraphDestroy(graph), "hipGraphDestroy")
+        g.check(c.set_stream(None), "set_stream")
+        g.check(hip.hipStreamDestroy(stream), "hipStreamDestroy")
