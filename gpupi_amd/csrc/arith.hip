@@ -11,6 +11,7 @@
 
 #include "common.hpp"
 #include "gpupi_pi.h"
+#include "gpupi_serve.h"
 
 namespace {
 
@@ -523,6 +524,10 @@ hipError_t batch_mp_mul_shared(BatchMPContext *ctx, BatchMPArray A1, BatchMPArra
 }
 
 namespace {
+// Of a multiply job's estimate (gpupi_serve_job_bytes): descriptors and
+// alignment.
+constexpr uint64_t kRaggedItemBytes = 4096;
+
 // The NTT launches of a ragged call: rows of whole products, and the
 // pieces of split ones (plans[q].m >= 2) with their assemblies, grouped by
 // transform size into launches filled to ntt_ragged_max_rows rows (a
@@ -580,18 +585,36 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
         }
         return f->second;
     };
+    // a context on a memory pool (a serving lane) takes no more scratch than
+    // its items' estimates reserve: a launch that shares a transform size, or
+    // the longest row's staging, with larger rows is cut where it would
+    uint64_t most_bytes = ~0ull;
+    if (ctx->cache->pool() != nullptr) {
+        most_bytes = 0;
+        for (uint32_t i : big)
+            most_bytes += gpupi_serve_job_bytes(GPUPI_JOB_MUL, items[i].L_a, items[i].L_b) -
+                          8ull * ((uint64_t)items[i].L_a + items[i].L_b) - kRaggedItemBytes;
+    }
     size_t ntt_bytes = 0;
     for (size_t g0 = 0; g0 < groups.size();) {
         const gpupi::NttShape shape = groups[g0].shape;
         const size_t cap = gpupi::ntt_ragged_max_rows(shape.k);
         Launch l{shape, host_rows.size(), 0, host_bset.size(), 0, host_asms.size(), 0, 0};
+        uint32_t row_limbs = 0;
         bidx.clear();
         size_t g1 = g0;
         for (; g1 < groups.size() && key(groups[g1].shape) == key(shape); ++g1) {
             const size_t q = groups[g1].q;
             const GpupiMulItem &it = items[big[q]];
             const uint32_t m = plans[q].m < 2 ? 1u : plans[q].m;
-            if (l.n > 0 && l.n + m > cap) break;
+            const uint32_t limbs =
+                std::max(row_limbs, m == 1 ? it.L_a + it.L_b : plans[q].s + std::min(it.L_a, it.L_b));
+            if (l.n > 0 && (l.n + m > cap ||
+                            gpupi::ntt_ragged_workspace_bytes((uint32_t)l.n + m, (uint32_t)l.nb + 1u,
+                                                              l.chunks + gpupi::assembly_chunks(it.L_a + it.L_b), limbs,
+                                                              shape) > most_bytes))
+                break;
+            row_limbs = limbs;
             if (m == 1) {
                 host_rows.push_back(gpupi::RaggedRow{it.A, it.B, it.C, it.L_a, it.L_b, b_of(l, it.B, it.L_b), 0});
             } else {
@@ -610,7 +633,8 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
             b.tau = std::max(b.tau, gpupi::ntt_tau(host_rows[r].L_a, host_rows[r].L_b, shape.k, shape.bits));
         }
         l.na = host_asms.size() - l.a0;
-        ntt_bytes = std::max(ntt_bytes, gpupi::ntt_ragged_workspace_bytes((uint32_t)l.n, (uint32_t)l.nb, l.chunks, shape));
+        ntt_bytes = std::max(
+            ntt_bytes, gpupi::ntt_ragged_workspace_bytes((uint32_t)l.n, (uint32_t)l.nb, l.chunks, row_limbs, shape));
         launches.push_back(l);
         g0 = g1;
     }
@@ -641,7 +665,7 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
     return hipSuccess;
 }
 
-hipError_t mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint32_t count) {
+static hipError_t mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uint32_t count) {
     // validate everything before launching anything
     std::vector<uint32_t> big;  // NTT products
     for (uint32_t i = 0; i < count; ++i) {

@@ -152,7 +152,7 @@ hipError_t launch_mul_ntt_pieces(const uint32_t *L, uint32_t LL, const uint32_t 
 // n assemblies, `chunks` chunks in all; `flags` holds one byte per chunk.
 hipError_t launch_ragged_assemble(const uint32_t *staging, uint64_t stride, const RaggedAssembly *as, uint32_t n,
                                   uint32_t chunks, uint8_t *flags, hipStream_t stream);
-size_t ntt_ragged_workspace_bytes(uint32_t N, uint32_t nb, uint32_t chunks, const NttShape &shape);
+size_t ntt_ragged_workspace_bytes(uint32_t N, uint32_t nb, uint32_t chunks, uint32_t row_limbs, const NttShape &shape);
 // N rows over nb B operands and n_asm assemblies of `chunks` chunks in all,
 // as device arrays with host copies: every row's digits fit the shape and
 // b < nb; rows without C (assembled) only above one tile (2^k > 4096).

@@ -1852,6 +1852,7 @@ struct NttJob {
     const RaggedAssembly *asms = nullptr;
     const RaggedAssembly *host_asms = nullptr;
     uint32_t n_asm = 0, asm_chunks = 0;
+    uint32_t row_limbs = 0;  // ragged: limbs of the longest row's product
     int k = 0;
     uint32_t bits = 32;    // of a digit
     size_t max_chunk = 0;  // rows per launch chunk at most (0: the default)
@@ -1867,8 +1868,9 @@ struct JobShape {
     uint32_t tau = kTauMax;  // parts of the transforms in use (the most of any product)
 };
 
-// Limbs from one staged product of a ragged launch to the next.
-uint64_t staging_stride(const NttJob &j) { return ((1ull << j.k) * j.bits) >> 5; }
+// Limbs from one staged product of a ragged launch to the next: what the
+// longest takes (the transform would hold a quarter more with 40-bit digits).
+uint64_t staging_stride(const NttJob &j) { return ((uint64_t)j.row_limbs + 3u) & ~3ull; }
 
 JobShape shape_of(const NttJob &j) {
     JobShape sh;
@@ -1889,7 +1891,7 @@ JobShape shape_of(const NttJob &j) {
         else if (j.host_rows != nullptr)
             for (uint32_t i = 0; i < pr.N; ++i) row(j.host_rows[i].L_a, j.host_rows[i].L_b);
         else {
-            limbs = staging_stride(j);
+            limbs = j.row_limbs;
             digits = K;
         }
         sh.Lc[q] = (uint32_t)limbs;
@@ -2415,7 +2417,8 @@ uint32_t ntt_piece_tau(int k, uint32_t s, uint32_t S) { return ntt_tau(s, S, k, 
 namespace {
 NttJob ragged_job(const RaggedRow *rows, const RaggedRow *host_rows, uint32_t N, const RaggedB *bset,
                   const RaggedB *host_bset, uint32_t nb, const RaggedAssembly *asms,
-                  const RaggedAssembly *host_asms, uint32_t n_asm, uint32_t asm_chunks, const NttShape &shape) {
+                  const RaggedAssembly *host_asms, uint32_t n_asm, uint32_t asm_chunks, uint32_t row_limbs,
+                  const NttShape &shape) {
     NttJob j;
     j.n_ops = 2;
     j.n_prods = 1;
@@ -2430,6 +2433,7 @@ NttJob ragged_job(const RaggedRow *rows, const RaggedRow *host_rows, uint32_t N,
     j.host_asms = host_asms;
     j.n_asm = n_asm;
     j.asm_chunks = asm_chunks;
+    j.row_limbs = row_limbs;
     set_shape(j, shape);
     return j;
 }
@@ -2493,7 +2497,8 @@ PiecesLayout pieces_layout(uint32_t LL, uint32_t LS, uint32_t m, uint32_t s) {
     l.bset_bytes = align256(sizeof(RaggedB));
     l.asm_bytes = align256(sizeof(RaggedAssembly));
     l.ntt_bytes =
-        job_workspace_bytes(ragged_job(nullptr, nullptr, m, nullptr, nullptr, 1, nullptr, nullptr, 1, l.chunks, l.shape));
+        job_workspace_bytes(ragged_job(nullptr, nullptr, m, nullptr, nullptr, 1, nullptr, nullptr, 1, l.chunks, s + LS,
+                                       l.shape));
     return l;
 }
 }  // namespace
@@ -2527,13 +2532,13 @@ hipError_t launch_mul_ntt_pieces(const uint32_t *L, uint32_t LL, const uint32_t 
     for (uint32_t i = 0; i < m; ++i) host_rows[i] = piece_row(i, L, LL, S, LS, m, s, 0);
     const RaggedB host_b{S, LS, tau};
     const RaggedAssembly host_as{C, LL + LS, s, LS, m, 0, 0};
-    return run_ntt(ragged_job(rows, host_rows.data(), m, bset, &host_b, 1, as, &host_as, 1, l.chunks, l.shape),
+    return run_ntt(ragged_job(rows, host_rows.data(), m, bset, &host_b, 1, as, &host_as, 1, l.chunks, s + LS, l.shape),
                    ws + l.rows_bytes + l.bset_bytes + l.asm_bytes, l.ntt_bytes, tables, stream);
 }
 
-size_t ntt_ragged_workspace_bytes(uint32_t N, uint32_t nb, uint32_t chunks, const NttShape &shape) {
-    return job_workspace_bytes(
-        ragged_job(nullptr, nullptr, N, nullptr, nullptr, nb, nullptr, nullptr, chunks ? 1u : 0u, chunks, shape));
+size_t ntt_ragged_workspace_bytes(uint32_t N, uint32_t nb, uint32_t chunks, uint32_t row_limbs, const NttShape &shape) {
+    return job_workspace_bytes(ragged_job(nullptr, nullptr, N, nullptr, nullptr, nb, nullptr, nullptr, chunks ? 1u : 0u,
+                                          chunks, row_limbs, shape));
 }
 
 hipError_t launch_mul_ntt_ragged(const RaggedRow *rows, const RaggedRow *host_rows, uint32_t N, const RaggedB *bset,
@@ -2546,7 +2551,9 @@ hipError_t launch_mul_ntt_ragged(const RaggedRow *rows, const RaggedRow *host_ro
         bset == nullptr || host_bset == nullptr || (n_asm > 0 && (asms == nullptr || host_asms == nullptr)) ||
         !ragged_ok(host_rows, N, host_bset, nb, host_asms, n_asm, chunks, shape))
         return hipErrorInvalidValue;
-    return run_ntt(ragged_job(rows, host_rows, N, bset, host_bset, nb, asms, host_asms, n_asm, chunks, shape),
+    uint32_t row_limbs = 0;
+    for (uint32_t i = 0; i < N; ++i) row_limbs = std::max(row_limbs, host_rows[i].L_a + host_rows[i].L_b);
+    return run_ntt(ragged_job(rows, host_rows, N, bset, host_bset, nb, asms, host_asms, n_asm, chunks, row_limbs, shape),
                    workspace, workspace_bytes, tables, stream);
 }
 

@@ -281,9 +281,11 @@ uint64_t gpupi_serve_job_bytes(int kind, uint32_t a, uint32_t b) {
     const uint64_t L = (uint64_t)a + b;
     uint64_t K = 16;
     while (K < L) K <<= 1;
-    // operands + product (8 B per limb) + ragged NTT scratch (4 planes of
-    // 8 B, staging 4 B, spill and flags: < 37 B per coefficient)
-    return 8 * L + 37 * K + 4096;
+    // operands + product (8 B per limb) + ragged NTT scratch, which
+    // gpupi_mul_ragged keeps within the rest on a memory pool: per coefficient
+    // 4 planes of 8 B (padded: an eighth more at the most), a limb of staging,
+    // spill words and flags, < 37.25 B; then descriptors and alignment
+    return 8 * L + 37 * K + K / 4 + 4096;
 }
 
 int gpupi_serve_admit(const uint64_t *bytes, const int32_t *kind, int n, uint64_t budget, uint64_t in_use,

@@ -1,6 +1,8 @@
 """GPU: the serving loop (gpupi_serve.h).  A mix of pi-digit and multiply
 jobs submitted together must give every job the result it gets alone, and
 those results must equal the oracle (GMP mpn_mul; the pi restatement)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -124,3 +126,32 @@ def test_small_budget_serializes_but_stays_exact():
         assert np.array_equal(data, oracle_mul(A, B))
     spans = sorted((r.start_ms, r.finish_ms) for r, _ in out.values())
     assert all(b[0] >= a[1] - 1e-6 for a, b in zip(spans, spans[1:]))  # one at a time
+
+
+@pytest.mark.parametrize("lengths", [
+    [(120000, 120000)], [(1 << 19, 1 << 19)], [(1 << 20, 5000)], [(3000000, 70000)],
+    # small rows next to larger ones, whose transform they could share
+    [(120000, 110000)] + [(5000 + i, 4000) for i in range(12)],
+    [(2 ** u // 2, 2 ** u // 2 - 5 * u) for u in range(13, 19) for _ in range(3)],
+    # a row whose digits fit half the transform of its limbs, and many shorter ones
+    [(9800, 9700)] + [(6000 + i, 5900) for i in range(60)],
+], ids=str)
+def test_ragged_scratch_on_a_pool_stays_within_the_estimates(lengths):
+    """A context on a memory pool (as the server's multiply lane) takes no more
+    scratch for a ragged call than its items' estimates hold besides their
+    operands and products."""
+    rng = np.random.default_rng(len(lengths))
+    pool = ctypes.c_void_p()
+    g.check(g.hip().hipDeviceGetDefaultMemPool(ctypes.byref(pool), 0), "hipDeviceGetDefaultMemPool")
+    pairs = [(rand_rows(rng, 1, a)[0], rand_rows(rng, 1, b)[0]) for a, b in lengths]
+    bufs = [(g.DeviceBuffer.from_array(a), g.DeviceBuffer.from_array(b), g.DeviceBuffer(4 * (a.size + b.size)))
+            for a, b in pairs]
+    with g.Context() as c:
+        g.check(g.lib().gpupi_set_memory_pool(c.ptr, pool), "gpupi_set_memory_pool")
+        g.check(c.mul_ragged([(x.ptr, y.ptr, z.ptr, a, b) for (x, y, z), (a, b) in zip(bufs, lengths)]), "mul_ragged")
+        g.synchronize()
+        used = c.workspace_size()
+    for (a, b), (_, _, z) in zip(pairs, bufs):
+        assert np.array_equal(z.download(np.uint32, count=a.size + b.size), oracle_mul(a, b)), (a.size, b.size)
+    room = sum(g.lib().gpupi_serve_job_bytes(g.JOB_MUL, a, b) - 8 * (a + b) for a, b in lengths)
+    assert 0 < used <= room, (used, room)

@@ -1,5 +1,7 @@
 """CPU: the serving loop's admission rule and footprint estimate
 (gpupi_serve.h), called through the C ABI with no device work."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -44,6 +46,29 @@ def test_footprint_estimates():
     # pi: the largest job of the serving mix (10^8 digits) fits the budget many times over
     assert lib.gpupi_serve_job_bytes(PI, 10 ** 8, 0) < 5 * GB
     assert lib.gpupi_serve_job_bytes(PI, 10 ** 5, 0) < lib.gpupi_serve_job_bytes(PI, 10 ** 8, 0)
+
+
+class _NttShape(ctypes.Structure):
+    _fields_ = [("k", ctypes.c_int), ("bits", ctypes.c_uint32)]
+
+
+def test_multiply_estimate_covers_its_scratch():
+    """A multiply job's reservation holds its operands, its product and the
+    scratch of its transform (the library's own layout), at lengths around
+    every power of two and where 40-, 36- and 34-bit digits fill it."""
+    lib = g.lib()
+    shape = getattr(lib, "_ZN5gpupi9ntt_shapeEjj")
+    shape.restype, shape.argtypes = _NttShape, [ctypes.c_uint32] * 2
+    scratch = getattr(lib, "_ZN5gpupi26ntt_ragged_workspace_bytesEjjjjRKNS_8NttShapeE")
+    scratch.restype, scratch.argtypes = ctypes.c_size_t, [ctypes.c_uint32] * 4 + [ctypes.POINTER(_NttShape)]
+    totals = [int(f * (1 << k)) + d for k in range(12, 29) for f in (0.55, 0.8, 0.92, 1.0, 1.05, 1.12, 1.24)
+              for d in (-1, 0, 1)]
+    for total in totals:
+        for la in (total // 2, total - total // 9):
+            lb = total - la
+            sh = shape(la, lb)
+            need = scratch(1, 1, 0, total, ctypes.byref(sh)) + 3 * 256  # and its descriptors
+            assert need <= lib.gpupi_serve_job_bytes(MUL, la, lb) - 8 * total, (la, lb, sh.k, sh.bits)
 
 
 def test_server_threading_simulation(tmp_path):
