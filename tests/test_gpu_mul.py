@@ -941,3 +941,21 @@ def test_small_ragged_calls_only_launch(count):
         g.check(hip.hipGraphDestroy(graph), "hipGraphDestroy")
         g.check(c.set_stream(None), "set_stream")
         g.check(hip.hipStreamDestroy(stream), "hipStreamDestroy")
+
+
+@pytest.mark.parametrize("la,k", [(1100000, 21), (1500000, 22), (2700000, 23)])
+def test_large_squares_run_whole(ctx, la, k):
+    """A square takes one transform of its operand, at the size of the whole
+    product, also where two different operands of its length run in pieces."""
+    A = rand_rows(np.random.default_rng(la), 1, la)
+    buf, va = g.upload_rows(A)
+    bufc, vc = g.upload_rows(np.zeros((1, 2 * la), np.uint32))
+    g.kernel_stats_reset(True)
+    try:
+        g.check(ctx.mul(va, va, vc), "square")
+        g.synchronize()
+        stats = {name: launches for name, launches, _, _ in g.kernel_stats(by_size=True)}
+    finally:
+        g.kernel_stats_reset(False)
+    assert np.array_equal(g.download_rows(vc, bufc), oracle_mul(A, A))
+    assert stats and all(name.endswith(f"@2^{k}") for name in stats), stats
