@@ -546,14 +546,11 @@ hipError_t launch_mul_mfma(const uint32_t *A, const uint32_t *B, uint32_t *C, ui
         std::swap(LA, LB);
         std::swap(sA, sB);
     }
-    if (N == 0 || N > 0x7fffffffu || LA == 0 || (uint64_t)LA + LB > kMulMfmaMaxTotal) return hipErrorInvalidValue;
+    if (N == 0 || LA == 0 || (uint64_t)LA + LB > kMulMfmaMaxTotal) return hipErrorInvalidValue;
     const bool few = LA + LB > kTileLimbs && N <= kFewRows;
     uint32_t W = 1;
     MfmaArgs a = shape_of(LA, LB, W);
     while (a.M + a.E - 1 > (few ? kFewG : kManyG)) a = shape_of(LA, LB, ++W);
-    a.A = A;
-    a.B = B;
-    a.C = C;
     a.sA = sA;
     a.sB = sB;
     a.sC = sC;
@@ -570,8 +567,16 @@ hipError_t launch_mul_mfma(const uint32_t *A, const uint32_t *B, uint32_t *C, ui
     const size_t lds = (a.lds_words + (few ? tiles * 1024u : 0u)) * 4u;
     if (k == nullptr || tiles > kMaxTiles || W > 4 || lds > 160 * 1024) return hipErrorInvalidValue;
     if (lds > 65536) GPUPI_RETURN_IF(allow_large_lds());
-    hipLaunchKernelGGL(k, dim3(N), dim3(kWave * W * (few ? kParts : 1)), lds, stream, a);
-    return hipGetLastError();
+    // a launch holds fewer than 2^32 threads
+    const uint32_t threads = kWave * W * (few ? kParts : 1u), most = 0xffffffffu / threads;
+    for (uint32_t r0 = 0; r0 < N; r0 += std::min(most, N - r0)) {
+        a.A = A + (size_t)r0 * sA;
+        a.B = B + (size_t)r0 * sB;
+        a.C = C + (size_t)r0 * sC;
+        hipLaunchKernelGGL(k, dim3(std::min(most, N - r0)), dim3(threads), lds, stream, a);
+        GPUPI_RETURN_IF(hipGetLastError());
+    }
+    return hipSuccess;
 }
 
 namespace {

@@ -959,3 +959,20 @@ def test_large_squares_run_whole(ctx, la, k):
         g.kernel_stats_reset(False)
     assert np.array_equal(g.download_rows(vc, bufc), oracle_mul(A, A))
     assert stats and all(name.endswith(f"@2^{k}") for name in stats), stats
+
+
+def test_more_rows_than_one_launch_holds(ctx):
+    """Matrix-core products of more rows than a launch's 2^32 threads cover
+    (64 per row): the rows around the seam, the first and the last."""
+    n, la, lb, seam = (1 << 26) + 77, 17, 18, (1 << 26) - 1
+    rng = np.random.default_rng(26)
+    A, B = rand_rows(rng, 1, la), rand_rows(rng, 1, lb)
+    (ba, va), (bb, vb) = g.upload_rows(A), g.upload_rows(B)
+    out = g.DeviceBuffer(4 * n * (la + lb))
+    out.fill(0xAB)
+    g.check(ctx.mul(va.view(batch_size=n, stride=0), vb.view(batch_size=n, stride=0),
+                    g.BatchMPArray(out.ptr, la + lb, n, la + lb)), "mul")
+    g.synchronize()
+    want = oracle_mul(A, B)[0]
+    for row in [0, 1, seam - 1, seam, seam + 1, n - 1] + [int(r) for r in rng.integers(0, n, size=50)]:
+        assert np.array_equal(out.download(np.uint32, count=la + lb, offset_bytes=4 * row * (la + lb)), want), row
