@@ -6,13 +6,14 @@ row; two columns + row), the 1024-limb boundary of the reference
 (batch_arith_test.cu:99-103), random shapes with random strides in the style
 of batch_mul_ntt_test.cu:531-556, and broadcast operands."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
 
 import gpupi_amd as g
 import oracle_ffi as of
-from helpers import rand_rows
+from helpers import rand_rows, to_int
 
 pytestmark = pytest.mark.gpu
 PAD = 0xDEADBEEF
@@ -976,3 +977,51 @@ def test_more_rows_than_one_launch_holds(ctx):
     want = oracle_mul(A, B)[0]
     for row in [0, 1, seam - 1, seam, seam + 1, n - 1] + [int(r) for r in rng.integers(0, n, size=50)]:
         assert np.array_equal(out.download(np.uint32, count=la + lb, offset_bytes=4 * row * (la + lb)), want), row
+
+
+@pytest.mark.parametrize("n", [3, 16384, 20000])
+@pytest.mark.parametrize("la,lb", [(127, 16), (128, 1), (129, 1), (129, 16), (380, 3), (1011, 12), (4087, 1), (4072, 16)])
+def test_short_operand_against_long(n, la, lb):
+    """Many and few rows of a short operand times a long one, around the
+    lengths and the number of rows where the schoolbook kernels change or used
+    to: GMP's products, and Python's for a row."""
+    if n * (la + lb) > 1 << 25:
+        n = (1 << 25) // (la + lb)
+    rng = np.random.default_rng(la + lb)
+    with g.Context() as c:
+        A, B = rand_rows(rng, n, la, "ones"), rand_rows(rng, n, lb, "random")
+        A[1::3] = rand_rows(rng, len(A[1::3]), la, "random")
+        assert np.array_equal(device_mul(c, A, B, sa=la + 1, sb=lb + 2), oracle_mul(A, B))
+        assert np.array_equal(device_mul(c, B, A), oracle_mul(B, A))
+        assert to_int(device_mul(c, A[:1], B[:1])[0]) == to_int(A[0]) * to_int(B[0])
+
+
+def test_short_operands_of_many_rows_take_the_matrix_cores():
+    """Rows of a short operand against a long one take no longer in a batch of
+    16384 than the same rows in calls of 8192 (a slower kernel for many rows
+    took three to nineteen times as long)."""
+    n, la, lb = 16384, 2000, 4
+    rng = np.random.default_rng(5)
+    with g.Context() as c:
+        (ba, va), (bb, vb) = g.upload_rows(rand_rows(rng, n, la)), g.upload_rows(rand_rows(rng, n, lb))
+        out = g.DeviceBuffer(4 * n * (la + lb))
+
+        def parts(rows):
+            for r in range(0, n, rows):
+                g.check(c.mul(g.BatchMPArray(ba.ptr + 4 * r * la, la, rows, la),
+                              g.BatchMPArray(bb.ptr + 4 * r * lb, lb, rows, lb),
+                              g.BatchMPArray(out.ptr + 4 * r * (la + lb), la + lb, rows, la + lb)), "mul")
+
+        def seconds(rows):
+            best = 1e9
+            for _ in range(5):
+                g.synchronize()
+                t0 = time.perf_counter()
+                for _ in range(10):
+                    parts(rows)
+                g.synchronize()
+                best = min(best, time.perf_counter() - t0)
+            return best
+
+        parts(n)
+        assert seconds(n) < 2.0 * seconds(n // 2)
