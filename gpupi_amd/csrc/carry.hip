@@ -194,9 +194,13 @@ __global__ void __launch_bounds__(256) carry_fixup_kernel(uint32_t *C, uint32_t 
 // bound by the time of a launch: one addition of 16000 limbs takes 4.4 us
 // instead of 6.8 with carry_fixup_kernel behind it, 64 of them 5.8 instead of
 // 6.8, and full chips gain too, by one reading of the flags (8192 rows of 4000
-// limbs 73 instead of 78, 1024 of 16000 limbs 35.3 instead of 36.3 us).
-// Sixteen waves are the largest block.
-constexpr uint32_t kRowWaves = 16;
+// limbs 73 instead of 78, 1024 additions of 12000 limbs 23.6 instead of 27.0).
+// Sixteen waves are the largest block.  Of 13 waves and more two blocks fill a
+// CU and wait on memory together, which costs the operations that read most:
+// the shifts of more rows than CUs go by chunks there (1024 of 16384 limbs
+// 34.6 instead of 42.8 us, 2048 of 14336 66.5 instead of 75; 256 of 14336
+// still 8.6 by rows, 10.5 by chunks).
+constexpr uint32_t kRowWaves = 16, kRowWavesMany = 12, kManyRows = 256;
 
 // Which chunk a wave works on.
 struct ChunkPos {
@@ -481,8 +485,13 @@ __device__ __forceinline__ void load4(const uint32_t *r, int64_t j0, uint32_t L,
 // carry_fixup_kernel completes longer rows).
 // Bound by HBM; the 16-byte accesses start at any limb, so row strides and
 // shifts need no alignment (R = (R1 << s) - R2 over 512 rows of 128249 limbs:
-// 271 us with a limb per lane, 158 us this way).
-template <AddSubKind K, bool ROW>
+// 271 us with a limb per lane, 158 us this way).  The shifted operand's limbs
+// lie at any offset from the others': as one limb and four (QUAD) well inside
+// the last cache, as five limbs beyond (64 rows of 2^20 limbs in
+// 16-byte aligned rows 159 / 150 us, 4096 of 10240 100 / 95; 64 of 128249,
+// 98 MB, 19.0 / 20.2; 30000 of 700, 252 MB, 44.0 / 39.0).
+constexpr uint64_t kShiftQuadBytes = 160ull << 20;
+template <AddSubKind K, bool ROW, bool QUAD>
 __global__ void __launch_bounds__(ROW ? kRowWaves * kWave : 256)
 addsub_vec_kernel(AddSubArgs a, uint32_t chunks_per_row, uint64_t total_chunks, uint8_t *flags) {
     constexpr bool kSub = OpTraits<K>::kSub;
@@ -506,7 +515,12 @@ addsub_vec_kernel(AddSubArgs a, uint32_t chunks_per_row, uint64_t total_chunks, 
             uint32_t w[5];
             const int64_t i = j0 - ws - 1;
             w[0] = (i >= 0 && i < (int64_t)a.L_a) ? ra[i] : 0u;
-            load4(ra, i + 1, a.L_a, w + 1);
+            if constexpr (QUAD) {
+                load4(ra, i + 1, a.L_a, w + 1);
+            } else {
+#pragma unroll
+                for (int t = 1; t < 5; ++t) w[t] = (i + t >= 0 && i + t < (int64_t)a.L_a) ? ra[i + t] : 0u;
+            }
 #pragma unroll
             for (int t = 0; t < 4; ++t) x[t] = bs ? (w[t + 1] << bs) | (w[t] >> (32u - bs)) : w[t + 1];
         } else if constexpr (K == AddSubKind::MulSmall) {
@@ -620,8 +634,11 @@ hipError_t run_addsub(const AddSubArgs &a, const SpillArgs &sp, uint8_t *flags, 
         return hipGetLastError();
     }
     const uint64_t total = (uint64_t)a.N * p.chunks_per_row;
+    constexpr bool kShift = K == AddSubKind::ShiftAdd || K == AddSubKind::ShiftSub;
     // one block per row where a row's chunks fit it
-    const bool rows = p.chunks_per_row > 1 && p.chunks_per_row <= kRowWaves;
+    const bool rows =
+        p.chunks_per_row > 1 && p.chunks_per_row <= (kShift && a.N > kManyRows ? kRowWavesMany : kRowWaves);
+    const bool quad = !kShift || 4ull * a.N * ((uint64_t)a.L_a + a.L_b + a.L_c) <= kShiftQuadBytes;
     const bool need_fix = p.chunks_per_row > 1 && !rows;
     if (p.chunks_per_row > 1 && flags == nullptr) return hipErrorInvalidValue;
     const uint64_t blocks = rows ? a.N : ceil_div64(total, 4);
@@ -643,7 +660,8 @@ hipError_t run_addsub(const AddSubArgs &a, const SpillArgs &sp, uint8_t *flags, 
                 const auto k = rows ? spill_add_vec_kernel<true> : spill_add_vec_kernel<false>;
                 hipLaunchKernelGGL(k, grid, block, 0, stream, a.C, a.stride_C, a.L_c, sp, p.chunks_per_row, total, fl);
             } else {
-                const auto k = rows ? addsub_vec_kernel<K, true> : addsub_vec_kernel<K, false>;
+                const auto k = !quad ? (rows ? addsub_vec_kernel<K, true, !kShift> : addsub_vec_kernel<K, false, !kShift>)
+                                     : (rows ? addsub_vec_kernel<K, true, true> : addsub_vec_kernel<K, false, true>);
                 hipLaunchKernelGGL(k, grid, block, 0, stream, a, p.chunks_per_row, total, fl);
             }
     }

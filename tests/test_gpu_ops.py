@@ -256,3 +256,25 @@ def test_rows_at_any_alignment(ctx, la, extra):
     g.synchronize()
     got = g.download_rows(va, bufa)
     assert [value(r) for r in got] == [(x + y) % (1 << (32 * la)) for x, y in zip(a, b)]
+
+
+@pytest.mark.parametrize("op", ["shift_add", "shift_sub"])
+@pytest.mark.parametrize("n,lc", [(256, 12290), (257, 12288), (257, 12290), (256, 16384), (257, 16384), (257, 16385),
+                                  (2100, 12288), (2100, 16384), (40000, 777), (9, 4000001)])
+def test_shifts_of_many_rows(ctx, op, n, lc):
+    """The shift operations around the numbers of rows and of 1024-limb chunks
+    where a block per row ends, and where the operands outgrow the last cache:
+    every row of a broadcast pair, at aligned and odd strides."""
+    rng = np.random.default_rng(n + lc)
+    for la, shift, pad in ((lc - 9, 255, 0), (lc - 3, 64, 1), (lc, 31, 3)):
+        A, B = rand_rows(rng, 1, la, "top" if pad == 1 else "random"), rand_rows(rng, 1, lc, "ones" if pad else "random")
+        (ba, va), (bb, vb) = g.upload_rows(A), g.upload_rows(B)
+        sc = lc + pad
+        buf = g.DeviceBuffer(4 * n * sc)
+        buf.fill(0x5E)
+        g.check(getattr(ctx, op)(va.view(batch_size=n, stride=0), vb.view(batch_size=n, stride=0), shift,
+                                 g.BatchMPArray(buf.ptr, lc, n, sc)), op)
+        g.synchronize()
+        got = buf.download(np.uint32, count=n * sc).reshape(n, sc)
+        assert to_int(got[0, :lc]) == closed_form(op, to_int(A[0]), to_int(B[0]), 0, shift, lc)
+        assert (got == got[0]).all() and (got[:, lc:] == 0x5E5E5E5E).all()
