@@ -1,6 +1,8 @@
 """GPU: every batched add/sub/shift/mul_small/exactdiv/shift_bits/length op
 through the C ABI, bit-exact against the oracle (and the closed form), with
 padding guards around every output row (batch_add_test.cu:33-35, 373-381)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -278,3 +280,22 @@ def test_shifts_of_many_rows(ctx, op, n, lc):
         got = buf.download(np.uint32, count=n * sc).reshape(n, sc)
         assert to_int(got[0, :lc]) == closed_form(op, to_int(A[0]), to_int(B[0]), 0, shift, lc)
         assert (got == got[0]).all() and (got[:, lc:] == 0x5E5E5E5E).all()
+
+
+@pytest.mark.parametrize("length", [255, 256, 257, 260, 300, 511, 512, 513, 1279, 1280, 1281, 1537])
+def test_row_lengths_around_the_scan_steps(ctx, length):
+    """Lengths of rows scanned a wave at a time, 256 limbs and then four times
+    as many: one row's top limb at every edge of those steps, below it zeros or
+    not, among zero rows; and all rows zero."""
+    tops = sorted({t for e in (0, 1, 4, 256, 512, 768, 1024, 1280) for d in (-1, 0, 1)
+                   for t in (e + d, length - e + d) if 0 <= t <= length})
+    for top in tops:
+        rows = np.zeros((9, length), dtype=np.uint32)
+        if top:
+            rows[4, top - 1] = 0x10
+            rows[7, :top - 1] = 0xFFFFFFFF
+        buf, arr = g.upload_rows(rows, length + 1, PAD)
+        assert ctx.limblength_max_value(arr) == top
+        r = ctypes.c_uint32(0)
+        g.check(ctx.bitlength_max(arr, ctypes.byref(r)), "bitlength_max")
+        assert r.value == (32 * (top - 1) + 5 if top else 0)
