@@ -1585,11 +1585,14 @@ size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Optional per-launch timing of the NTT kernels (HIP events on the launch
 // stream) with each launch's algorithmic bytes, for live roofline numbers.
-enum KernelKind { kColFwdLimbs, kColFwd, kRowFused, kRowPair, kColInv, kColInvLimbs, kLocal, kKindCount };
+enum KernelKind {
+    kColFwdLimbs, kColFwd, kRowFused, kRowPair, kColInv, kColInvLimbs, kLocal, kThinFwd, kThinRow, kThinInv, kKindCount
+};
 const char *const kKindNames[kKindCount] = {"ntt_col_fwd_kernel<limbs>", "ntt_col_fwd_kernel",
                                             "ntt_row_fused_kernel", "ntt_row_pair_kernel",
                                             "ntt_col_inv_kernel", "ntt_col_inv_limbs_kernel",
-                                            "ntt_local_kernel"};
+                                            "ntt_local_kernel", "ntt_thin_fwd_kernel",
+                                            "ntt_thin_row_kernel", "ntt_thin_inv_kernel"};
 struct StatRecord {
     int kind, log2K;
     hipEvent_t start, stop;
@@ -2146,7 +2149,7 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
         const uint32_t deep = a.tau_tiles;
         if (thin && fwd_rows > 0) {
             const uint32_t n = 2u << (k - kThinTileLog2);
-            GPUPI_RETURN_IF(timed(kColFwdLimbs, k, 4.0 * (double)limb_reads + fwd_tb, stream, [&] {
+            GPUPI_RETURN_IF(timed(kThinFwd, k, 4.0 * (double)limb_reads + fwd_tb, stream, [&] {
                 hipLaunchKernelGGL(ntt_thin_fwd_kernel, blocks(fwd_rows, n, 0), dim3(256), 0, stream, args(n, 0));
             }));
         } else if (fwd_rows > 0) {
@@ -2179,7 +2182,7 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
         if (prod_rows == 0) continue;
         if (thin) {
             const double row_tb = (j.prods[0].a == j.prods[0].b ? 2 : 3) * prod_tb;
-            GPUPI_RETURN_IF(timed(kRowFused, k, row_tb, stream, [&] {
+            GPUPI_RETURN_IF(timed(kThinRow, k, row_tb, stream, [&] {
                 dispatch_m<kThinRowLo, kThinRowMax>(p.log2M[1], [&](auto mc) {
                     constexpr int M = decltype(mc)::value, LT = thin_row_tile(M);
                     const uint32_t n = 2u << (k - LT);
@@ -2188,7 +2191,7 @@ hipError_t run_ntt(const NttJob &j, void *workspace, size_t workspace_bytes, con
                 });
             }));
             const uint32_t n = 1u << (k - kThinTileLog2);
-            GPUPI_RETURN_IF(timed(kColInvLimbs, k, prod_tb + 4.0 * (double)limb_writes + 8.0 * prod_rows * runs,
+            GPUPI_RETURN_IF(timed(kThinInv, k, prod_tb + 4.0 * (double)limb_writes + 8.0 * prod_rows * runs,
                                   stream, [&] {
                 hipLaunchKernelGGL(ntt_thin_inv_kernel, blocks(prod_rows, n, 0), dim3(512), 0, stream, args(n, 0));
             }));

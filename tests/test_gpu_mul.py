@@ -1025,3 +1025,20 @@ def test_short_operands_of_many_rows_take_the_matrix_cores():
 
         parts(n)
         assert seconds(n) < 2.0 * seconds(n // 2)
+
+
+@pytest.mark.parametrize("n,la,lb,thin", [(1, 4096, 4095, True), (4, 100000, 90000, True), (200, 4096, 4095, False),
+                                          (1, 1048576, 1000000, False)])
+def test_kernel_statistics_name_the_kernels_that_ran(ctx, n, la, lb, thin):
+    """Short launches' thin tiles have names of their own in the live
+    statistics, one forward, row and inverse launch of each kind."""
+    rng = np.random.default_rng(la)
+    A, B = rand_rows(rng, n, la), rand_rows(rng, n, lb)
+    g.kernel_stats_reset(True)
+    try:
+        assert np.array_equal(device_mul(ctx, A, B), oracle_mul(A, B))
+        names = sorted(name for name, launches, *_ in g.kernel_stats() if launches == 1)
+    finally:
+        g.kernel_stats_reset(False)
+    full = ["ntt_col_fwd_kernel<limbs>", "ntt_col_inv_limbs_kernel", "ntt_row_fused_kernel"]
+    assert names == (["ntt_thin_fwd_kernel", "ntt_thin_inv_kernel", "ntt_thin_row_kernel"] if thin else full)
