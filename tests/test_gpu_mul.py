@@ -1042,3 +1042,94 @@ def test_kernel_statistics_name_the_kernels_that_ran(ctx, n, la, lb, thin):
         g.kernel_stats_reset(False)
     full = ["ntt_col_fwd_kernel<limbs>", "ntt_col_inv_limbs_kernel", "ntt_row_fused_kernel"]
     assert names == (["ntt_thin_fwd_kernel", "ntt_thin_inv_kernel", "ntt_thin_row_kernel"] if thin else full)
+
+
+def digit_limbs(digits, bits):
+    """The most limbs that make this many digits."""
+    return digits * bits // 32
+
+
+@pytest.mark.parametrize("k", [13, 14, 16, 18, 19, 20, 21, 22, 23])
+def test_parts_of_truncated_transforms(ctx, k):
+    """Products whose digits fill 10, 12, 14 or 16 parts of 2^k points exactly,
+    one digit less and one more (and just over half of them), on full tiles of
+    that size as the kernel statistics show: pairs of rows, a broadcast operand
+    and a shared pair, against GMP; nothing is written past a row."""
+    K, rng = 1 << k, np.random.default_rng(1000 + k)
+    # digits of the shorter operand: 40 bits up to FORTY of them, else 36
+    bits, short = (40, K // 8 - 3) if k <= 20 else (36, K // 6)
+    totals = [K // 2 + 1] + [K * t // 16 + d for t in (10, 12, 14) for d in (-1, 0, 1)] + [K - 1, K]
+    if k > 20:
+        totals = totals[k % 2::2] + [K]
+    # sizes set by hand (to the built-in ones) keep short launches on full tiles
+    g.ntt_set_split(k, *(g.ntt_get_split(k)[:-1] if k < 20 else (0,)))
+    try:
+        for i, total in enumerate(totals):
+            la, lb = digit_limbs(total - short, bits), digit_limbs(short, bits)
+            A = rand_rows(rng, 2, la, ("random", "ones", "top")[i % 3])
+            B = rand_rows(rng, 2, lb, ("ones", "random")[i % 2])
+            g.kernel_stats_reset(True)
+            assert np.array_equal(device_mul(ctx, A, B, sa=la + 1), oracle_mul(A, B)), total
+            names = {name for name, *_ in g.kernel_stats(by_size=True)}
+            g.kernel_stats_reset(False)
+            assert names and all(n.endswith(f"@2^{k}") and "thin" not in n for n in names), (total, names)
+            if i % 3 == 0:
+                assert np.array_equal(device_mul(ctx, A, B, b_broadcast=True), oracle_mul(A, np.repeat(B[:1], 2, axis=0)))
+                A2 = rand_rows(rng, 2, la - la // 9)
+                got = device_mul_shared(ctx, A, A2, B)
+                assert np.array_equal(got[0], oracle_mul(A, B)) and np.array_equal(got[1], oracle_mul(A2, B))
+    finally:
+        g.kernel_stats_reset(False)
+        g.ntt_set_split(k, 0)
+
+
+@pytest.mark.parametrize("k", [13, 15, 17])
+def test_parts_of_ragged_rows(ctx, k):
+    """One ragged launch of rows that fill different numbers of parts of 2^k
+    points, each exactly, one digit less and one more, some sharing an operand."""
+    K, rng = 1 << k, np.random.default_rng(2000 + k)
+    short = K // 5
+    shared = rand_rows(rng, 1, digit_limbs(short, 40))[0]
+    sb = g.DeviceBuffer.from_array(shared)
+    rows = []
+    for i, total in enumerate([K // 2 + 1] * 9 + [K * t // 16 + d for t in (10, 12, 14) for d in (-1, 0, 1)] + [K]):
+        a = rand_rows(rng, 1, digit_limbs(total - short, 40), ("random", "ones")[i % 2])[0]
+        b = shared if i % 3 else rand_rows(rng, 1, digit_limbs(short, 40), "top")[0]
+        rows.append((a, b, g.DeviceBuffer.from_array(a), sb if b is shared else g.DeviceBuffer.from_array(b),
+                     g.DeviceBuffer.from_array(np.full(a.size + b.size + 1, PAD, dtype=np.uint32))))
+    g.kernel_stats_reset(True)
+    try:
+        g.check(ctx.mul_ragged([(x.ptr, y.ptr, z.ptr, a.size, b.size) for a, b, x, y, z in rows]), "mul_ragged")
+        g.synchronize()
+        sizes = {name.split("@2^")[1] for name, *_ in g.kernel_stats(by_size=True)}
+    finally:
+        g.kernel_stats_reset(False)
+    assert sizes == {str(k)}, sizes
+    for a, b, _, _, z in rows:
+        got = z.download(np.uint32, count=a.size + b.size + 1)
+        assert got[-1] == PAD
+        assert np.array_equal(got[:-1], oracle_mul(a.reshape(1, -1), b.reshape(1, -1))[0]), (a.size, b.size)
+
+
+def test_every_tile_pairing_with_streamed_and_truncated_planes(ctx):
+    """Two rows of 2^23 points whose planes go past the caches and fill 12 of
+    16 parts: every tile pairing gives GMP's product."""
+    rng = np.random.default_rng(23)
+    la, lb = 3200000, 3500000
+    A, B = rand_rows(rng, 2, la), rand_rows(rng, 2, lb, "ones")
+    want = oracle_mul(A, B)
+    (ba, va), (bb, vb) = g.upload_rows(A), g.upload_rows(B)
+    bc, vc = g.upload_rows(np.zeros((2, la + lb), np.uint32))
+    builtin = g.ntt_get_launch()
+    try:
+        for mask in range(16):
+            g.ntt_set_launch(mask, builtin[1])
+            bc.fill(0)
+            g.kernel_stats_reset(True)
+            g.check(ctx.mul(va, vb, vc), "mul")
+            g.synchronize()
+            sizes = {name.split("@2^")[1] for name, *_ in g.kernel_stats(by_size=True)}
+            assert sizes == {"23"} and np.array_equal(g.download_rows(vc, bc), want), mask
+    finally:
+        g.kernel_stats_reset(False)
+        g.ntt_set_launch(*builtin)
