@@ -25,8 +25,18 @@ def oracle():
 
 
 @pytest.fixture(scope="session")
-def ctx():
+def shared_context():
     import gpupi_amd
     c = gpupi_amd.Context()
     yield c
     c.close()
+
+
+@pytest.fixture
+def ctx(shared_context):
+    """The session's context, with the crossover that a fresh one has (tests
+    that move it leave it somewhere else)."""
+    import gpupi_amd
+    from helpers import DEFAULT_NTT_MIN_LIMBS
+    gpupi_amd.check(shared_context.set_ntt_threshold(DEFAULT_NTT_MIN_LIMBS), "set_ntt_threshold")
+    return shared_context

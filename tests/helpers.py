@@ -5,6 +5,8 @@ from __future__ import annotations
 import numpy as np
 
 MASK32 = 0xFFFFFFFF
+# L_a + L_b from which a fresh context's products take the NTT
+DEFAULT_NTT_MIN_LIMBS = 4089
 
 
 def to_int(row) -> int:

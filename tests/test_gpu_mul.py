@@ -13,7 +13,7 @@ import pytest
 
 import gpupi_amd as g
 import oracle_ffi as of
-from helpers import rand_rows, to_int
+from helpers import DEFAULT_NTT_MIN_LIMBS, rand_rows, to_int
 
 pytestmark = pytest.mark.gpu
 PAD = 0xDEADBEEF
@@ -1133,3 +1133,25 @@ def test_every_tile_pairing_with_streamed_and_truncated_planes(ctx):
     finally:
         g.kernel_stats_reset(False)
         g.ntt_set_launch(*builtin)
+
+
+@pytest.mark.parametrize("leave", [384, 2, None])
+def test_every_test_starts_at_the_shipped_crossover(ctx, leave):
+    """The shared context sends the products to the NTT that a fresh one does,
+    whatever the test before left behind: 4089 limbs in all and not 4088."""
+    def ntt_kernels(c, total):
+        A, B = (rand_rows(np.random.default_rng(total), 1, n) for n in (total // 2, total - total // 2))
+        g.kernel_stats_reset(True)
+        try:
+            assert np.array_equal(device_mul(c, A, B), oracle_mul(A, B))
+            return [name for name, *_ in g.kernel_stats()]
+        finally:
+            g.kernel_stats_reset(False)
+
+    with g.Context() as fresh:
+        for total in (500, DEFAULT_NTT_MIN_LIMBS - 1, DEFAULT_NTT_MIN_LIMBS, 5000):
+            want = ntt_kernels(fresh, total)
+            assert bool(want) == (total >= DEFAULT_NTT_MIN_LIMBS)
+            assert ntt_kernels(ctx, total) == want, total
+    if leave is not None:
+        g.check(ctx.set_ntt_threshold(leave), "set_ntt_threshold")
