@@ -114,9 +114,10 @@ def tune_splits(ctx, ops: Operands, k: int, reps: int = 3, log=None, shared: boo
     return sorted(res, key=lambda r: r[1])
 
 
-def tune_crossover(ctx, ops: Operands, totals=(128, 192, 256, 320, 384, 512, 768, 1024), reps: int = 5):
+def tune_crossover(ctx, ops: Operands, totals=(384, 512, 1024, 2048, 3072, 4088, 4096, 6144), reps: int = 5):
     """Smallest L_a + L_b (of the candidates) from which the NTT is faster
-    than the schoolbook kernels on full batches."""
+    than the schoolbook kernels on full batches: the matrix cores up to 4088
+    limbs in all, one wave per product above."""
     best = None
     for t in totals:
         A, B, C = ops.arrays(t // 2)

@@ -38,3 +38,24 @@ def test_bench_refuses_more_than_one_gpu():
                        timeout=120)
     assert r.returncode == 2
     assert "one GPU" in r.stderr and r.stdout == ""
+
+
+def test_crossover_tuner_finds_the_shipped_crossover(monkeypatch):
+    """With schoolbook products that beat the NTT up to 4088 limbs in all, the
+    tuner's own candidates bracket that length."""
+    from gpupi_amd import tune
+    from helpers import DEFAULT_NTT_MIN_LIMBS
+
+    class Ctx:
+        def set_ntt_threshold(self, n):
+            self.school = n > 2
+            return 0
+
+    class Ops:
+        def arrays(self, length):
+            return 2 * length, None, None
+
+    monkeypatch.setattr(tune, "time_mul", lambda ctx, A, B, C, reps:
+                        (1.0 if A < DEFAULT_NTT_MIN_LIMBS else 9.0) if ctx.school else 2.0)
+    best = tune.tune_crossover(Ctx(), Ops())
+    assert best is not None and DEFAULT_NTT_MIN_LIMBS <= best <= DEFAULT_NTT_MIN_LIMBS + 8
