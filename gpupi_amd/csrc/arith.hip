@@ -342,7 +342,8 @@ namespace {
 //   two pieces of ceil(L / 2) limbs at K' = K/2 when their digits fit;
 //   m >= 3 equal pieces of at least S limbs at a smaller K' when even their
 //     full transforms cost at most 0.8 of 3 K.
-// Two pieces are two products sharing S's transform, the first written in
+// (A square is never put in pieces: it has one transform, not two.)  Two
+// pieces are two products sharing S's transform, the first written in
 // place, and one add finishes.  More are the rows of one ragged launch
 // sequence (piece_row), staged and assembled.  Transforms of 2^22 points and
 // up for two pieces, 2^21 for more (smaller products are bound by launches,
@@ -554,8 +555,8 @@ hipError_t ragged_launches(BatchMPContext *ctx, const GpupiMulItem *items, const
                      [&](const Group &x, const Group &y) { return key(x.shape) < key(y.shape); });
     // a launch sequence of few rows takes 35-45 us whatever its size, and 2^20
     // points more in another take 25: up to that many, rows join the next
-    // larger transform (14 pairs of 2^8..2^16 limbs: 287 -> 111 us; with
-    // 2^22 points 164 pairs of 2^8..2^18 limbs 536 -> 656 us)
+    // larger transform (14 pairs of 2^8..2^16 limbs 233 -> 102 us, 164
+    // pairs of 2^8..2^18 limbs 750 -> 650; with 2^22 points 715)
     constexpr uint64_t kJoinPoints = 1ull << 20;
     for (size_t e = groups.size(), top = e; e > 0;) {
         size_t b = e;

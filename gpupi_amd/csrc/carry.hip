@@ -8,11 +8,14 @@
 // wave settles 64 limbs per step instead of the reference's 32-lane
 // Kogge-Stone scans (reference batch_mul_addsub_warp.h:5-85).
 //
-// Layout: one wave owns a chunk of SEG*64 consecutive limbs of one row
-// (coalesced 256-byte segments).  Rows longer than a chunk get a second,
-// tiny kernel: each chunk looks back at its predecessors' (generate,
-// all-propagate) flags and, only if its carry-in is 1, ripples it through
-// its own limbs.  Rows of at most kThreadRowMax limbs use one thread per row.
+// Layout: rows of at most kThreadRowMax limbs take one thread each; up to 512
+// limbs one wave (addsub_chunk_kernel, coalesced 256-byte segments); longer
+// rows one wave per chunk of 1024 limbs, four limbs per lane
+// (addsub_vec_kernel, spill_add_vec_kernel).  The chunks of a row that one
+// block holds (kRowWaves) settle the carries between them in LDS; longer rows
+// get a second, tiny kernel: each chunk looks back at its predecessors'
+// (generate, all-propagate) flags and, only if its carry-in is 1, ripples it
+// through its own limbs.
 #include <type_traits>
 
 #include "common.hpp"

@@ -91,8 +91,9 @@ hipError_t launch_mul_naive(const uint32_t *A, const uint32_t *B, uint32_t *C, u
                             uint32_t L_a, uint32_t L_b, uint32_t stride_A, uint32_t stride_B,
                             uint32_t stride_C, hipStream_t stream);
 // Products C = A B of N rows on the matrix cores, LA, LB >= 1 and LA + LB at
-// most kMulMfmaMaxTotal (16 tiles of 256 limbs; one limb per tile boundary is
-// left for the recoding's extra digits).
+// most kMulMfmaMaxTotal: four groups of five tiles hold every split of up to
+// 4095 limbs (of 513 blocks of 32 digits in all, the recoding's carries among
+// them); this is the last multiple of eight limbs.
 constexpr uint32_t kMulMfmaMaxTotal = 4088;
 hipError_t launch_mul_mfma(const uint32_t *A, const uint32_t *B, uint32_t *C, uint32_t N, uint32_t LA, uint32_t LB,
                            uint32_t sA, uint32_t sB, uint32_t sC, hipStream_t stream);

@@ -1,11 +1,14 @@
 // Schoolbook batched products for short operands (reference
 // batch_mul_naive.cu:8-273 covers the same role with warp-32 kernels).
 //
-// Two wave64 designs:
-//  * thread per product (short operand <= 16 limbs): the short operand and a
-//    sliding window of partial sums live in registers; the long operand
-//    streams through, one 32x32+32+32 -> 64-bit multiply-add per limb pair.
-//  * wave per product: operands staged in LDS; lane l owns output columns
+// Three designs, chosen by launch_mul_naive:
+//  * thread per product (short operand <= 16 limbs against up to 128, or one
+//    too long for the others): the short operand and a sliding window of
+//    partial sums live in registers; the long operand streams through, one
+//    32x32+32+32 -> 64-bit multiply-add per limb pair.
+//  * the matrix cores (mul_mfma.hip): up to 4088 limbs in all.
+//  * wave per product, for the longer ones that a raised threshold sends here:
+//    operands staged in LDS; lane l owns output columns
 //    256g + 4l .. +3 and accumulates each column as lo32 + hi64 (no carry
 //    handling in the inner loop: t = a*b + lo fits 64 bits).  Columns are
 //    turned into limbs with two lane shifts (y_{k-1}, z_{k-2}) and one
