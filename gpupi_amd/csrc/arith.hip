@@ -707,7 +707,7 @@ static hipError_t mul_ragged(BatchMPContext *ctx, const GpupiMulItem *items, uin
         GPUPI_RETURN_IF(gpupi::launch_mul_naive(r.A, r.B, r.C, 1, r.L_a, r.L_b, r.L_a, r.L_b, r.L_a + r.L_b,
                                                 ctx->stream));
     } else {
-        GPUPI_RETURN_IF(gpupi::launch_mul_mfma_ragged(small, *ctx->cache, ctx->stream));
+        GPUPI_RETURN_IF(gpupi::launch_mul_mfma_ragged(std::move(small), *ctx->cache, ctx->stream));
     }
     if (big.empty()) return hipSuccess;
     // NTT rows, one launch sequence per transform size (and row chunk):

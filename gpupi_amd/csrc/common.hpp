@@ -106,7 +106,7 @@ struct MfmaRow {
     uint32_t L_a, L_b;
 };
 class BlockCache;
-hipError_t launch_mul_mfma_ragged(const std::vector<MfmaRow> &products, BlockCache &cache, hipStream_t stream);
+hipError_t launch_mul_mfma_ragged(std::vector<MfmaRow> products, BlockCache &cache, hipStream_t stream);
 bool mul_naive_supports(uint32_t L_a, uint32_t L_b);
 
 hipError_t launch_mul_ntt(const uint32_t *A, const uint32_t *B, uint32_t *C, void *workspace,

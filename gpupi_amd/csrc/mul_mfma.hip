@@ -69,23 +69,18 @@ struct MfmaArgs {
 
 // A ragged launch carries its products in the kernel's arguments: no device
 // memory to fill, nothing to wait for, and a captured launch holds its own
-// copy.  A product is three words, its limb addresses (multiples of four) over
-// the lengths, so that as many as possible go into the 4 KB that a launch's
-// arguments may take: launches follow each other, and with rows of 32 bytes,
+// copy.  A product is three words (arg_word), so that as many as possible go
+// into the 4 KB that a launch's arguments may take: launches follow each other, and with rows of 32 bytes,
 // 96 to a launch, 600 products of 2^9..2^11 limbs took 156 us instead of 87.
 // Above six launches the same rows go into a block of device memory, one
 // launch per number of tile groups (600 products of 2^9..2^11 limbs 87 us from
 // arguments against 98 from memory, 1500 of them 186 against 155, 12000 2042
 // against 879).
 constexpr uint32_t kArgRows = 168, kArgRowsMost = 6 * kArgRows;
-constexpr int kLengthBits = 12;
 struct ArgRow {
     uint64_t a, b, c;
 };
-static_assert(kMulMfmaMaxTotal <= 1u << kLengthBits, "a length fits its bits");
-inline uint64_t arg_word(const uint32_t *p, uint32_t length) { return (uint64_t)(uintptr_t)p << (kLengthBits - 2) | length; }
-__device__ __forceinline__ uint32_t *arg_limbs(uint64_t w) { return reinterpret_cast<uint32_t *>(w >> kLengthBits << 2); }
-__device__ __forceinline__ uint32_t arg_length(uint64_t w) { return (uint32_t)w & ((1u << kLengthBits) - 1u); }
+static_assert(kMulMfmaMaxTotal <= 1u << kArgLengthBits, "a length fits its bits");
 struct MfmaRaggedArgs {
     uint32_t W;
     ArgRow rows[kArgRows];
@@ -333,9 +328,9 @@ mul_mfma_kernel(ARGS args) {
     const size_t row = RAGGED ? 0 : blockIdx.x;
     if constexpr (RAGGED) {
         const ArgRow rr = args.rows[blockIdx.x];
-        a.A = arg_limbs(rr.a);
-        a.B = arg_limbs(rr.b);
-        a.C = arg_limbs(rr.c);
+        a.A = reinterpret_cast<const uint32_t *>(arg_address(rr.a));
+        a.B = reinterpret_cast<const uint32_t *>(arg_address(rr.b));
+        a.C = reinterpret_cast<uint32_t *>(arg_address(rr.c));
         a.LA = arg_length(rr.a);
         a.LB = arg_length(rr.b);
         a.na = blocks_of(a.LA);
@@ -597,7 +592,13 @@ hipError_t launch_ragged(RaggedKernel<ARGS> kernel, const ARGS &args, uint32_t n
 }
 }  // namespace
 
-hipError_t launch_mul_mfma_ragged(const std::vector<MfmaRow> &products, BlockCache &cache, hipStream_t stream) {
+hipError_t launch_mul_mfma_ragged(std::vector<MfmaRow> products, BlockCache &cache, hipStream_t stream) {
+    // addresses that no word holds take a launch each
+    const auto packs = [](const MfmaRow &r) { return arg_packs((uintptr_t)r.A) && arg_packs((uintptr_t)r.B) && arg_packs((uintptr_t)r.C); };
+    const auto rest = std::stable_partition(products.begin(), products.end(), packs);
+    for (auto r = rest; r != products.end(); ++r)
+        GPUPI_RETURN_IF(launch_mul_mfma(r->A, r->B, r->C, 1, r->L_a, r->L_b, r->L_a, r->L_b, r->L_a + r->L_b, stream));
+    products.erase(rest, products.end());
     const size_t n = products.size();
     // in the order of their tile groups: a launch takes those of its last
     size_t start[kRaggedMaxW + 2] = {};  // start[w]: products of fewer than w groups
@@ -617,9 +618,9 @@ hipError_t launch_mul_mfma_ragged(const std::vector<MfmaRow> &products, BlockCac
         std::copy_n(start, kRaggedMaxW + 1, at);
         for (size_t i = 0; i < n; ++i) {
             const MfmaRow &r = products[i];
-            uint64_t a = arg_word(r.A, r.L_a), b = arg_word(r.B, r.L_b);
+            uint64_t a = arg_word((uintptr_t)r.A, r.L_a), b = arg_word((uintptr_t)r.B, r.L_b);
             if (r.L_a > r.L_b) std::swap(a, b);
-            rows[at[groups[i]]++] = ArgRow{a, b, arg_word(r.C, 0)};
+            rows[at[groups[i]]++] = ArgRow{a, b, arg_word((uintptr_t)r.C, 0)};
         }
     }
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;

@@ -31,6 +31,14 @@ struct RaggedB {
     const uint32_t *B;
     uint32_t L, tau;
 };
+// A limb address and a length in one word: the address, a multiple of four
+// below 2^54 (arg_packs), over the length.
+constexpr int kArgLengthBits = 12;
+GPUPI_HD bool arg_packs(uint64_t address) { return (address & 3u) == 0 && address >> (66 - kArgLengthBits) == 0; }
+GPUPI_HD uint64_t arg_word(uint64_t address, uint32_t length) { return address << (kArgLengthBits - 2) | length; }
+GPUPI_HD uint64_t arg_address(uint64_t w) { return w >> kArgLengthBits << 2; }
+GPUPI_HD uint32_t arg_length(uint64_t w) { return (uint32_t)w & ((1u << kArgLengthBits) - 1u); }
+
 // A product L * S (c = |L| + |S| limbs) run in m pieces of s limbs of L (the
 // last one shorter) against S: its pieces are the launch's rows row0 ..
 // row0 + m - 1, and C word x is the sum of piece floor(x / s)'s product

@@ -83,3 +83,14 @@ def test_digits_and_runs(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=600)
     assert out.returncode == 0, out.stdout + out.stderr
     assert "digit check: ok" in out.stdout
+
+
+def test_argument_words_keep_addresses_and_lengths(tmp_path):
+    """ragged.hpp: the words of a ragged launch's arguments hold every address
+    they accept, and refuse unaligned ones and those past 2^54."""
+    exe = tmp_path / "arg_word_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "gpupi_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "native", "arg_word_check.cpp"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=600)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert "arg words: ok" in out.stdout
