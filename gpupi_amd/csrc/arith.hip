@@ -453,7 +453,7 @@ hipError_t batch_mp_mul(BatchMPContext *ctx, BatchMPArray A, BatchMPArray B, Bat
     }
     // (a square transforms its one operand once, which pieces would not: whole
     // / in pieces 1100000 limbs 83 / 165 us, 1500000 132 / 163, 9000000 534 / 1066)
-    const bool square = A.data == B.data && A.length == B.length;
+    const bool square = A.data == B.data && A.length == B.length && A.stride == B.stride;
     if (C.batch_size == 1 && !square && ctx->pipeline_form != GPUPI_FORM_PLAIN) {
         const bool a_long = A.length >= B.length;
         const BatchMPArray &L = a_long ? A : B, &S = a_long ? B : A;

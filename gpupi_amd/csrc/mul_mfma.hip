@@ -70,12 +70,12 @@ struct MfmaArgs {
 // A ragged launch carries its products in the kernel's arguments: no device
 // memory to fill, nothing to wait for, and a captured launch holds its own
 // copy.  A product is three words (arg_word), so that as many as possible go
-// into the 4 KB that a launch's arguments may take: launches follow each other, and with rows of 32 bytes,
-// 96 to a launch, 600 products of 2^9..2^11 limbs took 156 us instead of 87.
-// Above six launches the same rows go into a block of device memory, one
-// launch per number of tile groups (600 products of 2^9..2^11 limbs 87 us from
-// arguments against 98 from memory, 1500 of them 186 against 155, 12000 2042
-// against 879).
+// into the 4 KB that a launch's arguments may take: launches follow each other,
+// and with rows of 32 bytes, 96 to a launch, 600 products of 2^9..2^11 limbs
+// took 156 us instead of 87.  Above six launches the same rows go into a block
+// of device memory, one launch per number of tile groups (600 products of
+// 2^9..2^11 limbs 87 us from arguments against 98 from memory, 1500 of them 186
+// against 155, 12000 2042 against 879).
 constexpr uint32_t kArgRows = 168, kArgRowsMost = 6 * kArgRows;
 struct ArgRow {
     uint64_t a, b, c;
@@ -594,7 +594,9 @@ hipError_t launch_ragged(RaggedKernel<ARGS> kernel, const ARGS &args, uint32_t n
 
 hipError_t launch_mul_mfma_ragged(std::vector<MfmaRow> products, BlockCache &cache, hipStream_t stream) {
     // addresses that no word holds take a launch each
-    const auto packs = [](const MfmaRow &r) { return arg_packs((uintptr_t)r.A) && arg_packs((uintptr_t)r.B) && arg_packs((uintptr_t)r.C); };
+    const auto packs = [](const MfmaRow &r) {
+        return arg_packs((uintptr_t)r.A) && arg_packs((uintptr_t)r.B) && arg_packs((uintptr_t)r.C);
+    };
     const auto rest = std::stable_partition(products.begin(), products.end(), packs);
     for (auto r = rest; r != products.end(); ++r)
         GPUPI_RETURN_IF(launch_mul_mfma(r->A, r->B, r->C, 1, r->L_a, r->L_b, r->L_a, r->L_b, r->L_a + r->L_b, stream));
